@@ -2374,8 +2374,8 @@ extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* eval
     std::vector<LeafJob> leaves;
     std::vector<uint64_t> leaf_prefix(1, 0);
     for (size_t j : tall) {
-        leaves.push_back(LeafJob{b->trees[j]->mats[0]->ptr, W[j], (uint32_t)W[j], 0, digests[j]});
-        leaf_prefix.push_back(leaf_prefix.back() + N[j]);
+        leaves.push_back(LeafJob{b->trees[j]->mats[0]->ptr, W[j], (uint32_t)W[j], (uint32_t)N[j], digests[j]});
+        leaf_prefix.push_back(leaf_prefix.back() + (N[j] + 63) / 64);  // a wave hashes 64 rows of one job
     }
     const size_t off_leaf = st.put(leaves.data(), leaves.size() * sizeof(LeafJob));
     const size_t off_leaf_prefix = st.put(leaf_prefix.data(), leaf_prefix.size() * 8);

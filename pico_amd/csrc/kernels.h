@@ -66,21 +66,22 @@ hipError_t launch_open_gather(const MatRef* mats, const uint32_t* shift, const u
                               hipStream_t stream);
 
 // ---- batched Merkle (merkle.hip): many single-matrix commits per launch ---
-// Jobs are found by binary search of the thread's global row / node index in
-// a prefix array (njobs + 1 entries, prefix[0] = 0).
+// Jobs are found by binary search of the wave's group of 64 rows (leaves; a
+// job's last group may be partial) or the lane's node index in a prefix array
+// (njobs + 1 entries, prefix[0] = 0).
 struct LeafJob {
     const uint32_t* data;  // rows x width, row stride `stride`
     uint64_t stride;
     uint32_t width;
-    uint32_t pad_;
+    uint32_t rows;
     uint32_t* digests;  // rows x 8
 };
 struct CompressJob {
     const uint32_t* prev;  // 2 n x 8
     uint32_t* next;        // n x 8
 };
-hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t* row_prefix, int njobs,
-                                  uint64_t total_rows, hipStream_t stream);
+hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t* group_prefix, int njobs,
+                                  uint64_t total_groups, hipStream_t stream);
 hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint64_t* node_prefix,
                                  int njobs, uint64_t total_nodes, hipStream_t stream);
 // dst[8 j + k] = src[j][k] for j < n (root digests of n trees)

@@ -9,41 +9,16 @@
 //               exist: next[i] = C(next[i], H(concat of their row i))
 //   H = PaddingFreeSponge<16, 8, 8> (overwrite mode, circuit/hash.rs:40-52)
 //   C = TruncatedPermutation (circuit/hash.rs:89-94)
-// One thread owns one permutation state for the whole row / node.
+// Layers of more than LANES_MAX_NODES nodes and every leaf hash run 64 states
+// per wave with the linear layers on the matrix cores (poseidon2_mx.h): the
+// grid deals groups of 64 rows or nodes to waves.
+#include <algorithm>
+
 #include "kernels.h"
 #include "poseidon2.h"
+#include "poseidon2_mx.h"
 
 namespace pg {
-
-// Absorb the concatenation of row `row` of mats[0..n) into st (which the
-// caller zeroes).  The cursor (k, j) is wave-uniform, so the matrix
-// descriptors are read through the scalar cache.
-template <class F>
-__device__ __forceinline__ void absorb_rows(uint32_t (&st)[16], const MatRef* mats, int n,
-                                            uint32_t total, uint64_t row) {
-    if (total == 0) return;
-    int k = 0;
-    uint32_t j = 0;
-    gcptr base = (gcptr)mats[0].data + row * mats[0].stride;
-    uint32_t wk = mats[0].width;
-    for (uint32_t off = 0; off < total; off += 8) {
-        uint32_t cnt = total - off < 8u ? total - off : 8u;
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            if ((uint32_t)t < cnt) {
-                while (j >= wk && k + 1 < n) {
-                    k++;
-                    j = 0;
-                    base = (gcptr)mats[k].data + row * mats[k].stride;
-                    wk = mats[k].width;
-                }
-                st[t] = base[j];
-                j++;
-            }
-        }
-        permute<F>(st);
-    }
-}
 
 // ---- one permutation over 16 lanes ---------------------------------------
 // A layer with few nodes cannot fill the GPU, so with one state per thread it
@@ -169,42 +144,207 @@ __global__ void __launch_bounds__(256) leaf8_lanes_kernel(const uint32_t* data, 
     if (l < 8) ((gptr)digests)[8 * row + l] = x;
 }
 
-// General leaf hash: any number of matrices, any widths.
-template <class F>
-__global__ void __launch_bounds__(256) leaf_hash_kernel(const MatRef* mats, int n, uint32_t total,
-                                                        uint64_t rows, uint32_t* digests) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    uint32_t st[16];
+// ---- hashing on the matrix cores --------------------------------------------
+// What bounds it: VALU issue, now of the S-boxes and the layer reductions.
+// A wave's two tiles of 32 states share every table read from LDS (31 KB per
+// workgroup, read once per permutation and wave).
+constexpr int MX_WAVES = 4;  // waves per workgroup
+constexpr int MX_THREADS = 64 * MX_WAVES;
+// Three waves per SIMD (168 registers): at four (128) the kernels spill, at two
+// the issue slots are not all filled (leaf hash of 2^21 x 256: 4.53 ms, 4.82
+// and 4.70).
+#define MX_KERNEL __global__ void __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte access at word alignment
+
+// The lane's place in its wave: state 32 t + n of tile t, words 4 h + i of the
+// rate and of the capacity.
+struct MxLane {
+    uint32_t n, h;
+    __device__ __forceinline__ MxLane() : n(threadIdx.x & 31u), h((threadIdx.x & 63u) >> 5) {}
+};
+// index of the wave in the grid (uniform)
+__device__ __forceinline__ uint64_t mx_wave() {
+    return (uint64_t)blockIdx.x * MX_WAVES + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+__device__ __forceinline__ mx4 mx_op(u32x4 v) { return __builtin_bit_cast(mx4, v ^ MX_BIAS); }
+__device__ __forceinline__ mx4 mx_op_words(const uint32_t* st) { return mx_op(u32x4{st[0], st[1], st[2], st[3]}); }
+
+// A cursor over the concatenation of one row of mats[0..n): the words
+// 8 c + 4 h .. + 3 of chunk c for the wave's two tiles.  The cursor (k, j) is
+// wave-uniform, so the matrix descriptors are read through the scalar cache.
+struct MxRows {
+    const MatRef* mats;
+    int n, k;
+    uint32_t j;
+    __device__ __forceinline__ MxRows(const MatRef* m, int nm) : mats(m), n(nm), k(0), j(0) {}
+    __device__ __forceinline__ void skip_ended() {
+        while (j >= mats[k].width && k + 1 < n) {
+            k++;
+            j = 0;
+        }
+    }
+    // cnt words of the chunk exist; the others read as word 0
+    __device__ __forceinline__ void chunk(u32x4 (&out)[2], const uint64_t (&row)[2], uint32_t cnt, uint32_t h) {
+        skip_ended();
+        if (cnt == 8 && j + 8 <= mats[k].width) {  // within one matrix
+            const gcptr base = (gcptr)mats[k].data + (j + 4 * h);
 #pragma unroll
-    for (int t = 0; t < 16; t++) st[t] = 0;
-    absorb_rows<F>(st, mats, n, total, i);
-    uint4* o = reinterpret_cast<uint4*>(digests + 8 * i);
-    o[0] = make_uint4(st[0], st[1], st[2], st[3]);
-    o[1] = make_uint4(st[4], st[5], st[6], st[7]);
+            for (int t = 0; t < 2; t++)
+                out[t] = *reinterpret_cast<const GLOBAL u32x4u*>(base + row[t] * mats[k].stride);
+            j += 8;
+            return;
+        }
+        const uint32_t* p[8];
+        uint64_t st[8];
+#pragma unroll
+        for (int w = 0; w < 8; w++) {
+            if ((uint32_t)w < cnt) {
+                skip_ended();
+                p[w] = mats[k].data + j;
+                st[w] = mats[k].stride;
+                j++;
+            } else {
+                p[w] = p[0];
+                st[w] = st[0];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const gcptr q = (gcptr)(h ? p[4 + i] : p[i]);
+            const uint64_t ld = h ? st[4 + i] : st[i];
+#pragma unroll
+            for (int t = 0; t < 2; t++) out[t][i] = q[row[t] * ld];
+        }
+    }
+};
+
+// Sponge state of 64 rows between permutations: `b`, the last S-boxes'
+// outputs (the zero state: S-box outputs of zero); the state words themselves
+// are formed only where a chunk is partial and at the end.
+template <class F>
+struct MxSponge {
+    mx4 b[2][2];
+    __device__ __forceinline__ MxSponge() {
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) b[t][s] = mx_op(u32x4{0});
+    }
+    // Absorbs a whole chunk
+    __device__ __forceinline__ void absorb8(const u32x4 (&in)[2], MxView<F>& v) {
+        int x[2][8];
+        v.fresh();
+        const mx4 rate[2] = {mx_op(in[0]), mx_op(in[1])};
+        mx_next<F>(x, rate, b, v);
+        mx_rounds<F>(b, x, v);
+    }
+    // Absorbs one chunk: cnt of its 8 words overwrite the rate words.
+    __device__ __forceinline__ void absorb(const u32x4 (&in)[2], uint32_t cnt, uint32_t h, MxView<F>& v) {
+        int x[2][8];
+        v.fresh();
+        if (cnt == 8) {
+            const mx4 rate[2] = {mx_op(in[0]), mx_op(in[1])};
+            mx_next<F>(x, rate, b, v);
+        } else {
+            uint32_t st[2][8];
+            mx_last<F>(st, b, v);
+            mx4 full[2][2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (4 * h + i < cnt) st[t][i] = in[t][i];
+                full[t][0] = mx_op_words(&st[t][0]);
+                full[t][1] = mx_op_words(&st[t][4]);
+            }
+            mx_init<F>(x, full, v);
+        }
+        mx_rounds<F>(b, x, v);
+    }
+    // absorbs the concatenated rows; total > 0
+    __device__ __forceinline__ void absorb_rows(MxRows src, const uint64_t (&row)[2], uint32_t total, uint32_t h,
+                                                MxView<F>& v) {
+        u32x4 next[2];
+        src.chunk(next, row, total < 8u ? total : 8u, h);
+        for (uint32_t off = 0; off < total; off += 8) {
+            const u32x4 cur[2] = {next[0], next[1]};
+            const uint32_t left = total - off;
+            // the next chunk's words are in flight during the permutation
+            if (left > 8) src.chunk(next, row, left - 8 < 8u ? left - 8 : 8u, h);
+            absorb(cur, left < 8u ? left : 8u, h, v);
+        }
+    }
+};
+
+// Row addresses of the wave's group; rows past the end shadow the last one.
+__device__ __forceinline__ void mx_group_rows(uint64_t (&row)[2], uint64_t group, uint64_t rows, const MxLane& l) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const uint64_t r = 64 * group + 32 * t + l.n;
+        row[t] = r < rows ? r : rows - 1;
+    }
+}
+__device__ __forceinline__ void mx_store_digests(uint32_t* digests, uint64_t group, uint64_t rows, const MxLane& l,
+                                                 const uint32_t (&st)[2][8]) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const uint64_t r = 64 * group + 32 * t + l.n;
+        if (r < rows)
+            *reinterpret_cast<GLOBAL u32x4*>((gptr)digests + 8 * r + 4 * l.h) =
+                u32x4{st[t][0], st[t][1], st[t][2], st[t][3]};
+    }
 }
 
-// One matrix whose width is a multiple of 8 and whose rows are 32-byte
-// aligned: every sponge chunk is two 16-byte loads.
+// General leaf hash: any number of matrices, any widths.
 template <class F>
-__global__ void __launch_bounds__(256) leaf_hash_w8_kernel(const uint32_t* data, uint64_t stride,
-                                                           uint32_t chunks, uint64_t rows,
-                                                           uint32_t* digests) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    const uint4* rp = reinterpret_cast<const uint4*>(data + i * stride);
-    uint32_t st[16];
-#pragma unroll
-    for (int t = 0; t < 16; t++) st[t] = 0;
-    for (uint32_t c = 0; c < chunks; c++) {
-        uint4 a = rp[2 * c], b = rp[2 * c + 1];
-        st[0] = a.x; st[1] = a.y; st[2] = a.z; st[3] = a.w;
-        st[4] = b.x; st[5] = b.y; st[6] = b.z; st[7] = b.w;
-        permute<F>(st);
+MX_KERNEL leaf_hash_kernel(const MatRef* mats, int n, uint32_t total,
+                                                               uint64_t rows, uint32_t* digests) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    const uint64_t group = mx_wave();
+    if (64 * group >= rows) return;
+    MxView<F> v(tab);
+    const MxLane l;
+    uint32_t st[2][8] = {};
+    if (total) {
+        uint64_t row[2];
+        mx_group_rows(row, group, rows, l);
+        MxSponge<F> sp;
+        sp.absorb_rows(MxRows(mats, n), row, total, l.h, v);
+        mx_last<F>(st, sp.b, v);
     }
-    uint4* o = reinterpret_cast<uint4*>(digests + 8 * i);
-    o[0] = make_uint4(st[0], st[1], st[2], st[3]);
-    o[1] = make_uint4(st[4], st[5], st[6], st[7]);
+    mx_store_digests(digests, group, rows, l, st);
+}
+
+// One matrix whose width is a multiple of 8 and whose rows are 16-byte
+// aligned: every sponge chunk is one 16-byte load per lane and tile.
+template <class F>
+MX_KERNEL leaf_hash_w8_kernel(const uint32_t* data, uint64_t stride,
+                                                                  uint32_t chunks, uint64_t rows,
+                                                                  uint32_t* digests) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    const uint64_t group = mx_wave();
+    if (64 * group >= rows) return;
+    MxView<F> v(tab);
+    const MxLane l;
+    uint64_t row[2];
+    mx_group_rows(row, group, rows, l);
+    const GLOBAL u32x4* rp[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) rp[t] = reinterpret_cast<const GLOBAL u32x4*>((gcptr)data + row[t] * stride + 4 * l.h);
+    u32x4 next[2] = {rp[0][0], rp[1][0]};
+    MxSponge<F> sp;
+    for (uint32_t c = 0; c < chunks; c++) {
+        const u32x4 cur[2] = {next[0], next[1]};
+        const uint32_t cn = c + 1 < chunks ? c + 1 : c;
+        next[0] = rp[0][2 * cn];  // in flight during the permutation
+        next[1] = rp[1][2 * cn];
+        sp.absorb8(cur, v);
+    }
+    uint32_t st[2][8];
+    mx_last<F>(st, sp.b, v);
+    mx_store_digests(digests, group, rows, l, st);
 }
 
 // One segment of the leaf sponge: columns [0, width) of a matrix view are
@@ -217,88 +357,189 @@ __global__ void __launch_bounds__(256) leaf_hash_w8_kernel(const uint32_t* data,
 // permutation (if any) and write the digest instead of the state.  The
 // segments of a row, concatenated, give the same digest as one pass of
 // absorb_rows over the whole row.
-template <class F, bool VEC>
-__global__ void __launch_bounds__(256) absorb_segment_kernel(const uint32_t* data, uint64_t stride,
-                                                             uint32_t width, uint32_t pos0, int first,
-                                                             int last, uint64_t rows, uint32_t* state,
-                                                             uint32_t* digests) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    uint32_t st[16];
-    if (first) {
+template <class F>
+MX_KERNEL absorb_segment_kernel(const uint32_t* data, uint64_t stride,
+                                                                    uint32_t width, uint32_t pos0, int first,
+                                                                    int last, uint64_t rows, uint32_t* state,
+                                                                    uint32_t* digests) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    const uint64_t group = mx_wave();
+    if (64 * group >= rows) return;
+    MxView<F> v(tab);
+    const MxLane l;
+    uint64_t row[2];
+    mx_group_rows(row, group, rows, l);
+    // st holds the state while a chunk is pending, b after a permutation
+    uint32_t st[2][8] = {};
+    if (!first) {
 #pragma unroll
-        for (int t = 0; t < 16; t++) st[t] = 0;
-    } else {
-        const GLOBAL u32x4* sp = reinterpret_cast<const GLOBAL u32x4*>((gcptr)state + 16 * i);
+        for (int t = 0; t < 2; t++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            u32x4 v = sp[q];
-            st[4 * q] = v.x; st[4 * q + 1] = v.y; st[4 * q + 2] = v.z; st[4 * q + 3] = v.w;
-        }
+            for (int s = 0; s < 2; s++) {
+                const u32x4 w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)state + 16 * row[t] + 8 * s + 4 * l.h);
+#pragma unroll
+                for (int i = 0; i < 4; i++) st[t][4 * s + i] = w[i];
+            }
     }
-    gcptr row = (gcptr)data + i * stride;
-    uint32_t pos = pos0;
-    if constexpr (VEC) {  // pos0 == 0, width % 8 == 0, 16-byte aligned rows
-        const GLOBAL u32x4* rp = reinterpret_cast<const GLOBAL u32x4*>(row);
-        for (uint32_t c = 0; c < width / 8; c++) {
-            u32x4 a = rp[2 * c], b = rp[2 * c + 1];
-            st[0] = a.x; st[1] = a.y; st[2] = a.z; st[3] = a.w;
-            st[4] = b.x; st[5] = b.y; st[6] = b.z; st[7] = b.w;
-            permute<F>(st);
-        }
-    } else {
-        uint32_t e = 0;
-        while (e < width) {  // pos and e are the same in every lane
-            const uint32_t take = width - e < 8 - pos ? width - e : 8 - pos;
+    mx4 b[2][2];
+    bool words = true;  // st is valid
+    uint32_t pos = pos0, e = 0;
+    while (e < width || (last && pos > 0)) {  // pos, e and words are the same in every lane
+        const uint32_t take = width - e < 8 - pos ? width - e : 8 - pos;
+        int x[2][8];
+        v.fresh();
+        if (!words && take == 8) {
+            mx4 rate[2];
 #pragma unroll
-            for (int t = 0; t < 8; t++)
-                if ((uint32_t)t >= pos && (uint32_t)t < pos + take) st[t] = row[e + (uint32_t)t - pos];
+            for (int t = 0; t < 2; t++)
+                rate[t] = mx_op(*reinterpret_cast<const GLOBAL u32x4u*>((gcptr)data + row[t] * stride + e + 4 * l.h));
+            mx_next<F>(x, rate, b, v);
+            e += 8;
+        } else {
+            if (!words) mx_last<F>(st, b, v);
+            words = true;
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t w = 4 * l.h + i;
+                    if (w >= pos && w < pos + take) st[t][i] = ((gcptr)data)[row[t] * stride + e + w - pos];
+                }
             e += take;
             pos += take;
-            if (pos == 8) {
-                permute<F>(st);
-                pos = 0;
-            }
-        }
-    }
-    if (last) {
-        if (pos > 0) permute<F>(st);
-        GLOBAL u32x4* o = reinterpret_cast<GLOBAL u32x4*>((gptr)digests + 8 * i);
-        o[0] = u32x4{st[0], st[1], st[2], st[3]};
-        o[1] = u32x4{st[4], st[5], st[6], st[7]};
-    } else {
-        GLOBAL u32x4* o = reinterpret_cast<GLOBAL u32x4*>((gptr)state + 16 * i);
+            if (pos < 8 && !(last && e >= width)) break;  // pending: the next segment fills it
+            mx4 full[2][2];
 #pragma unroll
-        for (int q = 0; q < 4; q++) o[q] = u32x4{st[4 * q], st[4 * q + 1], st[4 * q + 2], st[4 * q + 3]};
+            for (int t = 0; t < 2; t++) {
+                full[t][0] = mx_op_words(&st[t][0]);
+                full[t][1] = mx_op_words(&st[t][4]);
+            }
+            mx_init<F>(x, full, v);
+            pos = 0;
+        }
+        mx_rounds<F>(b, x, v);
+        words = false;
+    }
+    if (!words) mx_last<F>(st, b, v);
+    if (last) {
+        mx_store_digests(digests, group, rows, l, st);
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const uint64_t r = 64 * group + 32 * t + l.n;
+        if (r >= rows) continue;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            *reinterpret_cast<GLOBAL u32x4*>((gptr)state + 16 * r + 8 * s + 4 * l.h) =
+                u32x4{st[t][4 * s], st[t][4 * s + 1], st[t][4 * s + 2], st[t][4 * s + 3]};
     }
 }
 
+// next[i] = C(prev[2i], prev[2i+1]), then with INJ: C(next[i], H(rows i of inj))
+template <class F, bool INJ>
+MX_KERNEL compress_kernel(const uint32_t* prev, uint32_t* next,
+                                                              uint64_t n_out, const MatRef* inj,
+                                                              int n_inj, uint32_t inj_width) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    MxView<F> v(tab);
+    const MxLane l;
+    const uint64_t stride = (uint64_t)gridDim.x * MX_WAVES;
+    for (uint64_t group = mx_wave(); 64 * group < n_out; group += stride) {
+        uint64_t row[2];
+        mx_group_rows(row, group, n_out, l);
+        u32x4 hash[2] = {u32x4{0}, u32x4{0}};
+        MxSponge<F> sp;
+        if constexpr (INJ) {
+            if (inj_width) {
+                uint32_t st[2][8];
+                sp.absorb_rows(MxRows(inj, n_inj), row, inj_width, l.h, v);
+                mx_last<F>(st, sp.b, v);
+#pragma unroll
+                for (int t = 0; t < 2; t++) hash[t] = u32x4{st[t][0], st[t][1], st[t][2], st[t][3]};
+            }
+        }
+        uint32_t st[2][8];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const u32x4 w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)prev + 16 * row[t] + 8 * s + 4 * l.h);
+#pragma unroll
+                for (int i = 0; i < 4; i++) st[t][4 * s + i] = w[i];
+            }
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < (INJ ? 2 : 1); k++) {
+            if (k) {
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) st[t][4 + i] = hash[t][i];
+            }
+            mx4 full[2][2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                full[t][0] = mx_op_words(&st[t][0]);
+                full[t][1] = mx_op_words(&st[t][4]);
+            }
+            int x[2][8];
+            v.fresh();
+            mx_init<F>(x, full, v);
+            mx_rounds<F>(sp.b, x, v);
+            mx_last<F>(st, sp.b, v);
+        }
+        mx_store_digests(next, group, n_out, l, st);
+    }
+}
+
+// The same with the injected rows already hashed: C(C(prev[2i], prev[2i+1]), inj[i])
 template <class F>
-__global__ void __launch_bounds__(256) compress_kernel(const uint32_t* prev, uint32_t* next,
-                                                       uint64_t n_out, const MatRef* inj,
-                                                       int n_inj, uint32_t inj_width) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_out) return;
-    const uint4* p = reinterpret_cast<const uint4*>(prev + 16 * i);
-    uint32_t st[16];
+MX_KERNEL compress_digest_kernel(const uint32_t* prev, const uint32_t* inj,
+                                                                     uint32_t* next, uint64_t n_out) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    MxView<F> v(tab);
+    const MxLane l;
+    const uint64_t stride = (uint64_t)gridDim.x * MX_WAVES;
+    for (uint64_t group = mx_wave(); 64 * group < n_out; group += stride) {
+        uint64_t row[2];
+        mx_group_rows(row, group, n_out, l);
+        u32x4 hash[2];
+        uint32_t st[2][8];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        uint4 v = p[q];
-        st[4 * q] = v.x; st[4 * q + 1] = v.y; st[4 * q + 2] = v.z; st[4 * q + 3] = v.w;
+        for (int t = 0; t < 2; t++) {
+            hash[t] = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)inj + 8 * row[t] + 4 * l.h);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const u32x4 w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)prev + 16 * row[t] + 8 * s + 4 * l.h);
+#pragma unroll
+                for (int i = 0; i < 4; i++) st[t][4 * s + i] = w[i];
+            }
+        }
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < 2; k++) {
+            if (k) {
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) st[t][4 + i] = hash[t][i];
+            }
+            mx4 full[2][2], b[2][2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                full[t][0] = mx_op_words(&st[t][0]);
+                full[t][1] = mx_op_words(&st[t][4]);
+            }
+            int x[2][8];
+            v.fresh();
+            mx_init<F>(x, full, v);
+            mx_rounds<F>(b, x, v);
+            mx_last<F>(st, b, v);
+        }
+        mx_store_digests(next, group, n_out, l, st);
     }
-    permute<F>(st);
-    if (n_inj > 0) {
-        uint32_t h[16];
-#pragma unroll
-        for (int t = 0; t < 16; t++) h[t] = 0;
-        absorb_rows<F>(h, inj, n_inj, inj_width, i);
-#pragma unroll
-        for (int t = 0; t < 8; t++) st[8 + t] = h[t];
-        permute<F>(st);
-    }
-    uint4* o = reinterpret_cast<uint4*>(next + 8 * i);
-    o[0] = make_uint4(st[0], st[1], st[2], st[3]);
-    o[1] = make_uint4(st[4], st[5], st[6], st[7]);
 }
 
 __global__ void open_gather_kernel(const MatRef* mats, const uint32_t* shift,
@@ -320,29 +561,6 @@ __global__ void open_gather_kernel(const MatRef* mats, const uint32_t* shift,
     }
 }
 
-template <class F>
-__global__ void __launch_bounds__(256) compress_digest_kernel(const uint32_t* prev, const uint32_t* inj,
-                                                              uint32_t* next, uint64_t n_out) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_out) return;
-    const GLOBAL u32x4* p = reinterpret_cast<const GLOBAL u32x4*>((gcptr)prev + 16 * i);
-    uint32_t st[16];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const u32x4 v = p[q];
-        st[4 * q] = v.x; st[4 * q + 1] = v.y; st[4 * q + 2] = v.z; st[4 * q + 3] = v.w;
-    }
-    permute<F>(st);
-    const GLOBAL u32x4* d = reinterpret_cast<const GLOBAL u32x4*>((gcptr)inj + 8 * i);
-    const u32x4 d0 = d[0], d1 = d[1];
-    st[8] = d0.x; st[9] = d0.y; st[10] = d0.z; st[11] = d0.w;
-    st[12] = d1.x; st[13] = d1.y; st[14] = d1.z; st[15] = d1.w;
-    permute<F>(st);
-    GLOBAL u32x4* o = reinterpret_cast<GLOBAL u32x4*>((gptr)next + 8 * i);
-    o[0] = u32x4{st[0], st[1], st[2], st[3]};
-    o[1] = u32x4{st[4], st[5], st[6], st[7]};
-}
-
 // ---- batched single-matrix commits --------------------------------------
 __device__ __forceinline__ int find_job(const uint64_t* __restrict__ prefix, int njobs, uint64_t i) {
     int lo = 0, hi = njobs;
@@ -353,68 +571,84 @@ __device__ __forceinline__ int find_job(const uint64_t* __restrict__ prefix, int
     return lo;
 }
 
-// Leaf layer of many jobs: thread -> (job, row); rows of any width.
+// Leaf layer of many jobs: wave -> (job, group of 64 rows); rows of any width.
 template <class F>
-__global__ void __launch_bounds__(256) leaf_hash_batch_kernel(const LeafJob* __restrict__ jobs,
-                                                              const uint64_t* __restrict__ prefix,
-                                                              int njobs, uint64_t total) {
-    const uint64_t gi = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= total) return;
-    const int j = find_job(prefix, njobs, gi);
-    const LeafJob jb = jobs[j];
-    const uint64_t row = gi - prefix[j];
-    const gcptr rp = (gcptr)jb.data + row * jb.stride;
-    uint32_t st[16];
+MX_KERNEL leaf_hash_batch_kernel(const LeafJob* __restrict__ jobs,
+                                                                     const uint64_t* __restrict__ prefix,
+                                                                     int njobs, uint64_t total) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    const uint64_t wave = mx_wave();
+    if (wave >= total) return;
+    const int j = __builtin_amdgcn_readfirstlane(find_job(prefix, njobs, wave));
+    const LeafJob* jb = jobs + j;
+    const uint64_t group = wave - prefix[j];
+    MxView<F> v(tab);
+    const MxLane l;
+    uint64_t row[2];
+    mx_group_rows(row, group, jb->rows, l);
+    const uint32_t width = jb->width;
+    gcptr rp[2];
 #pragma unroll
-    for (int t = 0; t < 16; t++) st[t] = 0;
-    const uint32_t full = jb.width / 8, tail = jb.width % 8;
-    if ((jb.width & 3u) == 0 && (jb.stride & 3u) == 0) {  // 16-byte aligned rows
-        const GLOBAL u32x4* r4 = reinterpret_cast<const GLOBAL u32x4*>(rp);
-        for (uint32_t c = 0; c < full; c++) {
-            const u32x4 a = r4[2 * c], b = r4[2 * c + 1];
-            st[0] = a.x; st[1] = a.y; st[2] = a.z; st[3] = a.w;
-            st[4] = b.x; st[5] = b.y; st[6] = b.z; st[7] = b.w;
-            permute<F>(st);
+    for (int t = 0; t < 2; t++) rp[t] = (gcptr)jb->data + row[t] * jb->stride + 4 * l.h;
+    MxSponge<F> sp;
+    auto load = [&](uint32_t off, u32x4 (&out)[2]) {  // words past the row's end read as word 0
+        if (off + 8 <= width) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) out[t] = *reinterpret_cast<const GLOBAL u32x4u*>(rp[t] + off);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) out[t][i] = rp[t][off + 4 * l.h + i < width ? (int64_t)(off + i) : -(int64_t)(4 * l.h)];
         }
-    } else {
-        for (uint32_t c = 0; c < full; c++) {
-#pragma unroll
-            for (int t = 0; t < 8; t++) st[t] = rp[8 * c + t];
-            permute<F>(st);
-        }
+    };
+    u32x4 next[2];
+    load(0, next);
+    for (uint32_t off = 0; off < width; off += 8) {
+        const u32x4 cur[2] = {next[0], next[1]};
+        if (off + 8 < width) load(off + 8, next);
+        sp.absorb(cur, width - off < 8u ? width - off : 8u, l.h, v);
     }
-    if (tail) {  // overwrite only the first `tail` state words
-        const gcptr tp = rp + 8 * full;
-#pragma unroll
-        for (int t = 0; t < 7; t++)
-            if ((uint32_t)t < tail) st[t] = tp[t];
-        permute<F>(st);
-    }
-    GLOBAL u32x4* o = reinterpret_cast<GLOBAL u32x4*>((gptr)jb.digests + 8 * row);
-    o[0] = u32x4{st[0], st[1], st[2], st[3]};
-    o[1] = u32x4{st[4], st[5], st[6], st[7]};
+    uint32_t st[2][8];
+    mx_last<F>(st, sp.b, v);
+    mx_store_digests(jb->digests, group, jb->rows, l, st);
 }
 
 template <class F>
-__global__ void __launch_bounds__(256) compress_batch_kernel(const CompressJob* __restrict__ jobs,
-                                                             const uint64_t* __restrict__ prefix,
-                                                             int njobs, uint64_t total) {
-    const uint64_t gi = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= total) return;
-    const int j = find_job(prefix, njobs, gi);
-    const CompressJob jb = jobs[j];
-    const uint64_t i = gi - prefix[j];
-    const GLOBAL u32x4* p = reinterpret_cast<const GLOBAL u32x4*>((gcptr)jb.prev + 16 * i);
-    uint32_t st[16];
+MX_KERNEL compress_batch_kernel(const CompressJob* __restrict__ jobs,
+                                                                    const uint64_t* __restrict__ prefix,
+                                                                    int njobs, uint64_t total) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    MxView<F> v(tab);
+    const MxLane l;
+    const uint64_t stride = (uint64_t)gridDim.x * MX_WAVES;
+    for (uint64_t group = mx_wave(); 64 * group < total; group += stride) {
+        uint64_t node[2];
+        mx_group_rows(node, group, total, l);
+        uint32_t* dst[2];
+        mx4 full[2][2], b[2][2];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const u32x4 v = p[q];
-        st[4 * q] = v.x; st[4 * q + 1] = v.y; st[4 * q + 2] = v.z; st[4 * q + 3] = v.w;
+        for (int t = 0; t < 2; t++) {  // each lane finds its own nodes' jobs
+            const int j = find_job(prefix, njobs, node[t]);
+            const uint64_t i = node[t] - prefix[j];
+            const gcptr src = (gcptr)jobs[j].prev + 16 * i + 4 * l.h;
+            dst[t] = jobs[j].next + 8 * i + 4 * l.h;
+#pragma unroll
+            for (int s = 0; s < 2; s++) full[t][s] = mx_op(*reinterpret_cast<const GLOBAL u32x4*>(src + 8 * s));
+        }
+        int x[2][8];
+        uint32_t st[2][8];
+        v.fresh();
+        mx_init<F>(x, full, v);
+        mx_rounds<F>(b, x, v);
+        mx_last<F>(st, b, v);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+            if (64 * group + 32 * t + l.n < total)
+                *reinterpret_cast<GLOBAL u32x4*>((gptr)dst[t]) = u32x4{st[t][0], st[t][1], st[t][2], st[t][3]};
     }
-    permute<F>(st);
-    GLOBAL u32x4* o = reinterpret_cast<GLOBAL u32x4*>((gptr)jb.next + 8 * i);
-    o[0] = u32x4{st[0], st[1], st[2], st[3]};
-    o[1] = u32x4{st[4], st[5], st[6], st[7]};
 }
 
 template <class F>
@@ -437,6 +671,11 @@ __global__ void gather_roots_kernel(const uint32_t* const* __restrict__ src, uin
 }
 
 static unsigned grid_for(uint64_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
+// workgroups for n rows, 64 per wave
+static unsigned mx_grid(uint64_t n) { return (unsigned)((n + 64 * MX_WAVES - 1) / (64 * MX_WAVES)); }
+// Compress kernels loop over the nodes with at most four workgroups per CU,
+// so the table load of a workgroup is shared by its waves' nodes.
+static unsigned mx_grid_loop(uint64_t n) { return std::min(mx_grid(n), 1024u); }
 
 hipError_t launch_gather_roots(const uint32_t* const* src, uint32_t* dst, int n, hipStream_t stream) {
     if (n == 0) return hipSuccess;
@@ -448,9 +687,9 @@ hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t
                                   uint64_t total, hipStream_t stream) {
     if (total == 0) return hipSuccess;
     if (field == FIELD_KOALABEAR)
-        leaf_hash_batch_kernel<KoalaBear><<<grid_for(total, 256), 256, 0, stream>>>(jobs, prefix, njobs, total);
+        leaf_hash_batch_kernel<KoalaBear><<<grid_for(total, MX_WAVES), MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
     else
-        leaf_hash_batch_kernel<BabyBear><<<grid_for(total, 256), 256, 0, stream>>>(jobs, prefix, njobs, total);
+        leaf_hash_batch_kernel<BabyBear><<<grid_for(total, MX_WAVES), MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
     return hipGetLastError();
 }
 
@@ -466,20 +705,20 @@ hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint6
         return hipGetLastError();
     }
     if (field == FIELD_KOALABEAR)
-        compress_batch_kernel<KoalaBear><<<grid_for(total, 256), 256, 0, stream>>>(jobs, prefix, njobs, total);
+        compress_batch_kernel<KoalaBear><<<mx_grid_loop(total), MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
     else
-        compress_batch_kernel<BabyBear><<<grid_for(total, 256), 256, 0, stream>>>(jobs, prefix, njobs, total);
+        compress_batch_kernel<BabyBear><<<mx_grid_loop(total), MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
     return hipGetLastError();
 }
 
 hipError_t launch_leaf_hash(int field, const MatRef* mats, int n, uint32_t total_width,
                             size_t rows, uint32_t* digests, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
-    const unsigned g = grid_for(rows, 256);
+    const unsigned g = mx_grid(rows);
     if (field == FIELD_KOALABEAR)
-        leaf_hash_kernel<KoalaBear><<<g, 256, 0, stream>>>(mats, n, total_width, rows, digests);
+        leaf_hash_kernel<KoalaBear><<<g, MX_THREADS, 0, stream>>>(mats, n, total_width, rows, digests);
     else
-        leaf_hash_kernel<BabyBear><<<g, 256, 0, stream>>>(mats, n, total_width, rows, digests);
+        leaf_hash_kernel<BabyBear><<<g, MX_THREADS, 0, stream>>>(mats, n, total_width, rows, digests);
     return hipGetLastError();
 }
 
@@ -491,19 +730,11 @@ hipError_t launch_absorb_segment(int field, const uint32_t* data, uint64_t strid
                                  hipStream_t stream) {
     if (rows == 0) return hipSuccess;
     if (pos0 > 7 || (!last && !state) || (last && !digests) || (!first && !state)) return hipErrorInvalidValue;
-    const bool vec = pos0 == 0 && width % 8 == 0 && stride % 4 == 0 && ((uintptr_t)data % 16) == 0;
-    const unsigned g = grid_for(rows, 256);
-    if (field == FIELD_KOALABEAR) {
-        if (vec)
-            absorb_segment_kernel<KoalaBear, true><<<g, 256, 0, stream>>>(data, stride, width, 0, first, last, rows, state, digests);
-        else
-            absorb_segment_kernel<KoalaBear, false><<<g, 256, 0, stream>>>(data, stride, width, pos0, first, last, rows, state, digests);
-    } else {
-        if (vec)
-            absorb_segment_kernel<BabyBear, true><<<g, 256, 0, stream>>>(data, stride, width, 0, first, last, rows, state, digests);
-        else
-            absorb_segment_kernel<BabyBear, false><<<g, 256, 0, stream>>>(data, stride, width, pos0, first, last, rows, state, digests);
-    }
+    const unsigned g = mx_grid(rows);
+    if (field == FIELD_KOALABEAR)
+        absorb_segment_kernel<KoalaBear><<<g, MX_THREADS, 0, stream>>>(data, stride, width, pos0, first, last, rows, state, digests);
+    else
+        absorb_segment_kernel<BabyBear><<<g, MX_THREADS, 0, stream>>>(data, stride, width, pos0, first, last, rows, state, digests);
     return hipGetLastError();
 }
 
@@ -518,11 +749,11 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
             leaf8_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(data, stride, rows, digests);
         return hipGetLastError();
     }
-    const unsigned g = grid_for(rows, 256);
+    const unsigned g = mx_grid(rows);
     if (field == FIELD_KOALABEAR)
-        leaf_hash_w8_kernel<KoalaBear><<<g, 256, 0, stream>>>(data, stride, width / 8, rows, digests);
+        leaf_hash_w8_kernel<KoalaBear><<<g, MX_THREADS, 0, stream>>>(data, stride, width / 8, rows, digests);
     else
-        leaf_hash_w8_kernel<BabyBear><<<g, 256, 0, stream>>>(data, stride, width / 8, rows, digests);
+        leaf_hash_w8_kernel<BabyBear><<<g, MX_THREADS, 0, stream>>>(data, stride, width / 8, rows, digests);
     return hipGetLastError();
 }
 
@@ -537,11 +768,18 @@ hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size
             compress_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(prev, next, n_out);
         return hipGetLastError();
     }
-    const unsigned g = grid_for(n_out, 256);
-    if (field == FIELD_KOALABEAR)
-        compress_kernel<KoalaBear><<<g, 256, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width);
-    else
-        compress_kernel<BabyBear><<<g, 256, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width);
+    const unsigned g = mx_grid_loop(n_out);
+    if (field == FIELD_KOALABEAR) {
+        if (n_inj > 0)
+            compress_kernel<KoalaBear, true><<<g, MX_THREADS, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width);
+        else
+            compress_kernel<KoalaBear, false><<<g, MX_THREADS, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width);
+    } else {
+        if (n_inj > 0)
+            compress_kernel<BabyBear, true><<<g, MX_THREADS, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width);
+        else
+            compress_kernel<BabyBear, false><<<g, MX_THREADS, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width);
+    }
     return hipGetLastError();
 }
 
@@ -556,11 +794,11 @@ hipError_t launch_compress_digest(int field, const uint32_t* prev, uint32_t* nex
             compress_digest_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(prev, inj, next, n_out);
         return hipGetLastError();
     }
-    const unsigned g = grid_for(n_out, 256);
+    const unsigned g = mx_grid_loop(n_out);
     if (field == FIELD_KOALABEAR)
-        compress_digest_kernel<KoalaBear><<<g, 256, 0, stream>>>(prev, inj, next, n_out);
+        compress_digest_kernel<KoalaBear><<<g, MX_THREADS, 0, stream>>>(prev, inj, next, n_out);
     else
-        compress_digest_kernel<BabyBear><<<g, 256, 0, stream>>>(prev, inj, next, n_out);
+        compress_digest_kernel<BabyBear><<<g, MX_THREADS, 0, stream>>>(prev, inj, next, n_out);
     return hipGetLastError();
 }
 

@@ -334,8 +334,7 @@ PG_HD void internal_layer_redc(uint32_t (&s)[16]) {
     }
 }
 
-// KoalaBear partial rounds per trip of their loop (the leaf-hash statistics
-// count the loop body this many times fewer than the rounds)
+// KoalaBear partial rounds per trip of their loop
 constexpr int P2_PARTIAL_UNROLL = 10;
 
 template <class F>

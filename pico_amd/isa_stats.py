@@ -2,14 +2,16 @@
 
 Compiles merkle.hip to device assembly and counts the VALU instructions one
 trip of the chunk loop of the single-matrix leaf-hash kernel executes (one
-sponge chunk = one Poseidon2 permutation plus its two 16-byte loads; a loop
-nested in it, KoalaBear's partial rounds, counted once per trip), per field,
-by opcode and by issue class.  Issue classes, from a per-opcode throughput microbenchmark on MI355X:
-  double   v_add_u32, v_sub_u32, v_subrev_u32, v_mov_b32, v_and_b32: up to
-           two per lane per clock (measured 64-70 T/s against the 39.3 T/s
-           single-issue ceiling), priced at half a slot
+sponge chunk: a wave permutes 64 states, so an instruction per wave is a lane
+slot per permutation), per field, by opcode and by issue class.  Issue
+classes, from a per-opcode throughput microbenchmark on MI355X:
+  double   v_add_u32, v_sub_u32, v_subrev_u32, v_mov_b32, v_and_b32,
+           v_xor_b32: up to two per lane per clock (measured 61-70 T/s against
+           the 39.3 T/s single-issue ceiling), priced at half a slot
   single   every other VALU opcode, one slot (the 32x32-bit multiplies and
-           64-bit adds measure at 0.90 of the ceiling, the rest at 0.97)
+           64-bit adds measure at 0.90 of the ceiling, the rest at 0.97); a
+           matrix instruction counts as the one slot it issues in (it keeps
+           the matrix core busy for 32 clocks beside the VALU)
 bench.py turns the slot count into the leaf hash's achieved issue rate.
 
 It also compiles ntt.hip and counts, for every instantiation of the LDE pass
@@ -47,7 +49,7 @@ def kernel_lines(asm, prefix):
     return out
 
 
-DOUBLE_ISSUE = {"v_add_u32", "v_sub_u32", "v_subrev_u32", "v_mov_b32", "v_and_b32"}
+DOUBLE_ISSUE = {"v_add_u32", "v_sub_u32", "v_subrev_u32", "v_mov_b32", "v_and_b32", "v_xor_b32"}
 
 
 def opcode(line):
@@ -136,31 +138,11 @@ def lde_stats(asm):
 
 def compile_asm(hipcc, src, asm_path):
     subprocess.run([hipcc, "-O3", "-std=c++17", "--offload-arch=gfx950", "-S", "--cuda-device-only",
+                    "-fconstexpr-steps=100000000",
                     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                     os.path.join(HERE, "csrc", src), "-o", asm_path],
                    check=True, stderr=subprocess.DEVNULL)
     return open(asm_path).read()
-
-
-def inner_loop(lines, body):
-    """The loop nested in `body` (the compiler's marker "Inner Loop Header:
-    Depth=2" to its backward branch), or []."""
-    start = next((i for i, l in enumerate(body) if "Loop Header: Depth=2" in l), None)
-    if start is None:
-        return []
-    m = re.match(r"^(\.LBB\w+):", body[start - 1] if not body[start].startswith(".LBB") else body[start])
-    label = m.group(1) if m else None
-    end = max((i for i, l in enumerate(body) if label and re.match(r"^\s+s_(?:cbranch_\w+|branch)\s+" + re.escape(label) + r"\b", l)),
-              default=None)
-    return body[start:end + 1] if end is not None else []
-
-
-def partial_trips():
-    """ROUNDS_P / P2_PARTIAL_UNROLL for KoalaBear (20 partial rounds), read
-    from poseidon2.h: the trips of the partial-round loop."""
-    src = open(os.path.join(HERE, "csrc", "poseidon2.h")).read()
-    unroll = int(re.search(r"constexpr int P2_PARTIAL_UNROLL = (\d+);", src).group(1))
-    return 20 // unroll
 
 
 def main(out_path):
@@ -173,11 +155,6 @@ def main(out_path):
         lines = kernel_lines(asm, prefix)
         body = loop_body(lines)
         hist = histogram(body)
-        # a nested loop (KoalaBear's partial rounds) runs `trips` times per chunk
-        inner = inner_loop(lines, body)
-        trips = partial_trips() if inner and field == "koalabear" else 1
-        for op, n in histogram(inner).items():
-            hist[op] = hist.get(op, 0) + (trips - 1) * n
         dbl = sum(n for op, n in hist.items() if op in DOUBLE_ISSUE)
         total = sum(hist.values())
         stats[field] = {
@@ -185,6 +162,7 @@ def main(out_path):
             "leaf_hash_w8_valu_per_chunk": total,
             "leaf_hash_w8_double_issue_per_chunk": dbl,
             "leaf_hash_w8_slots_per_chunk": (total - dbl) + 0.5 * dbl,
+            "leaf_hash_w8_mfma_per_chunk": sum(n for op, n in hist.items() if op.startswith("v_mfma")),
             "leaf_hash_w8_opcodes": dict(sorted(hist.items(), key=lambda kv: -kv[1])),
             "lde_kernels": ntt.get(field, []),
         }
