@@ -1183,16 +1183,34 @@ static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const st
         if (r < 0) return r;
         hashed = r == STAGE_HASHED;
     }
+    // layers below a layer of n nodes down to the next height that has
+    // matrices (their rows are hashed into that layer) or to the root
+    auto layers_below = [&](size_t n_, size_t g) {
+        int c = 0;
+        for (; n_ > 1 && !(g < n && mats[order[g]]->rows == n_ / 2); n_ /= 2) c++;
+        return c;
+    };
+    size_t len = H, off = 0, gi = g1;
     if (hashed) {
+    } else if (g1 - g0 == 1 && first->cols == 8 && H <= TREE_MAX_NODES) {
+        const int c = layers_below(H, g1);
+        TIMED(kt, "leaf_hash_w8", s, launch_tree_layers(field, first->ptr, 8, 1, H, 1 + c, t->digests, s));
+        for (int k = 0; k < c; k++, len /= 2) off += len;
     } else if (g1 - g0 == 1 && first->cols % 8 == 0 && first->cols > 0 && ((uintptr_t)first->ptr % 16) == 0)
         TIMED(kt, "leaf_hash_w8", s,
               launch_leaf_hash_w8(field, first->ptr, first->cols, (uint32_t)first->cols, H, t->digests, s));
     else
         TIMED(kt, "leaf_hash", s, launch_leaf_hash(field, d_sorted + g0, (int)(g1 - g0), wsum, H, t->digests, s));
     // compress + inject
-    size_t len = H, off = 0, gi = g1;
     while (len > 1) {
         const size_t nl = len / 2;
+        const int c = nl <= TREE_MAX_NODES ? layers_below(len, gi) : 0;
+        if (c) {
+            TIMED(kt, "compress", s,
+                  launch_tree_layers(field, t->digests + 8 * off, 0, 0, nl, c, t->digests + 8 * (off + len), s));
+            for (int k = 0; k < c; k++, len /= 2) off += len;
+            continue;
+        }
         size_t gj = gi;
         uint32_t iw = 0;
         while (gj < n && mats[order[gj]]->rows == nl) iw += (uint32_t)mats[order[gj++]]->cols;

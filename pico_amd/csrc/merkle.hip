@@ -103,19 +103,47 @@ __device__ __forceinline__ uint32_t permute_lanes(uint32_t x, int l) {
     return x;
 }
 
-// Layers of at most this many nodes (or leaves) take the 16-lane kernels:
-// above it the 16x larger thread count costs more than the latency saved.
-constexpr uint64_t LANES_MAX_NODES = 1u << 14;
+// Layers of at most this many nodes take the 16-lane kernels: above it the
+// 16x larger thread count costs more than the latency saved.
+constexpr uint64_t LANES_MAX_NODES = TREE_MAX_NODES;
 
-// next[i] = C(prev[2i], prev[2i+1]): the two child digests are the state.
-// Thread 16 i + l is lane l of node i; a node's 16 lanes leave together.
-template <class F>
-__global__ void __launch_bounds__(256) compress_lanes_kernel(const uint32_t* prev, uint32_t* next, uint64_t n_out) {
-    const uint64_t node = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
+// Several layers of a tree in one launch.  The first layer's n0 nodes are
+// C(in[2i], in[2i+1]) or, with LEAF8, the hashes of n0 rows of exactly 8 words
+// (one sponge chunk, st = (row, 0^8)); layers n0, n0/2, ... follow each other
+// at `out`, as a tree stores them.  A workgroup computes the `layers` layers
+// over its 2^log_per nodes of the first one: their children pass through LDS,
+// so a layer costs one permutation's latency (3.2 us) instead of a launch (4.3
+// us and the gap before it): the 9 layers above 512 leaves 32 us in two
+// launches, 45 us and more in nine.  16 lanes per node; a node's lanes stay
+// together.
+constexpr int TREE_THREADS = 1024;
+constexpr int TREE_MAX_PER = 128;  // first-layer nodes of a workgroup
+template <class F, bool LEAF8>
+__global__ void __launch_bounds__(TREE_THREADS) tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0,
+                                                                   int log_per, int layers, uint32_t* out) {
+    __shared__ uint32_t buf[2][8 * TREE_MAX_PER];
     const int l = (int)(threadIdx.x & 15u);
-    if (node >= n_out) return;
-    const uint32_t x = permute_lanes<F>(((gcptr)prev)[16 * node + l], l);
-    if (l < 8) ((gptr)next)[8 * node + l] = x;
+    gptr layer = (gptr)out;
+    for (int i = 0; i < layers; i++) {
+        const uint32_t cnt = (1u << log_per) >> i;
+        const uint64_t base = (uint64_t)blockIdx.x * cnt;
+        for (uint32_t nd = threadIdx.x >> 4; nd < cnt; nd += blockDim.x >> 4) {
+            uint32_t x;
+            if (i > 0)
+                x = buf[(i - 1) & 1][16 * nd + l];
+            else if constexpr (LEAF8)
+                x = l < 8 ? ((gcptr)in)[(base + nd) * stride + l] : 0u;
+            else
+                x = ((gcptr)in)[16 * (base + nd) + l];
+            x = permute_lanes<F>(x, l);
+            if (l < 8) {
+                buf[i & 1][8 * nd + l] = x;
+                layer[8 * (base + nd) + l] = x;
+            }
+        }
+        __syncthreads();
+        layer += 8 * (n0 >> i);
+    }
 }
 
 // next[i] = C(C(prev[2i], prev[2i+1]), inj[i]) with the digests inj[i] of the
@@ -131,17 +159,6 @@ __global__ void __launch_bounds__(256) compress_digest_lanes_kernel(const uint32
     uint32_t x = permute_lanes<F>(((gcptr)prev)[16 * node + l], l);
     x = permute_lanes<F>(l < 8 ? x : d, l);
     if (l < 8) ((gptr)next)[8 * node + l] = x;
-}
-
-// Rows of exactly 8 words: one sponge chunk, st = (row, 0^8).
-template <class F>
-__global__ void __launch_bounds__(256) leaf8_lanes_kernel(const uint32_t* data, uint64_t stride, uint64_t rows,
-                                                          uint32_t* digests) {
-    const uint64_t row = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    const int l = (int)(threadIdx.x & 15u);
-    if (row >= rows) return;
-    const uint32_t x = permute_lanes<F>(l < 8 ? ((gcptr)data)[row * stride + l] : 0u, l);
-    if (l < 8) ((gptr)digests)[8 * row + l] = x;
 }
 
 // ---- hashing on the matrix cores --------------------------------------------
@@ -741,14 +758,6 @@ hipError_t launch_absorb_segment(int field, const uint32_t* data, uint64_t strid
 hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride, uint32_t width,
                                size_t rows, uint32_t* digests, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
-    if (width == 8 && rows <= LANES_MAX_NODES) {
-        const unsigned g = grid_for(rows * 16, 256);
-        if (field == FIELD_KOALABEAR)
-            leaf8_lanes_kernel<KoalaBear><<<g, 256, 0, stream>>>(data, stride, rows, digests);
-        else
-            leaf8_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(data, stride, rows, digests);
-        return hipGetLastError();
-    }
     const unsigned g = mx_grid(rows);
     if (field == FIELD_KOALABEAR)
         leaf_hash_w8_kernel<KoalaBear><<<g, MX_THREADS, 0, stream>>>(data, stride, width / 8, rows, digests);
@@ -757,17 +766,44 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
     return hipGetLastError();
 }
 
+// Nodes (or 8-word rows) of the first layer, at most TREE_MAX_NODES: 64 per
+// workgroup and seven layers a launch, one workgroup for all the rest once a
+// layer has at most 128 nodes.
+template <class F>
+static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, bool leaf8, uint64_t n0, int layers, uint32_t* out,
+                                hipStream_t s) {
+    while (layers > 0) {
+        int log_per = 6;
+        if (n0 <= (uint64_t)TREE_MAX_PER)
+            log_per = __builtin_ctzll(n0);
+        const int now = std::min(layers, log_per + 1);
+        const unsigned threads = std::min((unsigned)TREE_THREADS, std::max(64u, 16u << log_per));
+        if (leaf8)
+            tree_layers_kernel<F, true><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, stride, n0, log_per, now, out);
+        else
+            tree_layers_kernel<F, false><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, 0, n0, log_per, now, out);
+        for (int i = 0; i < now; i++) {  // the last layer written feeds the next launch
+            in = out;
+            out += 8 * n0;
+            n0 >>= 1;
+        }
+        leaf8 = false;
+        layers -= now;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
+                              uint32_t* out, hipStream_t stream) {
+    if (layers <= 0) return hipSuccess;
+    if (n0 == 0 || n0 > TREE_MAX_NODES || (n0 & (n0 - 1)) || (n0 >> (layers - 1)) == 0) return hipErrorInvalidValue;
+    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf8 != 0, n0, layers, out, stream)
+                                    : tree_layers_t<BabyBear>(in, stride, leaf8 != 0, n0, layers, out, stream);
+}
+
 hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
                            const MatRef* inj, int n_inj, uint32_t inj_width, hipStream_t stream) {
     if (n_out == 0) return hipSuccess;
-    if (n_inj == 0 && n_out <= LANES_MAX_NODES) {
-        const unsigned g = grid_for(n_out * 16, 256);
-        if (field == FIELD_KOALABEAR)
-            compress_lanes_kernel<KoalaBear><<<g, 256, 0, stream>>>(prev, next, n_out);
-        else
-            compress_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(prev, next, n_out);
-        return hipGetLastError();
-    }
     const unsigned g = mx_grid_loop(n_out);
     if (field == FIELD_KOALABEAR) {
         if (n_inj > 0)
