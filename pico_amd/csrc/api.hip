@@ -1192,11 +1192,12 @@ static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const st
     };
     size_t len = H, off = 0, gi = g1;
     if (hashed) {
-    } else if (g1 - g0 == 1 && first->cols == 8 && H <= TREE_MAX_NODES) {
+    } else if (g1 - g0 == 1 && first->cols == 8 && H <= SMALL_MAX_NODES) {
         const int c = layers_below(H, g1);
         TIMED(kt, "leaf_hash_w8", s, launch_tree_layers(field, first->ptr, 8, 1, H, 1 + c, t->digests, s));
         for (int k = 0; k < c; k++, len /= 2) off += len;
-    } else if (g1 - g0 == 1 && first->cols % 8 == 0 && first->cols > 0 && ((uintptr_t)first->ptr % 16) == 0)
+    } else if (g1 - g0 == 1 && first->cols % 8 == 0 && first->cols > 0 && ((uintptr_t)first->ptr % 16) == 0 &&
+             H > SMALL_MAX_NODES)
         TIMED(kt, "leaf_hash_w8", s,
               launch_leaf_hash_w8(field, first->ptr, first->cols, (uint32_t)first->cols, H, t->digests, s));
     else
@@ -1204,7 +1205,7 @@ static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const st
     // compress + inject
     while (len > 1) {
         const size_t nl = len / 2;
-        const int c = nl <= TREE_MAX_NODES ? layers_below(len, gi) : 0;
+        const int c = nl <= SMALL_MAX_NODES ? layers_below(len, gi) : 0;
         if (c) {
             TIMED(kt, "compress", s,
                   launch_tree_layers(field, t->digests + 8 * off, 0, 0, nl, c, t->digests + 8 * (off + len), s));

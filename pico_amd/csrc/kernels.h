@@ -55,11 +55,11 @@ hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size
 // prev[2i+1]), inj[i]) for 8-word digests inj[i].
 hipError_t launch_compress_digest(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
                                   const uint32_t* inj, hipStream_t stream);
-// Up to log2(n0) + 1 layers of a tree at once, n0 <= TREE_MAX_NODES a power of
+// Up to log2(n0) + 1 layers of a tree at once, n0 <= SMALL_MAX_NODES a power of
 // two: the first layer's nodes are C(in[2i], in[2i+1]), or with leaf8 the
 // hashes of n0 rows of 8 words (row pitch `stride`); the layers n0, n0/2, ...
 // are written one after the other at out.
-constexpr uint64_t TREE_MAX_NODES = 1u << 14;
+constexpr uint64_t SMALL_MAX_NODES = 1u << 15;
 hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
                               uint32_t* out, hipStream_t stream);
 // Opening gather: for each query q < nq and matrix k, copy row

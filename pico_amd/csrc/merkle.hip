@@ -9,9 +9,9 @@
 //               exist: next[i] = C(next[i], H(concat of their row i))
 //   H = PaddingFreeSponge<16, 8, 8> (overwrite mode, circuit/hash.rs:40-52)
 //   C = TruncatedPermutation (circuit/hash.rs:89-94)
-// Layers of more than LANES_MAX_NODES nodes and every leaf hash run 64 states
-// per wave with the linear layers on the matrix cores (poseidon2_mx.h): the
-// grid deals groups of 64 rows or nodes to waves.
+// The linear layers run on the matrix cores (poseidon2_mx.h).  Layers of more
+// than SMALL_MAX_NODES rows or nodes take 64 states per wave, smaller ones 16:
+// the grid deals groups of that many rows or nodes to waves.
 #include <algorithm>
 
 #include "kernels.h"
@@ -19,147 +19,6 @@
 #include "poseidon2_mx.h"
 
 namespace pg {
-
-// ---- one permutation over 16 lanes ---------------------------------------
-// A layer with few nodes cannot fill the GPU, so with one state per thread it
-// costs one permutation's latency (about 5200 dependent VALU instructions,
-// ~11 us on MI355X) however small it is: the top ~15 layers of every tree
-// and the small FRI rounds.  For those layers the 16 lanes of a DPP row
-// (lanes 16r .. 16r+15 of a wave) hold one state, lane l holding s_l: the
-// S-boxes of a full round run side by side, and the linear layers take their
-// cross-lane terms from DPP moves (quad_perm inside groups of 4 lanes,
-// row_ror across the groups): about 35 dependent VALU instructions per
-// round, 983 per permutation against ~5200.  All arithmetic is on reduced
-// values, so the result is the same permutation word for word.
-static __constant__ P2Const<KoalaBear> kLaneKb = make_p2const<KoalaBear>();
-static __constant__ P2Const<BabyBear> kLaneBb = make_p2const<BabyBear>();
-
-template <class F>
-__device__ __forceinline__ const P2Const<F>& lane_consts() {
-    if constexpr (F::P == KoalaBear::P)
-        return kLaneKb;
-    else
-        return kLaneBb;
-}
-
-// v from lane CTRL selects, within the lane's DPP row (every lane active)
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_from(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
-}
-constexpr int DPP_QUAD_SWAP1 = 0xB1;  // quad_perm [1,0,3,2]
-constexpr int DPP_QUAD_SWAP2 = 0x4E;  // quad_perm [2,3,0,1]
-constexpr int DPP_QUAD_NEXT = 0x39;   // quad_perm [1,2,3,0]: lane i of a quad reads lane i+1
-constexpr int DPP_ROW_ROR4 = 0x124;
-constexpr int DPP_ROW_ROR8 = 0x128;
-
-// Sum over the lane's group of 4, then over the 4 groups: both orbits are
-// complete whichever way the moves rotate.
-template <class F>
-__device__ __forceinline__ uint32_t quad_sum(uint32_t x) {
-    const uint32_t a = fadd<F>(x, dpp_from<DPP_QUAD_SWAP1>(x));
-    return fadd<F>(a, dpp_from<DPP_QUAD_SWAP2>(a));
-}
-template <class F>
-__device__ __forceinline__ uint32_t across_quads(uint32_t y) {
-    const uint32_t u = fadd<F>(y, dpp_from<DPP_ROW_ROR4>(y));
-    return fadd<F>(u, dpp_from<DPP_ROW_ROR8>(u));
-}
-
-// External layer: M4 row i is (2, 3, 1, 1) rotated by i, i.e.
-// y_i = (x_0 + x_1 + x_2 + x_3) + x_i + 2 x_{i+1 mod 4}; then
-// s_i = y_i + sum over the four groups of y at position i mod 4.
-template <class F>
-__device__ __forceinline__ uint32_t external_lanes(uint32_t x) {
-    const uint32_t nx = dpp_from<DPP_QUAD_NEXT>(x);
-    const uint32_t y = fadd<F>(fadd<F>(quad_sum<F>(x), x), fadd<F>(nx, nx));
-    return fadd<F>(y, across_quads<F>(y));
-}
-
-// Internal layer: s_i = s_i diag_i + sum of all 16
-template <class F>
-__device__ __forceinline__ uint32_t internal_lanes(uint32_t x, uint32_t diag) {
-    return fadd<F>(fmul<F>(x, diag), across_quads<F>(quad_sum<F>(x)));
-}
-
-// x = s_l in, P(s)_l out; l = lane index within the DPP row.
-template <class F>
-__device__ __forceinline__ uint32_t permute_lanes(uint32_t x, int l) {
-    const P2Const<F>& K = lane_consts<F>();
-    uint32_t rc[8];
-#pragma unroll
-    for (int r = 0; r < 8; r++) rc[r] = K.ext_rc[r][l];
-    const uint32_t diag = K.diag[l];
-    x = external_lanes<F>(x);
-#pragma unroll
-    for (int r = 0; r < 4; r++) x = external_lanes<F>(sbox<F>(fadd<F>(x, rc[r])));
-#pragma unroll
-    for (int r = 0; r < F::ROUNDS_P; r++) {
-        const uint32_t v = sbox<F>(fadd<F>(x, P2<F>::K.int_rc[r]));
-        x = internal_lanes<F>(l == 0 ? v : x, diag);
-    }
-#pragma unroll
-    for (int r = 4; r < 8; r++) x = external_lanes<F>(sbox<F>(fadd<F>(x, rc[r])));
-    return x;
-}
-
-// Layers of at most this many nodes take the 16-lane kernels: above it the
-// 16x larger thread count costs more than the latency saved.
-constexpr uint64_t LANES_MAX_NODES = TREE_MAX_NODES;
-
-// Several layers of a tree in one launch.  The first layer's n0 nodes are
-// C(in[2i], in[2i+1]) or, with LEAF8, the hashes of n0 rows of exactly 8 words
-// (one sponge chunk, st = (row, 0^8)); layers n0, n0/2, ... follow each other
-// at `out`, as a tree stores them.  A workgroup computes the `layers` layers
-// over its 2^log_per nodes of the first one: their children pass through LDS,
-// so a layer costs one permutation's latency (3.2 us) instead of a launch (4.3
-// us and the gap before it): the 9 layers above 512 leaves 32 us in two
-// launches, 45 us and more in nine.  16 lanes per node; a node's lanes stay
-// together.
-constexpr int TREE_THREADS = 1024;
-constexpr int TREE_MAX_PER = 128;  // first-layer nodes of a workgroup
-template <class F, bool LEAF8>
-__global__ void __launch_bounds__(TREE_THREADS) tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0,
-                                                                   int log_per, int layers, uint32_t* out) {
-    __shared__ uint32_t buf[2][8 * TREE_MAX_PER];
-    const int l = (int)(threadIdx.x & 15u);
-    gptr layer = (gptr)out;
-    for (int i = 0; i < layers; i++) {
-        const uint32_t cnt = (1u << log_per) >> i;
-        const uint64_t base = (uint64_t)blockIdx.x * cnt;
-        for (uint32_t nd = threadIdx.x >> 4; nd < cnt; nd += blockDim.x >> 4) {
-            uint32_t x;
-            if (i > 0)
-                x = buf[(i - 1) & 1][16 * nd + l];
-            else if constexpr (LEAF8)
-                x = l < 8 ? ((gcptr)in)[(base + nd) * stride + l] : 0u;
-            else
-                x = ((gcptr)in)[16 * (base + nd) + l];
-            x = permute_lanes<F>(x, l);
-            if (l < 8) {
-                buf[i & 1][8 * nd + l] = x;
-                layer[8 * (base + nd) + l] = x;
-            }
-        }
-        __syncthreads();
-        layer += 8 * (n0 >> i);
-    }
-}
-
-// next[i] = C(C(prev[2i], prev[2i+1]), inj[i]) with the digests inj[i] of the
-// injected rows computed beforehand: the second state is the first one's
-// output with its upper half replaced by inj[i].
-template <class F>
-__global__ void __launch_bounds__(256) compress_digest_lanes_kernel(const uint32_t* prev, const uint32_t* inj,
-                                                                    uint32_t* next, uint64_t n_out) {
-    const uint64_t node = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    const int l = (int)(threadIdx.x & 15u);
-    if (node >= n_out) return;
-    const uint32_t d = l < 8 ? 0u : ((gcptr)inj)[8 * node + (l - 8)];
-    uint32_t x = permute_lanes<F>(((gcptr)prev)[16 * node + l], l);
-    x = permute_lanes<F>(l < 8 ? x : d, l);
-    if (l < 8) ((gptr)next)[8 * node + l] = x;
-}
 
 // ---- hashing on the matrix cores --------------------------------------------
 // What bounds it: VALU issue, now of the S-boxes and the layer reductions.
@@ -201,12 +60,13 @@ struct MxRows {
         }
     }
     // cnt words of the chunk exist; the others read as word 0
-    __device__ __forceinline__ void chunk(u32x4 (&out)[2], const uint64_t (&row)[2], uint32_t cnt, uint32_t h) {
+    template <int T>
+    __device__ __forceinline__ void chunk(u32x4 (&out)[T], const uint64_t (&row)[T], uint32_t cnt, uint32_t h) {
         skip_ended();
         if (cnt == 8 && j + 8 <= mats[k].width) {  // within one matrix
             const gcptr base = (gcptr)mats[k].data + (j + 4 * h);
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < T; t++)
                 out[t] = *reinterpret_cast<const GLOBAL u32x4u*>(base + row[t] * mats[k].stride);
             j += 8;
             return;
@@ -230,7 +90,7 @@ struct MxRows {
             const gcptr q = (gcptr)(h ? p[4 + i] : p[i]);
             const uint64_t ld = h ? st[4 + i] : st[i];
 #pragma unroll
-            for (int t = 0; t < 2; t++) out[t][i] = q[row[t] * ld];
+            for (int t = 0; t < T; t++) out[t][i] = q[row[t] * ld];
         }
     }
 };
@@ -559,6 +419,119 @@ MX_KERNEL compress_digest_kernel(const uint32_t* prev, const uint32_t* inj,
     }
 }
 
+// ---- small layers: 16 states per wave ------------------------------------------
+// A layer costs a permutation's latency however few nodes it has: 2.2 us this
+// way, 7 us with 64 states per wave.  Up to SMALL_MAX_NODES (2^15: two waves
+// per SIMD) it is the faster form: one layer of 2^15 nodes 6.7 against 8.1 us,
+// two-chunk leaves of 2^15 rows 10.8 against 14.8 us; at 2^16 the 64-state form
+// still takes one wave per SIMD (8.8 us) and this one four.
+constexpr int S_WAVES = 4;
+constexpr int S_THREADS = 64 * S_WAVES;
+#define MX16_KERNEL __global__ void __launch_bounds__(S_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// the lane's state in its wave and its quarter of the words
+struct Mx16Lane {
+    uint32_t n, q;
+    __device__ __forceinline__ Mx16Lane() : n(threadIdx.x & 15u), q((threadIdx.x & 63u) >> 4) {}
+};
+__device__ __forceinline__ uint32_t mx16_wave() { return (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// Digest (lane groups 0 and 1) of row `row` of the concatenated matrices; the
+// whole wave calls it.
+template <class F>
+__device__ __forceinline__ u32x4 mx16_hash_rows(const Mx16<F>& P, MxRows src, uint64_t row, uint32_t total, uint32_t q) {
+    const uint64_t rows1[1] = {row};
+    const uint32_t h = q & 1u;
+    u32x4 next[1] = {u32x4{0}};
+    if (total) src.chunk<1>(next, rows1, total < 8u ? total : 8u, h);
+    mx4 st = mx4{0};
+#pragma clang loop unroll(disable)
+    for (uint32_t off = 0; off < total; off += 8) {
+        const u32x4 cur = next[0];
+        const uint32_t left = total - off;
+        if (left > 8) src.chunk<1>(next, rows1, left - 8 < 8u ? left - 8 : 8u, h);  // in flight
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (4 * q + i < (left < 8u ? left : 8u)) st[i] = (int)cur[i];
+        st = P.permute(Mx16<F>::op(st));
+    }
+    return mx16_words<F>(st);
+}
+
+template <class F>
+MX16_KERNEL leaf_hash_small_kernel(const MatRef* mats, int n, uint32_t total, uint64_t rows, uint32_t* digests) {
+    const Mx16<F> P;
+    const Mx16Lane l;
+    const uint64_t r = ((uint64_t)blockIdx.x * S_WAVES + mx16_wave()) * 16 + l.n;
+    const u32x4 d = mx16_hash_rows<F>(P, MxRows(mats, n), r < rows ? r : rows - 1, total, l.q);
+    if (r < rows && l.q < 2) *reinterpret_cast<GLOBAL u32x4*>((gptr)digests + 8 * r + 4 * l.q) = d;
+}
+
+// next[i] = C(C(prev[2i], prev[2i+1]), x_i): x_i the hash of rows i of inj, or
+// inj_digests[i] when that is given
+template <class F>
+MX16_KERNEL compress_small_kernel(const uint32_t* prev, uint32_t* next, uint64_t n_out, const MatRef* inj, int n_inj,
+                                  uint32_t inj_width, const uint32_t* inj_digests) {
+    const Mx16<F> P;
+    const Mx16Lane l;
+    const uint64_t r = ((uint64_t)blockIdx.x * S_WAVES + mx16_wave()) * 16 + l.n;
+    const uint64_t rr = r < n_out ? r : n_out - 1;
+    u32x4 d;  // group q: words 4 (q & 1) .. of x_i
+    if (inj_digests) {
+        d = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)inj_digests + 8 * rr + 4 * (l.q & 1u));
+    } else {
+        d = mx16_hash_rows<F>(P, MxRows(inj, n_inj), rr, inj_width, l.q);
+#pragma unroll
+        for (int i = 0; i < 4; i++)  // groups 2 and 3 read groups 0 and 1
+            d[i] = __builtin_amdgcn_permlane32_swap(d[i], d[i], false, false)[0];
+    }
+    const u32x4 w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)prev + 16 * rr + 4 * l.q);
+    mx4 st = __builtin_bit_cast(mx4, w);
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < 2; k++) {
+        if (k && l.q >= 2) st = __builtin_bit_cast(mx4, d);
+        st = P.permute(Mx16<F>::op(st));
+    }
+    if (r < n_out && l.q < 2) *reinterpret_cast<GLOBAL u32x4*>((gptr)next + 8 * r + 4 * l.q) = mx16_words<F>(st);
+}
+
+// Several layers of a tree in one launch.  The first layer's n0 nodes are
+// C(in[2i], in[2i+1]) or, with LEAF8, the hashes of n0 rows of exactly 8 words
+// (one sponge chunk, st = (row, 0^8)); layers n0, n0/2, ... follow each other
+// at `out`, as a tree stores them.  A workgroup computes the `layers` layers
+// over its 2^log_per nodes of the first one: their children pass through LDS,
+// so a layer costs one permutation's latency instead of a launch (4.3 us and
+// the gap before it).
+constexpr int TREE_MAX_PER = 128;  // first-layer nodes of a workgroup
+template <class F, bool LEAF8>
+MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0, int log_per, int layers, uint32_t* out) {
+    __shared__ u32x4 buf[2][2 * TREE_MAX_PER];
+    const Mx16<F> P;
+    const Mx16Lane l;
+    const uint32_t wave = mx16_wave(), waves = blockDim.x >> 6;
+    gptr layer = (gptr)out;
+    for (int i = 0; i < layers; i++) {
+        const uint32_t cnt = (1u << log_per) >> i;
+        const uint64_t base = (uint64_t)blockIdx.x * cnt;
+        for (uint32_t g = wave; 16 * g < cnt; g += waves) {  // the wave's group of 16 nodes
+            const uint32_t nd = 16 * g + l.n, nr = nd < cnt ? nd : cnt - 1;
+            u32x4 w;
+            if (i > 0)
+                w = buf[(i - 1) & 1][4 * nr + l.q];
+            else if constexpr (LEAF8)
+                w = l.q < 2 ? u32x4(*reinterpret_cast<const GLOBAL u32x4u*>((gcptr)in + (base + nr) * stride + 4 * l.q)) : u32x4{0};
+            else
+                w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)in + 16 * (base + nr) + 4 * l.q);
+            w = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
+            if (l.q < 2 && nd < cnt) {
+                buf[i & 1][2 * nd + l.q] = w;
+                *reinterpret_cast<GLOBAL u32x4*>(layer + 8 * (base + nd) + 4 * l.q) = w;
+            }
+        }
+        __syncthreads();
+        layer += 8 * (n0 >> i);
+    }
+}
+
 __global__ void open_gather_kernel(const MatRef* mats, const uint32_t* shift,
                                    const uint32_t* col_off, int n_mats, uint32_t total_width,
                                    const uint32_t* digests, const uint64_t* layer_off, int log_h,
@@ -669,17 +642,17 @@ MX_KERNEL compress_batch_kernel(const CompressJob* __restrict__ jobs,
 }
 
 template <class F>
-__global__ void __launch_bounds__(256) compress_batch_lanes_kernel(const CompressJob* __restrict__ jobs,
-                                                                   const uint64_t* __restrict__ prefix,
-                                                                   int njobs, uint64_t total) {
-    const uint64_t gi = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    const int l = (int)(threadIdx.x & 15u);
-    if (gi >= total) return;
-    const int j = find_job(prefix, njobs, gi);
-    const CompressJob jb = jobs[j];
-    const uint64_t i = gi - prefix[j];
-    const uint32_t x = permute_lanes<F>(((gcptr)jb.prev)[16 * i + l], l);
-    if (l < 8) ((gptr)jb.next)[8 * i + l] = x;
+MX16_KERNEL compress_batch_small_kernel(const CompressJob* __restrict__ jobs, const uint64_t* __restrict__ prefix,
+                                        int njobs, uint64_t total) {
+    const Mx16<F> P;
+    const Mx16Lane l;
+    const uint64_t r = ((uint64_t)blockIdx.x * S_WAVES + mx16_wave()) * 16 + l.n;
+    const uint64_t rr = r < total ? r : total - 1;
+    const int j = find_job(prefix, njobs, rr);
+    const uint64_t i = rr - prefix[j];
+    const u32x4 w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)jobs[j].prev + 16 * i + 4 * l.q);
+    const u32x4 d = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
+    if (r < total && l.q < 2) *reinterpret_cast<GLOBAL u32x4*>((gptr)jobs[j].next + 8 * i + 4 * l.q) = d;
 }
 
 __global__ void gather_roots_kernel(const uint32_t* const* __restrict__ src, uint32_t* __restrict__ dst, int n) {
@@ -690,6 +663,8 @@ __global__ void gather_roots_kernel(const uint32_t* const* __restrict__ src, uin
 static unsigned grid_for(uint64_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 // workgroups for n rows, 64 per wave
 static unsigned mx_grid(uint64_t n) { return (unsigned)((n + 64 * MX_WAVES - 1) / (64 * MX_WAVES)); }
+// workgroups for n rows or nodes, 16 per wave
+static unsigned small_grid(uint64_t n) { return (unsigned)((n + 16 * S_WAVES - 1) / (16 * S_WAVES)); }
 // Compress kernels loop over the nodes with at most four workgroups per CU,
 // so the table load of a workgroup is shared by its waves' nodes.
 static unsigned mx_grid_loop(uint64_t n) { return std::min(mx_grid(n), 1024u); }
@@ -713,12 +688,12 @@ hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t
 hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint64_t* prefix, int njobs,
                                  uint64_t total, hipStream_t stream) {
     if (total == 0) return hipSuccess;
-    if (total <= LANES_MAX_NODES) {
-        const unsigned g = grid_for(total * 16, 256);
+    if (total <= SMALL_MAX_NODES) {
+        const unsigned g = small_grid(total);
         if (field == FIELD_KOALABEAR)
-            compress_batch_lanes_kernel<KoalaBear><<<g, 256, 0, stream>>>(jobs, prefix, njobs, total);
+            compress_batch_small_kernel<KoalaBear><<<g, S_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
         else
-            compress_batch_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(jobs, prefix, njobs, total);
+            compress_batch_small_kernel<BabyBear><<<g, S_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
         return hipGetLastError();
     }
     if (field == FIELD_KOALABEAR)
@@ -731,6 +706,13 @@ hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint6
 hipError_t launch_leaf_hash(int field, const MatRef* mats, int n, uint32_t total_width,
                             size_t rows, uint32_t* digests, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
+    if (rows <= SMALL_MAX_NODES) {
+        if (field == FIELD_KOALABEAR)
+            leaf_hash_small_kernel<KoalaBear><<<small_grid(rows), S_THREADS, 0, stream>>>(mats, n, total_width, rows, digests);
+        else
+            leaf_hash_small_kernel<BabyBear><<<small_grid(rows), S_THREADS, 0, stream>>>(mats, n, total_width, rows, digests);
+        return hipGetLastError();
+    }
     const unsigned g = mx_grid(rows);
     if (field == FIELD_KOALABEAR)
         leaf_hash_kernel<KoalaBear><<<g, MX_THREADS, 0, stream>>>(mats, n, total_width, rows, digests);
@@ -766,7 +748,7 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
     return hipGetLastError();
 }
 
-// Nodes (or 8-word rows) of the first layer, at most TREE_MAX_NODES: 64 per
+// Nodes (or 8-word rows) of the first layer, at most SMALL_MAX_NODES: 64 per
 // workgroup and seven layers a launch, one workgroup for all the rest once a
 // layer has at most 128 nodes.
 template <class F>
@@ -777,7 +759,7 @@ static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, bool leaf8,
         if (n0 <= (uint64_t)TREE_MAX_PER)
             log_per = __builtin_ctzll(n0);
         const int now = std::min(layers, log_per + 1);
-        const unsigned threads = std::min((unsigned)TREE_THREADS, std::max(64u, 16u << log_per));
+        const unsigned threads = std::min((unsigned)S_THREADS, std::max(64u, 4u << log_per));
         if (leaf8)
             tree_layers_kernel<F, true><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, stride, n0, log_per, now, out);
         else
@@ -796,7 +778,7 @@ static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, bool leaf8,
 hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
                               uint32_t* out, hipStream_t stream) {
     if (layers <= 0) return hipSuccess;
-    if (n0 == 0 || n0 > TREE_MAX_NODES || (n0 & (n0 - 1)) || (n0 >> (layers - 1)) == 0) return hipErrorInvalidValue;
+    if (n0 == 0 || n0 > SMALL_MAX_NODES || (n0 & (n0 - 1)) || (n0 >> (layers - 1)) == 0) return hipErrorInvalidValue;
     return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf8 != 0, n0, layers, out, stream)
                                     : tree_layers_t<BabyBear>(in, stride, leaf8 != 0, n0, layers, out, stream);
 }
@@ -804,6 +786,13 @@ hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, in
 hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
                            const MatRef* inj, int n_inj, uint32_t inj_width, hipStream_t stream) {
     if (n_out == 0) return hipSuccess;
+    if (n_inj > 0 && n_out <= SMALL_MAX_NODES) {
+        if (field == FIELD_KOALABEAR)
+            compress_small_kernel<KoalaBear><<<small_grid(n_out), S_THREADS, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width, nullptr);
+        else
+            compress_small_kernel<BabyBear><<<small_grid(n_out), S_THREADS, 0, stream>>>(prev, next, n_out, inj, n_inj, inj_width, nullptr);
+        return hipGetLastError();
+    }
     const unsigned g = mx_grid_loop(n_out);
     if (field == FIELD_KOALABEAR) {
         if (n_inj > 0)
@@ -822,12 +811,11 @@ hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size
 hipError_t launch_compress_digest(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
                                   const uint32_t* inj, hipStream_t stream) {
     if (n_out == 0) return hipSuccess;
-    if (n_out <= LANES_MAX_NODES) {
-        const unsigned g = grid_for(n_out * 16, 256);
+    if (n_out <= SMALL_MAX_NODES) {
         if (field == FIELD_KOALABEAR)
-            compress_digest_lanes_kernel<KoalaBear><<<g, 256, 0, stream>>>(prev, inj, next, n_out);
+            compress_small_kernel<KoalaBear><<<small_grid(n_out), S_THREADS, 0, stream>>>(prev, next, n_out, nullptr, 0, 0, inj);
         else
-            compress_digest_lanes_kernel<BabyBear><<<g, 256, 0, stream>>>(prev, inj, next, n_out);
+            compress_small_kernel<BabyBear><<<small_grid(n_out), S_THREADS, 0, stream>>>(prev, next, n_out, nullptr, 0, 0, inj);
         return hipGetLastError();
     }
     const unsigned g = mx_grid_loop(n_out);

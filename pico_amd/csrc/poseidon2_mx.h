@@ -115,11 +115,21 @@ constexpr int mx_digit(int32_t v, int plane) {
     return d;
 }
 
+// the four bytes by which coefficient c enters digit plane `plane`
+template <class F>
+constexpr uint32_t mx_operand_word(uint64_t c, int plane) {
+    uint32_t word = 0;
+    for (int b = 0; b < 4 && c; b++) {
+        const uint64_t v = ((c << (16 + 8 * (b & 1))) % F::P << (b >= 2 ? 16 : 0)) % F::P;
+        word |= (uint32_t)(mx_digit(mx_centered(v, F::P), plane) & 255) << (8 * b);
+    }
+    return word;
+}
+
 template <class F>
 constexpr uint64_t mx_external(int r, int c) {
     return M4_COEF[r % 4][c % 4] * ((r / 4 == c / 4) ? 2u : 1u);
 }
-constexpr uint32_t mx_reduce_once(uint64_t v, uint32_t p) { return (uint32_t)(v % p); }
 
 template <class F>
 constexpr uint64_t mx_diag(int i) {  // canonical internal diagonal
@@ -135,15 +145,8 @@ constexpr void mx_fill(uint32_t (&a)[64][4], const MxLin& L, In input, Row row) 
         int out = -1, plane = 0;
         row(lane % 32, out, plane);
         for (int i = 0; i < 4; i++) {
-            uint32_t word = 0;
             const int in = input(lane / 32, i);
-            if (out >= 0 && in >= 0 && L.m[out][in])
-                for (int b = 0; b < 4; b++) {
-                    const uint64_t c = (L.m[out][in] << (16 + 8 * (b & 1))) % F::P;
-                    const uint64_t cb = (c << (b >= 2 ? 16 : 0)) % F::P;
-                    word |= (uint32_t)(mx_digit(mx_centered(cb, F::P), plane) & 255) << (8 * b);
-                }
-            a[lane][i] = word;
+            a[lane][i] = out >= 0 && in >= 0 ? mx_operand_word<F>(L.m[out][in], plane) : 0;
         }
     }
 }
@@ -190,21 +193,83 @@ constexpr void mx_state_step(uint32_t (&a)[64][4], const MxLin& L, int in0, int 
 // 2 h + i % 2
 constexpr int mx_round(int pair, int h, int i) { return 8 * pair + 4 * (i / 2) + 2 * h + i % 2; }
 
+// The permutation's linear layers (see above); `forms` row r: round r's form
+// over the state words and the x' of the blocks of four before its own.
+template <class F>
+struct MxParts {
+    MxLin ext, merged, fin;
+    uint64_t forms[F::ROUNDS_P][40];
+};
+template <class F>
+constexpr MxParts<F> make_mx_parts() {
+    constexpr uint64_t p = F::P;
+    constexpr int RP = F::ROUNDS_P;
+    MxParts<F> t{};
+    for (int r = 0; r < 16; r++)
+        for (int c = 0; c < 16; c++) t.ext.m[r][c] = mx_external<F>(r, c);
+    // the last external layer of one permutation and the first of the next,
+    // whose rate words are overwritten: the capacity words' share
+    for (int r = 0; r < 16; r++) {
+        for (int e = 0; e < 16; e++) {
+            uint64_t v = 0;
+            for (int c = 8; c < 16; c++) v += t.ext.m[r][c] * t.ext.m[c][e];
+            t.merged.m[r][e] = v % p;
+        }
+        t.merged.k[r] = P2<F>::K.ext_rc[0][r];
+        for (int c = 0; c < 8; c++)  // the new rate words' byte offsets
+            t.merged.k[r] = (t.merged.k[r] + t.ext.m[r][c] * 0x808080u) % p;
+    }
+    // partial rounds: columns P^k q, rows e_0 P^r and P^RP over the state
+    uint64_t d[16] = {};
+    for (int i = 0; i < 16; i++) d[i] = mx_diag<F>(i);
+    uint64_t pq[24][16] = {};
+    for (int i = 0; i < 16; i++) pq[0][i] = i == 0 ? (d[0] + 1) % p : 1;
+    for (int k = 1; k < RP; k++) {
+        uint64_t sum = 0;
+        for (int i = 1; i < 16; i++) sum += pq[k - 1][i];
+        for (int i = 0; i < 16; i++) pq[k][i] = (sum + (i ? d[i] * pq[k - 1][i] : 0)) % p;
+    }
+    uint64_t pw[16][16] = {};  // P^r
+    for (int i = 0; i < 16; i++) pw[i][i] = 1;
+    for (int r = 0; r <= RP; r++) {
+        for (int o = 0; o < (r < RP ? 1 : 16); o++)
+            for (int c = 0; c < 16; c++) {
+                uint64_t v = 0;
+                for (int k = 0; k < 16; k++) v += pw[o][k] * t.ext.m[k][c] % p;
+                if (r < RP)
+                    t.forms[r][c] = v % p;
+                else
+                    t.fin.m[o][c] = v % p;
+            }
+        for (int c = 0; c < 16; c++) {  // pw <- P pw
+            uint64_t sum = 0;
+            for (int i = 1; i < 16; i++) sum += pw[i][c];
+            for (int i = 0; i < 16; i++) pw[i][c] = (sum + (i ? d[i] * pw[i][c] : 0)) % p;
+        }
+    }
+    for (int r = 0; r < RP; r++)
+        for (int j = 0; j < r / 4 * 4; j++) t.forms[r][16 + j] = pq[r - 1 - j][0];
+    for (int o = 0; o < 16; o++) {
+        for (int j = 0; j < RP; j++) t.fin.m[o][16 + j] = pq[RP - 1 - j][o];
+        t.fin.k[o] = P2<F>::K.ext_rc[4][o];
+    }
+    return t;
+}
+
 template <class F>
 constexpr MxTable<F> make_mx_table() {
     using S = MxShape<F>;
-    constexpr uint64_t p = F::P;
     constexpr int RP = F::ROUNDS_P;
     MxTable<F> t{};
-    const uint64_t rinv = cpow_canon(F::P, (uint32_t)((1ull << 32) % p), F::P - 2);
-    (void)rinv;
-    // external layer
-    MxLin ext{};
-    for (int r = 0; r < 16; r++)
-        for (int c = 0; c < 16; c++) ext.m[r][c] = mx_external<F>(r, c);
+    const MxParts<F> parts = make_mx_parts<F>();
+    MxLin ext = parts.ext;
     for (int s = 0; s < 2; s++)
-        for (int y = 0; y < 2; y++) mx_state_step<F>(t.a[S::EXT + 2 * s + y], ext, 8 * s, y);
-    // its biases with each round's constants (words are in Montgomery form)
+        for (int y = 0; y < 2; y++) {
+            mx_state_step<F>(t.a[S::EXT + 2 * s + y], ext, 8 * s, y);
+            mx_state_step<F>(t.a[S::MERGED + 2 * s + y], parts.merged, 8 * s, y);
+        }
+    // the external layer's biases with each round's constants (words are in
+    // Montgomery form)
     auto ext_bias = [&](int slot, int round) {
         for (int i = 0; i < 16; i++) ext.k[i] = round < 0 ? 0 : P2<F>::K.ext_rc[round][i];
         mx_state_bias<F>(t.c[slot], ext, 16);
@@ -212,67 +277,11 @@ constexpr MxTable<F> make_mx_table() {
     ext_bias(S::B_INIT, 0);
     for (int r = 0; r < 8; r++)
         if (r != 3) ext_bias(S::B_EXT + r, r == 7 ? -1 : r + 1);
-    // the last external layer of one permutation and the first of the next,
-    // whose rate words are overwritten: the capacity words' share
-    MxLin mrg{};
-    for (int r = 0; r < 16; r++)
-        for (int e = 0; e < 16; e++) {
-            uint64_t v = 0;
-            for (int c = 8; c < 16; c++) v += ext.m[r][c] * ext.m[c][e];
-            mrg.m[r][e] = v % p;
-        }
-    for (int s = 0; s < 2; s++)
-        for (int y = 0; y < 2; y++) mx_state_step<F>(t.a[S::MERGED + 2 * s + y], mrg, 8 * s, y);
-    for (int i = 0; i < 16; i++) {
-        mrg.k[i] = P2<F>::K.ext_rc[0][i];
-        for (int c = 0; c < 8; c++) mrg.k[i] = (mrg.k[i] + ext.m[i][c] * 0x808080u) % p;  // the new rate words
-    }
-    mx_state_bias<F>(t.c[S::B_MERGED], mrg, 16);
-    // partial rounds: rows e_0 P^r and P^RP over the state, columns P^k q
-    uint64_t d[16] = {};
-    for (int i = 0; i < 16; i++) d[i] = mx_diag<F>(i);
-    uint64_t pq[24][16] = {};  // P^k q
-    for (int i = 0; i < 16; i++) pq[0][i] = i == 0 ? (d[0] + 1) % p : 1;
-    for (int k = 1; k < RP; k++) {
-        uint64_t sum = 0;
-        for (int i = 1; i < 16; i++) sum += pq[k - 1][i];
-        for (int i = 0; i < 16; i++) pq[k][i] = (sum + (i ? d[i] * pq[k - 1][i] : 0)) % p;
-    }
-    // row vectors: state -> state at partial round r, entry 0; kept as
-    // columns: col[i] = P^r e_i for every i
-    uint64_t pw[16][16] = {};  // P^r, [row][col]
-    for (int i = 0; i < 16; i++) pw[i][i] = 1;
-    MxLin fin{};
-    uint64_t form[24][16] = {};  // e_0 P^r M_E
-    for (int r = 0; r <= RP; r++) {
-        if (r < RP) {
-            for (int c = 0; c < 16; c++) {
-                uint64_t v = 0;
-                for (int k = 0; k < 16; k++) v += pw[0][k] * ext.m[k][c] % p;
-                form[r][c] = v % p;
-            }
-            for (int c = 0; c < 16; c++) {  // pw <- P pw
-                uint64_t sum = 0;
-                for (int i = 1; i < 16; i++) sum += pw[i][c];
-                for (int i = 0; i < 16; i++) pw[i][c] = (sum + (i ? d[i] * pw[i][c] : 0)) % p;
-            }
-        } else {
-            for (int o = 0; o < 16; o++)
-                for (int c = 0; c < 16; c++) {
-                    uint64_t v = 0;
-                    for (int k = 0; k < 16; k++) v += pw[o][k] * ext.m[k][c] % p;
-                    fin.m[o][c] = v % p;
-                }
-        }
-    }
-    for (int o = 0; o < 16; o++) {
-        for (int j = 0; j < RP; j++) fin.m[o][16 + j] = pq[RP - 1 - j][o];
-        fin.k[o] = P2<F>::K.ext_rc[4][o];
-    }
+    mx_state_bias<F>(t.c[S::B_MERGED], parts.merged, 16);
     for (int s = 0; s < 2 + S::PAIRS; s++)
         for (int y = 0; y < 2; y++)
             mx_fill<F>(
-                t.a[S::FINAL + 2 * s + y], fin,
+                t.a[S::FINAL + 2 * s + y], parts.fin,
                 [&](int h, int i) {
                     if (s < 2) return 8 * s + 4 * h + i;
                     const int r = mx_round(s - 2, h, i);
@@ -283,7 +292,7 @@ constexpr MxTable<F> make_mx_table() {
                     out = mx_word(mx_row_h(r), j % 8);
                     plane = y + 2 * (j / 8);
                 });
-    mx_state_bias<F>(t.c[S::B_FINAL], fin, 16 + RP);
+    mx_state_bias<F>(t.c[S::B_FINAL], parts.fin, 16 + RP);
     // forms of pair m: output 4 beta + o is round 8 m + 4 beta + o (o = 2 h +
     // g), register j = 8 beta + 2 plane + g
     for (int m = 0; m < S::PAIRS; m++) {
@@ -291,8 +300,7 @@ constexpr MxTable<F> make_mx_table() {
         for (int q = 0; q < 8; q++) {
             const int r = 8 * m + q;
             if (r >= RP) continue;
-            for (int c = 0; c < 16; c++) f.m[q][c] = form[r][c];
-            for (int j = 0; j < 8 * m + 4 * (q / 4); j++) f.m[q][16 + j] = pq[r - 1 - j][0];
+            for (int c = 0; c < 40; c++) f.m[q][c] = parts.forms[r][c];
             f.k[q] = P2<F>::K.int_rc[r];
         }
         auto rows = [&](bool second_only) {
@@ -315,6 +323,102 @@ constexpr MxTable<F> make_mx_table() {
                 for (int g = 0; g < 2; g++)
                     mx_bias<F>(f, 4 * beta + 2 * h + g, 16 + 8 * m + 4 * beta, t.c[S::B_FORMS + m][h][8 * beta + g],
                                t.c[S::B_FORMS + m][h][8 * beta + 4 + g]);
+    }
+    return t;
+}
+
+// ---- 16 states per wave ------------------------------------------------------
+// For layers that do not fill the GPU a permutation costs its latency, which
+// is the instructions a wave issues (one in 4.2 cycles, dependent or not).
+// Here a wave holds 16 states, four lanes each, on v_mfma_i32_16x16x64_i8:
+// lane l holds column (state) l % 16 and, with q = l / 16, state words 4 q + i
+// as register i: the 16 words of a state are one 64-deep step.  D row 4 q + i
+// is the same word of the same lane, so a layer is one matrix instruction per
+// plane.  A block of partial rounds is one instruction per step: row 4 o +
+// plane, so lane group q holds all planes of the block's form q; the four
+// forms are spread over the lane groups by permlane swaps and every group runs
+// the four S-boxes.  x'_r is operand word r % 16 -> group r % 4, register r / 4
+// of step r / 16.  The tables stay in registers (192 for KoalaBear).
+// A tree layer of at most 64 nodes per CU: 3.2 us with one state on 16 lanes
+// (additions by DPP moves), 7 us with 64 states per wave, 2.2 us this way;
+// the 8 layers above 2^8 digests 36.5 -> 21.2 us, a leaf layer of 512 rows x
+// 16 13.7 -> 6.9 us.
+template <class F>
+struct Mx16Shape {
+    static constexpr int RP = F::ROUNDS_P;
+    static constexpr int BLOCKS = (RP + 3) / 4;
+    static constexpr int STEPS = 1 + (RP + 15) / 16;  // of the layer after the partial rounds
+    static_assert(BLOCKS <= 5, "the forms read at most one step of x'");
+    static constexpr int EXT = 0;    // [plane 4]
+    static constexpr int FORMS = 4;  // block 0: one step; the others: state, x'
+    static constexpr int forms(int b) { return FORMS + (b ? 2 * b - 1 : 0); }
+    static constexpr int FINAL = FORMS + 2 * BLOCKS - 1;  // [step][plane 4]
+    static constexpr int NA = FINAL + 4 * STEPS;
+    // biases: before full rounds 0..7 (4: after the partial rounds), after the last
+    static constexpr int NC = 9;
+};
+template <class F>
+struct alignas(64) Mx16Table {
+    uint32_t a[Mx16Shape<F>::NA][64][4];
+    int32_t c[Mx16Shape<F>::NC][2][16];             // planes 0 and 2 of word w
+    int32_t f[Mx16Shape<F>::BLOCKS][16];            // plane i of form q at 4 q + i
+};
+template <class F>
+constexpr Mx16Table<F> make_mx16_table() {
+    using S = Mx16Shape<F>;
+    constexpr int RP = F::ROUNDS_P;
+    Mx16Table<F> t{};
+    const MxParts<F> parts = make_mx_parts<F>();
+    // one step: input(q, i), row(r) -> output and plane
+    auto fill = [&](uint32_t (&a)[64][4], const MxLin& L, auto input, auto row) {
+        for (int lane = 0; lane < 64; lane++) {
+            int out = -1, plane = 0;
+            row(lane % 16, out, plane);
+            for (int i = 0; i < 4; i++) {
+                const int in = input(lane / 16, i);
+                a[lane][i] = out >= 0 && in >= 0 ? mx_operand_word<F>(L.m[out][in], plane) : 0;
+            }
+        }
+    };
+    auto state = [](int q, int i) { return 4 * q + i; };
+    auto rounds = [](int step) {
+        return [step](int q, int i) {
+            const int r = 16 * step + 4 * i + q;
+            return r < RP ? 16 + r : -1;
+        };
+    };
+    for (int p = 0; p < 4; p++) {
+        auto rows = [p](int r, int& out, int& plane) {
+            out = r;
+            plane = p;
+        };
+        fill(t.a[S::EXT + p], parts.ext, state, rows);
+        fill(t.a[S::FINAL + p], parts.fin, state, rows);
+        for (int s = 1; s < S::STEPS; s++) fill(t.a[S::FINAL + 4 * s + p], parts.fin, rounds(s - 1), rows);
+    }
+    for (int b = 0; b < S::BLOCKS; b++) {
+        MxLin f{};
+        for (int o = 0; o < 4; o++) {
+            if (4 * b + o >= RP) continue;
+            for (int c = 0; c < 40; c++) f.m[o][c] = parts.forms[4 * b + o][c];
+            f.k[o] = P2<F>::K.int_rc[4 * b + o];
+        }
+        auto rows = [](int r, int& out, int& plane) {
+            out = r / 4;
+            plane = r % 4;
+        };
+        fill(t.a[S::forms(b)], f, state, rows);
+        if (b) fill(t.a[S::forms(b) + 1], f, rounds(0), rows);
+        for (int o = 0; o < 4; o++) mx_bias<F>(f, o, 16 + 4 * b, t.f[b][4 * o], t.f[b][4 * o + 2]);
+    }
+    MxLin ext = parts.ext;
+    for (int k = 0; k < S::NC; k++) {
+        for (int w = 0; w < 16; w++) ext.k[w] = k == 8 ? 0 : P2<F>::K.ext_rc[k][w];
+        for (int w = 0; w < 16; w++)
+            if (k == 4)
+                mx_bias<F>(parts.fin, w, 16 + RP, t.c[k][0][w], t.c[k][1][w]);
+            else
+                mx_bias<F>(ext, w, 16, t.c[k][0][w], t.c[k][1][w]);
     }
     return t;
 }
@@ -618,6 +722,107 @@ __device__ __forceinline__ void mx_last(uint32_t (&st)[2][8], const mx4 (&b)[2][
             const uint32_t r = (uint32_t)x[t][o], s = r + F::P;
             st[t][o] = s < r ? s : r;
         }
+}
+
+// ---- device: 16 states per wave ---------------------------------------------
+static __device__ const Mx16Table<KoalaBear> kMx16Kb = make_mx16_table<KoalaBear>();
+static __device__ const Mx16Table<BabyBear> kMx16Bb = make_mx16_table<BabyBear>();
+
+template <class F>
+struct Mx16 {
+    using S = Mx16Shape<F>;
+    mx4 a[S::NA], c[S::NC][2], f[S::BLOCKS];
+    bool q1, q2;  // bits of the lane group q
+
+    __device__ __forceinline__ Mx16() {
+        const int lane = threadIdx.x & 63, q = lane >> 4;
+        const Mx16Table<F>* t;
+        if constexpr (F::P == KoalaBear::P)
+            t = &kMx16Kb;
+        else
+            t = &kMx16Bb;
+#pragma unroll
+        for (int k = 0; k < S::NA; k++) a[k] = *reinterpret_cast<const mx4*>(&t->a[k][lane][0]);
+#pragma unroll
+        for (int k = 0; k < S::NC; k++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) c[k][p] = *reinterpret_cast<const mx4*>(&t->c[k][p][4 * q]);
+#pragma unroll
+        for (int b = 0; b < S::BLOCKS; b++) f[b] = *reinterpret_cast<const mx4*>(&t->f[b][4 * q]);
+        q1 = q & 1;
+        q2 = q & 2;
+    }
+    static __device__ __forceinline__ mx4 mma(mx4 x, mx4 y, mx4 z) {
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(x, y, z, 0, 0, 0);
+    }
+    // operand word of a state word
+    static __device__ __forceinline__ mx4 op(mx4 w) { return w ^ (int)MX_BIAS; }
+
+    // one linear layer of NS steps: this lane's four outputs
+    template <int NS>
+    __device__ __forceinline__ mx4 layer(const mx4 (&in)[NS], int base, int k) const {
+        mx4 y[4] = {c[k][0], mx4{0}, c[k][1], mx4{0}};
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int p = 0; p < 4; p++) y[p] = mma(a[base + 4 * s + p], in[s], y[p]);
+        mx4 x;
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = mx_join<F>(y[0][i], y[1][i], y[2][i], y[3][i]);
+        return x;
+    }
+    static __device__ __forceinline__ mx4 sbox(mx4 x) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = mx_sbox_op<F>(x[i]);
+        return x;
+    }
+    // The permutation: operand words of the state in, state words (any int32) out
+    __device__ __forceinline__ mx4 permute(mx4 st) const {
+        mx4 in[S::STEPS];
+        {
+            const mx4 one[1] = {st};
+            in[0] = sbox(layer<1>(one, S::EXT, 0));
+        }
+#pragma unroll
+        for (int r = 1; r < 4; r++) {
+            const mx4 one[1] = {in[0]};
+            in[0] = sbox(layer<1>(one, S::EXT, r));
+        }
+#pragma unroll
+        for (int s = 1; s < S::STEPS; s++) in[s] = mx4{0};
+#pragma unroll
+        for (int b = 0; b < S::BLOCKS; b++) {
+            mx4 y = mma(a[S::forms(b)], in[0], f[b]);
+            if (b) y = mma(a[S::forms(b) + 1], in[1], y);
+            // group q holds form q: give every group all four
+            const unsigned u = (unsigned)mx_join<F>(y[0], y[1], y[2], y[3]);
+            const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+            const auto lo = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+            const auto hi = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+            int w[4] = {(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
+            mx_block<F>(w, S::RP - 4 * b);
+            in[1 + b / 4][b % 4] = (int)((uint32_t)(q1 ? (q2 ? w[3] : w[1]) : (q2 ? w[2] : w[0])) ^ MX_BIAS);
+        }
+        in[0] = sbox(layer<S::STEPS>(in, S::FINAL, 4));
+#pragma unroll
+        for (int r = 5; r < 8; r++) {
+            const mx4 one[1] = {in[0]};
+            in[0] = sbox(layer<1>(one, S::EXT, r));
+        }
+        const mx4 one[1] = {in[0]};
+        return layer<1>(one, S::EXT, 8);
+    }
+};
+// state words of a permutation, reduced
+template <class F>
+__device__ __forceinline__ u32x4 mx16_words(mx4 x) {
+    u32x4 w;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t r = (uint32_t)x[i], s = r + F::P;
+        w[i] = s < r ? s : r;
+    }
+    return w;
 }
 
 }  // namespace pg

@@ -1,8 +1,8 @@
-"""Poseidon2 on the matrix cores (64 states per wave, two tiles of 32) at the
-sizes where it can go wrong: heights below, at and above one wave's 64 rows,
-rows whose 8-word chunks are partial or cross matrices, layers above the
-16-lane kernels' limit with and without injected rows, and words at the ends
-of the field's range.  Every digest layer equals the oracle's, bit for bit."""
+"""Poseidon2 on the matrix cores (16 or 64 states per wave) at the sizes where
+it can go wrong: heights below, at and above one wave's rows, rows whose 8-word
+chunks are partial or cross matrices, leaf layers and compress layers on both
+sides of the limit between the two forms (2^15) with and without injected
+rows, several layers per launch, and words at the ends of the field's range.  Every digest layer equals the oracle's, bit for bit."""
 import numpy as np
 import pytest
 
@@ -37,11 +37,28 @@ def test_leaf_rows(ctx, oracle, f, widths):
 @pytest.mark.parametrize("f", FIELDS)
 @pytest.mark.parametrize("inj", [(), (8,), (5,), (3, 14)], ids=str)
 def test_tall_layers(ctx, oracle, f, inj):
-    # 2^16 leaves: the 2^15-node layer is above the 16-lane kernels' limit
-    hosts = [oracle.random_matrix(f, 1, 1 << 16, 8)]
-    hosts += [oracle.random_matrix(f, 10 + k, 1 << 15, w) for k, w in enumerate(inj)]
-    hosts += [oracle.random_matrix(f, 20 + k, 64, w) for k, w in enumerate(inj)]
+    # 2^17 leaves: layers of 2^16 and 2^15 nodes are above and at the limit
+    hosts = [oracle.random_matrix(f, 1, 1 << 17, 8)]
+    for log_h in (16, 15, 6):
+        hosts += [oracle.random_matrix(f, 10 * log_h + k, 1 << log_h, w) for k, w in enumerate(inj)]
     check_tree(ctx, oracle, f, hosts)
+
+
+@pytest.mark.parametrize("f", FIELDS)
+@pytest.mark.parametrize("widths", [(16,), (7, 6)], ids=str)
+@pytest.mark.parametrize("log_h", [15, 16])
+def test_leaf_limit(ctx, oracle, f, widths, log_h):
+    check_tree(ctx, oracle, f, [oracle.random_matrix(f, 3 + i, 1 << log_h, w) for i, w in enumerate(widths)])
+
+
+@pytest.mark.parametrize("f", FIELDS)
+def test_layers_per_launch(ctx, oracle, f):
+    # every first-layer size: partial waves, one and two passes of a
+    # workgroup, a second launch after seven layers, from 8-word rows and from
+    # digests
+    for log_h in range(0, 11):
+        for w in (8, 9):
+            check_tree(ctx, oracle, f, [oracle.random_matrix(f, log_h, 1 << log_h, w)])
 
 
 @pytest.mark.parametrize("f", FIELDS)
