@@ -1043,6 +1043,7 @@ struct pg_tree {
     size_t digest_bytes = 0;
     void* meta = nullptr;  // device: MatRef orig[n], shift[n], coloff[n], layer_off[log_h + 1]
     size_t meta_bytes = 0;
+    std::shared_ptr<DevMem> shared_meta;  // FRI trees: one block for all rounds (meta is null)
     MatRef* d_mats = nullptr;
     uint32_t* d_shift = nullptr;
     uint32_t* d_coloff = nullptr;
@@ -2897,7 +2898,8 @@ extern "C" int pg_fri_fold(pg_ctx* ctx, int field, const pg_buf* v, const uint32
     PG_TRY(get_twiddles(ctx, l.s, field, ln, &tw));
     pg_buf* o;
     PG_TRY(buf_new(ctx, v->rows / 2, 4, &o));
-    hipError_t e = launch_fri_fold(field, v->ptr, v->rows / 2, beta, (const uint32_t*)tw->ptr, o->ptr, l.s);
+    hipError_t e = launch_fri_fold(field, v->ptr, v->rows / 2, nullptr, beta, (const uint32_t*)tw->ptr, nullptr, o->ptr,
+                                   l.s);
     if (e == hipSuccess) e = hipStreamSynchronize(l.s);
     if (e != hipSuccess) {
         pg_buf_free(o);
@@ -2942,61 +2944,112 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
             return fail(PG_E_INVALID, "input %d must be 2^%d x 4", k, k);
     for (int k = 0; k <= max_log; k++) PG_TRY(need_dense(inputs[k], "pg_fri_commit_phase"));
     if (log_stop > L0) return fail(PG_E_INVALID, "log_stop > input length");
+    static_assert(sizeof(pg_challenger) == 4 * CHALLENGER_WORDS, "the device reads the challenger as words");
     PG_TRY(bind_device(ctx));
     Lease l(ctx);
     std::unique_ptr<pg_fri, void (*)(pg_fri*)> f(new pg_fri, pg_fri_free);
     f->ctx = ctx;
     f->field = field;
     f->log_max = L0;
-    pg_buf* cur;
-    PG_TRY(buf_new(ctx, (size_t)1 << L0, 4, &cur));
-    HIP_TRY(hipMemcpyAsync(cur->ptr, inputs[L0]->ptr, cur->bytes, hipMemcpyDeviceToDevice, l.s));
-    int r = 0;
-    int len_log = L0;
-    while (len_log > log_stop) {
-        // commit the current vector as (n/2) x 8 leaves; the tree owns it
-        pg_buf* leaves = new pg_buf(*cur);
-        leaves->rows = cur->rows / 2;
-        leaves->cols = 8;
-        cur->owned = false;  // ownership moves to `leaves`
-        pg_buf_free(cur);
-        pg_tree* t;
-        int rc = mmcs_commit_on_stream(ctx, l.s, field, {leaves}, {true}, roots_out + 8 * r, &t);
-        if (rc != PG_OK) {
-            (void)hipStreamSynchronize(l.s);  // the first round's copy may still be writing it
-            pg_buf_free(leaves);
-            return rc;
+    // Everything is allocated before the first launch and the challenger runs
+    // on the device: a round's last tree launch observes the root and samples
+    // beta, which the fold reads from device memory, so the rounds queue up
+    // without the host in between.
+    const int R = L0 - log_stop;
+    const size_t nf = (size_t)1 << log_stop;
+    const size_t o_roots = align_up(4 * CHALLENGER_WORDS, 256), o_betas = o_roots + align_up(32 * (size_t)R, 256),
+                 o_fin = o_betas + align_up(16 * (size_t)R, 256), res_bytes = o_fin + 16 * nf;
+    int rc;
+    auto res = make_devmem(ctx, res_bytes, &rc);
+    if (!res) return rc;
+    uint8_t* const dres = (uint8_t*)res->ptr;
+    std::vector<std::shared_ptr<DevMem>> tws(R);
+    std::vector<uint8_t> hm;
+    std::vector<size_t> off_mats(R), off_zero(R), off_layer(R);
+    for (int r = 0; r < R; r++) {
+        PG_TRY(get_twiddles(ctx, l.s, field, L0 - r, &tws[r]));
+        TreePtr t(new pg_tree, pg_tree_free);
+        t->ctx = ctx;
+        t->field = field;
+        t->H = (size_t)1 << (L0 - r - 1);
+        t->log_h = L0 - r - 1;
+        t->total_width = 8;
+        pg_buf* leaves;
+        PG_TRY(buf_new(ctx, t->H, 8, &leaves));  // the round's vector, two ext4 elements a row
+        t->mats = {leaves};
+        t->owned = {true};
+        t->digest_bytes = (2 * t->H - 1) * 32;
+        void* p;
+        PG_TRY(ctx_alloc(ctx, t->digest_bytes, &p));
+        t->digests = (uint32_t*)p;
+        // descriptors for openings: the matrix, its shift and column (zeros), layer offsets
+        off_mats[r] = hm.size();
+        off_zero[r] = align_up(off_mats[r] + sizeof(MatRef), 256);
+        off_layer[r] = off_zero[r] + 256;
+        hm.resize(align_up(off_layer[r] + 8 * (size_t)(t->log_h + 1), 256), 0);
+        const MatRef m{leaves->ptr, 8, 8, 0};
+        memcpy(hm.data() + off_mats[r], &m, sizeof m);
+        uint64_t off = 0;
+        for (int j = 0; j <= t->log_h; j++) {
+            memcpy(hm.data() + off_layer[r] + 8 * j, &off, 8);
+            off += t->H >> j;
         }
-        f->trees.push_back(t);
-        for (int k = 0; k < 8; k++) pg_challenger_observe(ch, roots_out[8 * r + k]);
-        uint32_t beta[4];
-        pg_challenger_sample_ext(ch, beta);
-        if (betas_out) memcpy(betas_out + 4 * r, beta, 16);
-        std::shared_ptr<DevMem> tw;
-        PG_TRY(get_twiddles(ctx, l.s, field, len_log, &tw));
-        PG_TRY(buf_new(ctx, (size_t)1 << (len_log - 1), 4, &cur));
-        auto kt = make_timer(ctx);
-        if (kt) kt->begin("fri_fold", l.s);
-        hipError_t e = launch_fri_fold(field, leaves->ptr, cur->rows, beta, (const uint32_t*)tw->ptr, cur->ptr, l.s);
-        if (kt) kt->end(l.s);
-        len_log--;
-        if (e == hipSuccess && inputs[len_log])
-            e = launch_field_add(field, cur->ptr, inputs[len_log]->ptr, cur->rows * 4, l.s);
-        const hipError_t es = hipStreamSynchronize(l.s);
-        if (e == hipSuccess) e = es;
-        if (e != hipSuccess) {
-            pg_buf_free(cur);
-            return fail(PG_E_DEVICE, "FRI fold round %d failed: %s", r, hipGetErrorString(e));
-        }
-        r++;
+        f->trees.push_back(t.release());
     }
-    const size_t nf = (size_t)1 << len_log;
-    std::vector<uint32_t> fin(nf * 4);
-    hipError_t e = hipMemcpyAsync(fin.data(), cur->ptr, nf * 16, hipMemcpyDeviceToHost, l.s);
-    if (e == hipSuccess) e = hipStreamSynchronize(l.s);
-    pg_buf_free(cur);
-    HIP_TRY(e);
-    if (final_out) memcpy(final_out, fin.data(), nf * 16);
+    std::shared_ptr<DevMem> meta;
+    if (R) {
+        meta = make_devmem(ctx, hm.size(), &rc);
+        if (!meta) return rc;
+    }
+    for (int r = 0; r < R; r++) {
+        uint8_t* const dm = (uint8_t*)meta->ptr;
+        pg_tree* const t = f->trees[r];
+        t->shared_meta = meta;
+        t->d_mats = (MatRef*)(dm + off_mats[r]);
+        t->d_shift = t->d_coloff = (uint32_t*)(dm + off_zero[r]);
+        t->d_layer_off = (uint64_t*)(dm + off_layer[r]);
+    }
+    SyncGuard guard(l.s);  // on an error below: wait for queued work before anything is freed
+    if (R) HIP_TRY(hipMemcpyAsync(meta->ptr, hm.data(), hm.size(), hipMemcpyHostToDevice, l.s));
+    HIP_TRY(hipMemcpyAsync(dres, ch, sizeof *ch, hipMemcpyHostToDevice, l.s));
+    HIP_TRY(hipMemcpyAsync(R ? (void*)f->trees[0]->mats[0]->ptr : (void*)(dres + o_fin), inputs[L0]->ptr,
+                           (size_t)16 << L0, hipMemcpyDeviceToDevice, l.s));
+    auto kt = make_timer(ctx);
+    for (int r = 0; r < R; r++) {
+        const pg_tree* const t = f->trees[r];
+        const uint32_t* const v = t->mats[0]->ptr;
+        uint32_t* const beta = (uint32_t*)(dres + o_betas) + 4 * r;
+        const TreeChallenge tc{(uint32_t*)dres, (uint32_t*)(dres + o_roots) + 8 * r, beta};
+        size_t len = t->H, off = 0;
+        if (len > SMALL_MAX_NODES) {
+            TIMED(kt, "leaf_hash_w8", l.s, launch_leaf_hash_w8(field, v, 8, 8, len, t->digests, l.s));
+            for (; len / 2 > SMALL_MAX_NODES; off += len, len /= 2)
+                TIMED(kt, "compress", l.s,
+                      launch_compress(field, t->digests + 8 * off, t->digests + 8 * (off + len), len / 2, nullptr, 0, 0,
+                                      l.s));
+            TIMED(kt, "compress", l.s,
+                  launch_tree_layers(field, t->digests + 8 * off, 0, 0, len / 2, log2_of(len), t->digests + 8 * (off + len),
+                                     l.s, &tc));
+        } else {
+            TIMED(kt, "leaf_hash_w8", l.s,
+                  launch_tree_layers(field, v, 8, 1, len, t->log_h + 1, t->digests, l.s, &tc));
+        }
+        const pg_buf* const add = inputs[t->log_h];  // the vectors have 2^(log_h + 1) and 2^log_h elements
+        uint32_t* const next = r + 1 < R ? f->trees[r + 1]->mats[0]->ptr : (uint32_t*)(dres + o_fin);
+        TIMED(kt, "fri_fold", l.s,
+              launch_fri_fold(field, v, t->H, beta, nullptr, (const uint32_t*)tws[r]->ptr, add ? add->ptr : nullptr,
+                              next, l.s));
+    }
+    std::vector<uint8_t> host(res_bytes);
+    HIP_TRY(hipMemcpyAsync(host.data(), dres, res_bytes, hipMemcpyDeviceToHost, l.s));
+    HIP_TRY(hipStreamSynchronize(l.s));
+    guard.armed = false;
+    memcpy(ch, host.data(), sizeof *ch);
+    if (R) memcpy(roots_out, host.data() + o_roots, 32 * (size_t)R);
+    if (R && betas_out) memcpy(betas_out, host.data() + o_betas, 16 * (size_t)R);
+    for (int r = 0; r < R; r++) memcpy(f->trees[r]->root, host.data() + o_roots + 32 * r, 32);
+    const uint32_t* const fin = (const uint32_t*)(host.data() + o_fin);
+    if (final_out) memcpy(final_out, fin, nf * 16);
     if (final_mode == 0) {
         for (size_t i = 1; i < nf; i++)
             if (memcmp(&fin[4 * i], &fin[0], 16))
@@ -3005,7 +3058,7 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
     } else {
         for (size_t i = 0; i < nf * 4; i++) pg_challenger_observe(ch, fin[i]);
     }
-    if (rounds_out) *rounds_out = r;
+    if (rounds_out) *rounds_out = R;
     *out = f.release();
     return PG_OK;
 }
@@ -3050,26 +3103,32 @@ extern "C" int pg_fri_answer_queries(pg_ctx* ctx, const pg_fri* f, const uint64_
     PG_TRY(bind_device(ctx));
     Lease l(ctx);
     const int R = (int)f->trees.size();
-    size_t path_words_per_q = 0;
-    for (int r = 0; r < R; r++) path_words_per_q += 8 * (size_t)f->trees[r]->log_h;
-    std::vector<uint64_t> leaf(nq);
-    std::vector<uint32_t> rows, paths;
-    size_t path_off = 0;
+    if (nq == 0 || R == 0) return PG_OK;
+    std::vector<FriOpenRound> rd(R);
+    size_t pw = 0;  // path words per query
     for (int r = 0; r < R; r++) {
         const pg_tree* t = f->trees[r];
-        for (size_t q = 0; q < nq; q++) leaf[q] = (idx[q] >> r) >> 1;
-        rows.assign(nq * 8, 0);
-        paths.assign(nq * t->log_h * 8, 0);
-        PG_TRY(open_on_stream(ctx, l.s, t, leaf.data(), nq, rows.data(), paths.data()));
-        for (size_t q = 0; q < nq; q++) {
-            const bool odd = (idx[q] >> r) & 1;
-            if (siblings_out) memcpy(siblings_out + (q * R + r) * 4, rows.data() + q * 8 + (odd ? 0 : 4), 16);
-            if (paths_out)
-                memcpy(paths_out + q * path_words_per_q + path_off, paths.data() + q * t->log_h * 8,
-                       t->log_h * 32);
-        }
-        path_off += 8 * (size_t)t->log_h;
+        rd[r] = FriOpenRound{t->mats[0]->ptr, t->digests, (uint32_t)t->log_h, (uint32_t)pw};
+        pw += 8 * (size_t)t->log_h;
     }
+    // indices and rounds up, every round's answers down, one launch
+    const size_t o_idx = align_up(R * sizeof(FriOpenRound), 256), o_sib = align_up(o_idx + nq * 8, 256),
+                 sib_bytes = nq * R * 16, o_paths = o_sib + align_up(sib_bytes, 256), bytes = o_paths + nq * pw * 4;
+    int rc;
+    auto d = make_devmem(ctx, bytes, &rc);
+    if (!d) return rc;
+    uint8_t* const dm = (uint8_t*)d->ptr;
+    std::vector<uint8_t> h(o_idx + nq * 8);
+    memcpy(h.data(), rd.data(), R * sizeof(FriOpenRound));
+    memcpy(h.data() + o_idx, idx, nq * 8);
+    SyncGuard guard(l.s);
+    HIP_TRY(hipMemcpyAsync(dm, h.data(), h.size(), hipMemcpyHostToDevice, l.s));
+    HIP_TRY(launch_fri_open((const FriOpenRound*)dm, R, (const uint64_t*)(dm + o_idx), (int)nq, (uint32_t)pw,
+                            (uint32_t*)(dm + o_sib), (uint32_t*)(dm + o_paths), l.s));
+    if (siblings_out) HIP_TRY(hipMemcpyAsync(siblings_out, dm + o_sib, sib_bytes, hipMemcpyDeviceToHost, l.s));
+    if (paths_out && pw) HIP_TRY(hipMemcpyAsync(paths_out, dm + o_paths, nq * pw * 4, hipMemcpyDeviceToHost, l.s));
+    HIP_TRY(hipStreamSynchronize(l.s));
+    guard.armed = false;
     return PG_OK;
 }
 

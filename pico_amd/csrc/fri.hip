@@ -1,4 +1,4 @@
-// fri.hip -- FRI arity-2 fold, vector add, proof-of-work search, and the
+// fri.hip -- FRI arity-2 fold, proof-of-work search, and the
 // element-wise helpers (representation conversion, seeded synthetic inputs).
 //
 // Fold semantics (p3 fold_even_odd; pinned in-tree by the query check at
@@ -14,10 +14,14 @@
 
 namespace pg {
 
+// beta is read from device memory when `beta` is given (in the commit phase the
+// tree's last launch has just sampled it, and no host round trip stands between
+// two rounds), else it is `host_beta`.
 template <class F>
 __global__ void __launch_bounds__(256) fri_fold_kernel(const uint32_t* __restrict__ v, uint64_t n_out,
-                                                       Ext4 half_beta, const uint32_t* __restrict__ tw,
-                                                       int log_n_out, uint32_t* __restrict__ out) {
+                                                       const uint32_t* __restrict__ beta, Ext4 host_beta,
+                                                       const uint32_t* __restrict__ tw, int log_n_out, const uint32_t* __restrict__ add,
+                                                       uint32_t* __restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_out) return;
     const uint4 a4 = reinterpret_cast<const uint4*>(v)[2 * i];
@@ -30,14 +34,15 @@ __global__ void __launch_bounds__(256) fri_fold_kernel(const uint32_t* __restric
 #pragma unroll
     for (int k = 0; k < 4; k++) s.c[k] = fhalve<F>(s.c[k]);
     const Ext4 d = escale<F>(esub<F>(a, b), x_inv);
-    const Ext4 o = eadd<F>(s, emul<F>(d, half_beta));
+    Ext4 half_beta;
+#pragma unroll
+    for (int k = 0; k < 4; k++) half_beta.c[k] = fhalve<F>(beta ? beta[k] : host_beta.c[k]);
+    Ext4 o = eadd<F>(s, emul<F>(d, half_beta));
+    if (add) {
+        const uint4 w = reinterpret_cast<const uint4*>(add)[i];
+        o = eadd<F>(o, Ext4{{w.x, w.y, w.z, w.w}});
+    }
     reinterpret_cast<uint4*>(out)[i] = make_uint4(o.c[0], o.c[1], o.c[2], o.c[3]);
-}
-
-template <class F>
-__global__ void field_add_kernel(uint32_t* out, const uint32_t* add, uint64_t n) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = fadd<F>(out[i], add[i]);
 }
 
 template <class F>
@@ -97,19 +102,17 @@ __global__ void fill_random_kernel(uint64_t seed, uint32_t* out, uint64_t n, int
 
 static unsigned blocks(uint64_t n) { return (unsigned)((n + 255) / 256); }
 
-hipError_t launch_fri_fold(int field, const uint32_t* v, size_t n_out, const uint32_t beta[4],
-                           const uint32_t* tw, uint32_t* out, hipStream_t stream) {
+hipError_t launch_fri_fold(int field, const uint32_t* v, size_t n_out, const uint32_t* beta, const uint32_t* host_beta,
+                           const uint32_t* tw, const uint32_t* add, uint32_t* out, hipStream_t stream) {
     if (n_out == 0) return hipSuccess;
+    Ext4 hb{{0, 0, 0, 0}};
+    for (int k = 0; k < 4 && host_beta; k++) hb.c[k] = host_beta[k];
     int log_n_out = 0;
     while ((1ull << log_n_out) < n_out) log_n_out++;
-    Ext4 hb;
-    if (field == FIELD_KOALABEAR) {
-        for (int k = 0; k < 4; k++) hb.c[k] = fhalve<KoalaBear>(beta[k]);
-        fri_fold_kernel<KoalaBear><<<blocks(n_out), 256, 0, stream>>>(v, n_out, hb, tw, log_n_out, out);
-    } else {
-        for (int k = 0; k < 4; k++) hb.c[k] = fhalve<BabyBear>(beta[k]);
-        fri_fold_kernel<BabyBear><<<blocks(n_out), 256, 0, stream>>>(v, n_out, hb, tw, log_n_out, out);
-    }
+    if (field == FIELD_KOALABEAR)
+        fri_fold_kernel<KoalaBear><<<blocks(n_out), 256, 0, stream>>>(v, n_out, beta, hb, tw, log_n_out, add, out);
+    else
+        fri_fold_kernel<BabyBear><<<blocks(n_out), 256, 0, stream>>>(v, n_out, beta, hb, tw, log_n_out, add, out);
     return hipGetLastError();
 }
 
@@ -130,15 +133,6 @@ hipError_t launch_rows_bitrev(const uint32_t* src, uint64_t ld, uint32_t w, int 
                               uint32_t* dst, hipStream_t stream) {
     if (nrows == 0 || w == 0) return hipSuccess;
     rows_bitrev_kernel<<<blocks(nrows * w), 256, 0, stream>>>(src, ld, w, q, r0, nrows, dst);
-    return hipGetLastError();
-}
-
-hipError_t launch_field_add(int field, uint32_t* out, const uint32_t* add, size_t n, hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    if (field == FIELD_KOALABEAR)
-        field_add_kernel<KoalaBear><<<blocks(n), 256, 0, stream>>>(out, add, n);
-    else
-        field_add_kernel<BabyBear><<<blocks(n), 256, 0, stream>>>(out, add, n);
     return hipGetLastError();
 }
 

@@ -60,8 +60,26 @@ hipError_t launch_compress_digest(int field, const uint32_t* prev, uint32_t* nex
 // hashes of n0 rows of 8 words (row pitch `stride`); the layers n0, n0/2, ...
 // are written one after the other at out.
 constexpr uint64_t SMALL_MAX_NODES = 1u << 15;
+// With `ch` the layers end at the root, which the duplex challenger at ch.state
+// then observes; four samples follow (an ext4 challenge).
+struct TreeChallenge {
+    uint32_t* state;  // pg_challenger: field, state[16], input[8], n_input, output[8], n_output
+    uint32_t* root;   // 8 words out
+    uint32_t* beta;   // 4 words out
+};
+constexpr int CHALLENGER_WORDS = 35;
 hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
-                              uint32_t* out, hipStream_t stream);
+                              uint32_t* out, hipStream_t stream, const TreeChallenge* ch = nullptr);
+// FRI query answers: for query q and round r, the sibling v_r[(idx[q] >> r) ^ 1]
+// (4 words at siblings[(q rounds + r) 4]) and the Merkle path of leaf
+// (idx[q] >> r) >> 1 (at paths[q path_words + path_off]).
+struct FriOpenRound {
+    const uint32_t* vec;
+    const uint32_t* digests;
+    uint32_t log_h, path_off;
+};
+hipError_t launch_fri_open(const FriOpenRound* rounds, int nrounds, const uint64_t* idx, int nq, uint32_t path_words,
+                           uint32_t* siblings, uint32_t* paths, hipStream_t stream);
 // Opening gather: for each query q < nq and matrix k, copy row
 // (idx[q] >> shift[k]) of mats[k] to rows_out[q * total_width + col_off[k] ..];
 // for each layer j < log_h, copy digest layer_j[(idx[q] >> j) ^ 1] to
@@ -178,11 +196,10 @@ hipError_t launch_reduce_rows(int field, const RoMat* mats, int nmats, const Ext
 // out[i] = (1/2 + beta/(2 x_i)) v[2i] + (1/2 - beta/(2 x_i)) v[2i+1],
 // x_i = w_n^{rev(i)}; v and out are ext4 arrays; tw is the twiddle table of
 // size n = 2 * n_out.
-hipError_t launch_fri_fold(int field, const uint32_t* v, size_t n_out, const uint32_t beta[4],
-                           const uint32_t* tw, uint32_t* out, hipStream_t stream);
-// out[i] += add[i] for i < n words (field addition)
-hipError_t launch_field_add(int field, uint32_t* out, const uint32_t* add, size_t n,
-                            hipStream_t stream);
+// beta: 4 words in device memory, or null and host_beta's 4 words on the host;
+// add (may be null): n_out ext4 elements added.
+hipError_t launch_fri_fold(int field, const uint32_t* v, size_t n_out, const uint32_t* beta,
+                           const uint32_t* host_beta, const uint32_t* tw, const uint32_t* add, uint32_t* out, hipStream_t stream);
 // Proof-of-work search: smallest witness w in [start, start + count) such
 // that the challenger state after observe(w) samples a value whose low
 // `bits` bits are zero.  state: 16 words; in: n_in pending inputs.

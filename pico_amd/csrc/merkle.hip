@@ -502,8 +502,52 @@ MX16_KERNEL compress_small_kernel(const uint32_t* prev, uint32_t* next, uint64_t
 // so a layer costs one permutation's latency instead of a launch (4.3 us and
 // the gap before it).
 constexpr int TREE_MAX_PER = 128;  // first-layer nodes of a workgroup
+
+// The duplex challenger (vm/src/compiler/recursion/circuit/challenger.rs:
+// 89-175) observes 8 words and samples an ext4 element: the wave's 16 columns
+// all hold the one state.  `root` and `pend` (16 words) are in LDS.  With k < 8
+// inputs pending, the 8 words fill one duplexing and leave k for the one that
+// sampling makes; the samples are output words 7, 6, 5, 4.
+template <class F>
+__device__ __forceinline__ void challenge_root(const Mx16<F>& P, const Mx16Lane& l, const TreeChallenge& ch,
+                                               const uint32_t* root, uint32_t* pend) {
+    const gptr st = (gptr)ch.state + 1, input = (gptr)ch.state + 17, n_input = (gptr)ch.state + 25,
+               output = (gptr)ch.state + 26, n_output = (gptr)ch.state + 34;
+    const uint32_t t = threadIdx.x, k = (uint32_t)__builtin_amdgcn_readfirstlane((int)*n_input);
+    if (t < 8) {
+        ((gptr)ch.root)[t] = root[t];
+        if (t < k) pend[t] = input[t];
+        pend[k + t] = root[t];
+    }
+    __threadfence_block();
+    u32x4 w;
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = l.q < 2 ? pend[4 * l.q + i] : st[4 * l.q + i];
+    w = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
+    if (k) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (4 * l.q + i < k) w[i] = pend[8 + 4 * l.q + i];
+        w = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
+    }
+    if (l.n == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            st[4 * l.q + i] = w[i];
+            if (l.q < 2) output[4 * l.q + i] = w[i];
+            if (l.q == 1) ((gptr)ch.beta)[3 - i] = w[i];
+        }
+    }
+    if (t < 8) input[t] = pend[t < k ? 8 + t : t];
+    if (t == 0) {
+        *n_input = 0;
+        *n_output = 4;
+    }
+}
+
 template <class F, bool LEAF8>
-MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0, int log_per, int layers, uint32_t* out) {
+MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0, int log_per, int layers, uint32_t* out,
+                               TreeChallenge ch) {
     __shared__ u32x4 buf[2][2 * TREE_MAX_PER];
     const Mx16<F> P;
     const Mx16Lane l;
@@ -530,6 +574,10 @@ MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0,
         __syncthreads();
         layer += 8 * (n0 >> i);
     }
+    if (ch.state && wave == 0) {  // one workgroup: the last layer is the root
+        __shared__ uint32_t pend[16];
+        challenge_root<F>(P, l, ch, reinterpret_cast<const uint32_t*>(buf[(layers - 1) & 1]), pend);
+    }
 }
 
 __global__ void open_gather_kernel(const MatRef* mats, const uint32_t* shift,
@@ -549,6 +597,26 @@ __global__ void open_gather_kernel(const MatRef* mats, const uint32_t* shift,
         const uint64_t sib = (index >> j) ^ 1u;
         paths_out[((uint64_t)q * log_h + j) * 8 + e] = digests[(layer_off[j] + sib) * 8 + e];
     }
+}
+
+__global__ void fri_open_kernel(const FriOpenRound* rounds, const uint64_t* idx, uint32_t path_words, uint32_t* siblings,
+                                uint32_t* paths) {
+    const uint32_t q = blockIdx.x, r = blockIdx.y;
+    const FriOpenRound rd = rounds[r];
+    const uint64_t i = idx[q] >> r, leaf = i >> 1, H = 1ull << rd.log_h;
+    if (threadIdx.x < 4) siblings[((uint64_t)q * gridDim.y + r) * 4 + threadIdx.x] = rd.vec[4 * (i ^ 1u) + threadIdx.x];
+    for (uint32_t t = threadIdx.x; t < rd.log_h * 8; t += blockDim.x) {
+        const uint32_t j = t >> 3;
+        const uint64_t off = 2 * (H - (H >> j));  // layer j's first digest
+        paths[(uint64_t)q * path_words + rd.path_off + t] = rd.digests[(off + ((leaf >> j) ^ 1u)) * 8 + (t & 7)];
+    }
+}
+
+hipError_t launch_fri_open(const FriOpenRound* rounds, int nrounds, const uint64_t* idx, int nq, uint32_t path_words,
+                           uint32_t* siblings, uint32_t* paths, hipStream_t stream) {
+    if (nq == 0 || nrounds == 0) return hipSuccess;
+    fri_open_kernel<<<dim3((unsigned)nq, (unsigned)nrounds), 128, 0, stream>>>(rounds, idx, path_words, siblings, paths);
+    return hipGetLastError();
 }
 
 // ---- batched single-matrix commits --------------------------------------
@@ -753,17 +821,18 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
 // layer has at most 128 nodes.
 template <class F>
 static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, bool leaf8, uint64_t n0, int layers, uint32_t* out,
-                                hipStream_t s) {
+                                hipStream_t s, const TreeChallenge* ch) {
     while (layers > 0) {
         int log_per = 6;
         if (n0 <= (uint64_t)TREE_MAX_PER)
             log_per = __builtin_ctzll(n0);
         const int now = std::min(layers, log_per + 1);
+        const TreeChallenge c = ch && now == layers ? *ch : TreeChallenge{};
         const unsigned threads = std::min((unsigned)S_THREADS, std::max(64u, 4u << log_per));
         if (leaf8)
-            tree_layers_kernel<F, true><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, stride, n0, log_per, now, out);
+            tree_layers_kernel<F, true><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, stride, n0, log_per, now, out, c);
         else
-            tree_layers_kernel<F, false><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, 0, n0, log_per, now, out);
+            tree_layers_kernel<F, false><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, 0, n0, log_per, now, out, c);
         for (int i = 0; i < now; i++) {  // the last layer written feeds the next launch
             in = out;
             out += 8 * n0;
@@ -776,11 +845,12 @@ static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, bool leaf8,
 }
 
 hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
-                              uint32_t* out, hipStream_t stream) {
+                              uint32_t* out, hipStream_t stream, const TreeChallenge* ch) {
     if (layers <= 0) return hipSuccess;
+    if (ch && (n0 >> (layers - 1)) != 1) return hipErrorInvalidValue;  // sampled from the root
     if (n0 == 0 || n0 > SMALL_MAX_NODES || (n0 & (n0 - 1)) || (n0 >> (layers - 1)) == 0) return hipErrorInvalidValue;
-    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf8 != 0, n0, layers, out, stream)
-                                    : tree_layers_t<BabyBear>(in, stride, leaf8 != 0, n0, layers, out, stream);
+    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf8 != 0, n0, layers, out, stream, ch)
+                                    : tree_layers_t<BabyBear>(in, stride, leaf8 != 0, n0, layers, out, stream, ch);
 }
 
 hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
