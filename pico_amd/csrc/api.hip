@@ -28,6 +28,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <set>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -3675,8 +3676,25 @@ extern "C" int pg_tune_import(const char* text) {
 }
 
 // ----------------------------------------------------- quotient values --
+// The resident form's plan (quotient.hip): column runs and their LDS slots,
+// constants, selectors, and the constraints cut into slices, one per wave.
+struct QResident {
+    struct Run {
+        uint32_t src, next, col0, count, slot0;  // src 0 main, 1 preprocessed, 2 permutation
+    };
+    std::vector<Run> runs;
+    std::vector<QrPiece> pieces;  // the runs cut into at most 64 columns
+    std::vector<std::pair<uint32_t, uint32_t>> consts;  // (leaf kind, value or index)
+    std::vector<QrSlice> slices;  // 4, 8 or 16, some perhaps empty
+    std::vector<uint32_t> code;
+    std::vector<uint32_t> folds;  // per instruction: the base assert it folds, or ~0
+    uint32_t const0 = 0, sel_word[3] = {0, 0, 0}, lds_words = 0;
+    uint32_t longest = 0;  // instructions of the longest slice
+};
+
 struct pg_air_program {
     int field = 0;
+    std::unique_ptr<QResident> resident;  // null: the program does not fit LDS or shares too much
     std::vector<QInstr> code;
     // Montgomery; at launch the public values, challenge words, regional sum
     // and global-sum coordinates follow them
@@ -3842,6 +3860,285 @@ extern "C" int pg_air_compile(int field, const pg_air_node* nodes, size_t nnodes
             if (lo[k][e] != NONE) las.push_back(LAssert{(uint32_t)lo[k][e], e, (uint32_t)j});
     }
     return air_compile_lowered(field, ln, las, (uint32_t)nasserts, out, nregs_out, ninstr_out);
+}
+
+static bool air_is_leaf(const pg_air_node& n) {
+    return n.kind != PG_AIR_ADD && n.kind != PG_AIR_SUB && n.kind != PG_AIR_NEG && n.kind != PG_AIR_MUL;
+}
+
+// The resident plan, or null.  The asserts are cut, in order, into at most W
+// slices (whole original asserts: an ext4 assert's coordinates share most of
+// their nodes); a node read by two slices is computed in both, so fewer
+// slices are taken where that would cost more than a quarter of the work.
+static std::unique_ptr<QResident> air_resident(const std::vector<pg_air_node>& nodes,
+                                               const std::vector<LAssert>& las) {
+    if (las.empty()) return nullptr;
+    // emission order of asserts [j0, j1): inner nodes operands first, then the assert
+    struct Item {
+        bool is_assert;
+        uint32_t node;
+    };
+    std::vector<uint32_t> stamp(nodes.size(), 0);
+    uint32_t now = 0;
+    std::vector<uint32_t> stack;
+    auto emit = [&](size_t j, std::vector<Item>* order) {  // the nodes assert j adds under the current stamp
+        uint32_t added = 0;
+        if (!air_is_leaf(nodes[las[j].node])) stack.push_back(las[j].node);
+        while (!stack.empty()) {
+            const uint32_t k = stack.back();
+            if (stamp[k] == now) {
+                stack.pop_back();
+                continue;
+            }
+            const pg_air_node& nd = nodes[k];
+            const bool binary = nd.kind != PG_AIR_NEG;
+            const bool wa = !air_is_leaf(nodes[nd.a]) && stamp[nd.a] != now;
+            const bool wb = binary && !air_is_leaf(nodes[nd.b]) && stamp[nd.b] != now;
+            if (wa || wb) {
+                if (wb) stack.push_back(nd.b);
+                if (wa) stack.push_back(nd.a);
+                continue;
+            }
+            stamp[k] = now;
+            stack.pop_back();
+            added++;
+            if (order) order->push_back(Item{false, k});
+        }
+        if (order) order->push_back(Item{true, las[j].node});
+        return added + 1;
+    };
+    // greedy cut at `target` instructions; returns the slices' first asserts
+    uint64_t total = 0;
+    auto cut = [&](uint64_t target, size_t most) {  // gives up past `most` slices
+        std::vector<size_t> first;
+        uint64_t cur = 0;
+        total = 0;
+        for (size_t j = 0; j < las.size() && first.size() <= most;) {
+            size_t j1 = j + 1;
+            while (j1 < las.size() && las[j1].orig == las[j].orig) j1++;
+            if (first.empty()) {
+                first.push_back(0);
+                now++;
+            }
+            uint64_t c = 0;
+            for (size_t i = j; i < j1; i++) c += emit(i, nullptr);
+            if (cur && cur + c > target) {  // starts a slice of its own
+                first.push_back(j);
+                now++;
+                cur = c = 0;
+                for (size_t i = j; i < j1; i++) c += emit(i, nullptr);
+                total += c;
+                cur = c;
+            } else {
+                cur += c;
+                total += c;
+            }
+            j = j1;
+        }
+        return first;
+    };
+    cut(UINT64_MAX, 1);
+    const uint64_t alone = total;
+    for (uint32_t W = QR_MAX_WAVES; W >= 4; W /= 2) {
+        if (W > 4 && alone < (uint64_t)W * QR_MIN_SLICE) continue;
+        uint64_t lo = 1, hi = alone;  // the smallest target that gives at most W slices
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) / 2;
+            if (cut(mid, W).size() <= W)
+                hi = mid;
+            else
+                lo = mid + 1;
+        }
+        std::vector<size_t> first = cut(lo, W);
+        if (first.size() > W || total * 4 > alone * 5) continue;
+        first.push_back(las.size());
+        const size_t S = first.size() - 1;
+        auto plan = std::make_unique<QResident>();
+        // columns read, as runs
+        std::array<std::set<uint32_t>, 6> cols;
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> consts;
+        uint32_t sel = 0;
+        auto leaf = [&](uint32_t k) {
+            const pg_air_node& nd = nodes[k];
+            switch (nd.kind) {
+                case PG_AIR_MAIN: cols[nd.a].insert(nd.b); break;
+                case PG_AIR_PREPROCESSED: cols[2 + nd.a].insert(nd.b); break;
+                case LK_PERM: cols[4 + nd.a].insert(nd.b); break;
+                case PG_AIR_IS_FIRST_ROW: sel |= 1; break;
+                case PG_AIR_IS_LAST_ROW: sel |= 2; break;
+                case PG_AIR_IS_TRANSITION: sel |= 4; break;
+                default: consts.emplace(std::make_pair(nd.kind, nd.kind == PG_AIR_CONSTANT ? nd.a : nd.b), 0); break;
+            }
+        };
+        consts.emplace(std::make_pair((uint32_t)PG_AIR_CONSTANT, 0u), 0);  // zero: negations, asserted leaves
+        std::vector<std::vector<Item>> order(S);
+        for (size_t k = 0; k < S; k++) {
+            now++;
+            for (size_t j = first[k]; j < first[k + 1]; j++) emit(j, &order[k]);
+            for (const Item& it : order[k]) {
+                const pg_air_node& nd = nodes[it.node];
+                if (air_is_leaf(nd)) {
+                    leaf(it.node);
+                } else if (!it.is_assert) {
+                    if (air_is_leaf(nodes[nd.a])) leaf(nd.a);
+                    if (nd.kind != PG_AIR_NEG && air_is_leaf(nodes[nd.b])) leaf(nd.b);
+                }
+            }
+        }
+        for (uint32_t gap = 8;; gap *= 4) {
+            plan->runs.clear();
+            uint32_t slot = 0;
+            for (uint32_t g = 0; g < 6; g++) {
+                uint32_t last = 0;
+                bool open = false;
+                for (uint32_t c : cols[g]) {
+                    if (!open || c - last > gap) {
+                        plan->runs.push_back(QResident::Run{g / 2, g % 2, c, 0, slot});
+                        open = true;
+                    }
+                    QResident::Run& r = plan->runs.back();
+                    slot += c + 1 - r.col0 - r.count;
+                    r.count = c + 1 - r.col0;
+                    last = c;
+                }
+            }
+            plan->const0 = slot * QRS_COL;
+            plan->pieces.clear();
+            for (const auto& r : plan->runs)
+                for (uint32_t c = 0; c < r.count; c += 64)
+                    plan->pieces.push_back(
+                        QrPiece{r.col0 + c, r.slot0 + c, std::min(64u, r.count - c) | r.src << 8 | r.next << 10, 0});
+            if (plan->pieces.size() <= (size_t)QR_MAX_PIECES) break;
+            if (gap > (1u << 24)) return nullptr;
+        }
+        if (plan->const0 > QR_MAX_WORDS) return nullptr;
+        uint32_t next = plan->const0;
+        for (auto& c : consts) {
+            c.second = next;
+            next += 64;
+            plan->consts.push_back(c.first);
+        }
+        for (int k = 0; k < 3; k++)
+            if (sel >> k & 1) {
+                plan->sel_word[k] = next;
+                next += 64;
+            }
+        const uint32_t zero = consts[std::make_pair((uint32_t)PG_AIR_CONSTANT, 0u)];
+        auto leaf_word = [&](uint32_t k) -> uint32_t {
+            const pg_air_node& nd = nodes[k];
+            uint32_t src;
+            switch (nd.kind) {
+                case PG_AIR_MAIN: src = 0; break;
+                case PG_AIR_PREPROCESSED: src = 1; break;
+                case LK_PERM: src = 2; break;
+                case PG_AIR_IS_FIRST_ROW: return plan->sel_word[0];
+                case PG_AIR_IS_LAST_ROW: return plan->sel_word[1];
+                case PG_AIR_IS_TRANSITION: return plan->sel_word[2];
+                default: return consts[std::make_pair(nd.kind, nd.kind == PG_AIR_CONSTANT ? nd.a : nd.b)];
+            }
+            for (const auto& r : plan->runs)
+                if (r.src == src && r.next == nd.a && nd.b >= r.col0 && nd.b < r.col0 + r.count)
+                    return (r.slot0 + nd.b - r.col0) * QRS_COL;
+            return 0;
+        };
+        std::vector<size_t> last_use(nodes.size()), item_of(nodes.size());
+        std::vector<uint32_t> reg(nodes.size(), 0);
+        bool fits = true;
+        for (size_t k = 0; k < S && fits; k++) {
+            const auto& ord = order[k];
+            for (size_t t = 0; t < ord.size(); t++) {
+                const uint32_t n = ord[t].node;
+                const pg_air_node& nd = nodes[n];
+                if (ord[t].is_assert) {
+                    last_use[n] = t;
+                    continue;
+                }
+                item_of[n] = t;
+                if (!air_is_leaf(nodes[nd.a])) last_use[nd.a] = t;
+                if (nd.kind != PG_AIR_NEG && !air_is_leaf(nodes[nd.b])) last_use[nd.b] = t;
+            }
+            const uint32_t base = next;
+            std::set<uint32_t> free_regs;
+            uint32_t nregs = 0;
+            QrSlice sl{};
+            sl.start = (uint32_t)(plan->code.size() / 2);
+            sl.regs = base;
+            auto word = [&](uint32_t n, size_t t, uint32_t prev_flag, uint32_t& fl) -> uint32_t {
+                if (air_is_leaf(nodes[n])) return leaf_word(n);
+                if (item_of[n] + 1 == t) {
+                    fl |= prev_flag;
+                    return zero;
+                }
+                return base + 64 * reg[n];
+            };
+            auto release = [&](uint32_t n, size_t t) {
+                if (!air_is_leaf(nodes[n]) && last_use[n] == t && last_use[n] != item_of[n] + 1) free_regs.insert(reg[n]);
+            };
+            uint32_t assert_at = (uint32_t)first[k];
+            for (size_t t = 0; t < ord.size(); t++) {
+                const uint32_t n = ord[t].node;
+                const pg_air_node& nd = nodes[n];
+                uint32_t fl = 0, a, b, dst = 0, fold = ~0u;
+                if (ord[t].is_assert) {
+                    fold = assert_at++;
+                    if (t && !ord[t - 1].is_assert && ord[t - 1].node == n) {  // fold in the instruction that made it
+                        plan->code.back() |= QF_ASSERT << 16;
+                        plan->folds.back() = fold;
+                        release(n, t);
+                        continue;
+                    }
+                    fl = QF_ADD | QF_ASSERT;
+                    a = air_is_leaf(nd) ? leaf_word(n) : base + 64 * reg[n];
+                    b = zero;
+                    release(n, t);
+                } else {
+                    const bool is_neg = nd.kind == PG_AIR_NEG;
+                    fl = nd.kind == PG_AIR_ADD ? QF_ADD : nd.kind == PG_AIR_MUL ? QF_MUL : QF_SUB;
+                    a = is_neg ? zero : word(nd.a, t, QF_PREV_A, fl);
+                    b = word(is_neg ? nd.a : nd.b, t, QF_PREV_B, fl);
+                    release(nd.a, t);
+                    if (!is_neg && nd.b != nd.a) release(nd.b, t);
+                    if (last_use[n] != t + 1) {  // else only the next instruction reads it
+                        if (free_regs.empty()) {
+                            reg[n] = nregs++;
+                        } else {
+                            reg[n] = *free_regs.begin();
+                            free_regs.erase(free_regs.begin());
+                        }
+                        dst = base + 64 * reg[n];
+                        fl |= QF_WRITE;
+                    }
+                }
+                fits = fits && base + 64 * nregs <= QR_MAX_WORDS;
+                if (!fits) break;
+                plan->code.push_back(a | b << 16);
+                plan->code.push_back(dst | fl << 16);
+                plan->folds.push_back(fold);
+            }
+            while (plan->code.size() % 8) {  // whole groups of four: zero + zero
+                plan->code.push_back(zero | zero << 16);
+                plan->code.push_back(0);
+                plan->folds.push_back(~0u);
+            }
+            sl.end = (uint32_t)(plan->code.size() / 2);
+            plan->slices.push_back(sl);
+            plan->longest = std::max(plan->longest, sl.end - sl.start);
+            next = base + 64 * std::max(nregs, 4u);  // the slice's sums end in its first four
+            fits = fits && next <= QR_MAX_WORDS;
+        }
+        if (!fits) continue;  // fewer slices hold fewer registers
+        while (plan->slices.size() < 4 || (plan->slices.size() & (plan->slices.size() - 1))) {
+            QrSlice sl{};  // a wave that only stages rows and finishes sums
+            sl.start = sl.end = (uint32_t)(plan->code.size() / 2);
+            sl.regs = next;
+            next += 256;
+            plan->slices.push_back(sl);
+        }
+        if (next > QR_MAX_WORDS) continue;
+        plan->lds_words = next;
+        return plan;
+    }
+    return nullptr;
 }
 
 static int air_compile_lowered(int field, const std::vector<pg_air_node>& lnodes, const std::vector<LAssert>& las,
@@ -4140,10 +4437,35 @@ static int air_compile_lowered(int field, const std::vector<pg_air_node>& lnodes
     if (prog->nregs > QUOTIENT_MAX_REGS)
         return fail(PG_E_UNSUPPORTED, "the program needs %u registers; at most %u are supported", prog->nregs,
                     QUOTIENT_MAX_REGS);
+    prog->resident = air_resident(lnodes, las);
     if (nregs_out) *nregs_out = prog->nregs;
     if (ninstr_out) *ninstr_out = (uint32_t)prog->code.size();
     *out = prog.release();
     return PG_OK;
+}
+
+// Which form evaluates `rows` rows.  Each has a latency (the longest chain one
+// wave runs) and a throughput (all rows over the chip); in nanoseconds, fitted
+// to runs of 22 programs of 8..2204 instructions over 2^15..2^21 rows:
+//   windowed: 32 us + max(0.36 us N + 0.9 us S, 3 us N + 15 us S per 2^21 rows)
+//     for N instructions and S staged windows;
+//   resident: 40 us + max(0.17 us L, 110 us + the work + 50 us per piece the
+//     prefetch does not hold, per 2^21 rows), the work 1.5 us an instruction
+//     or, where the slices are uneven, 1 us times waves times the longest L.
+// Measured either side (windowed / resident): 2^18 rows, one product of three
+// columns for each of 4 columns 43 / 59 us, 12 columns 63 / 64, 32 columns 115 /
+// 79; 2^21 rows, 4 columns 100 / 178, 12 columns 291 / 212, 256 columns 4350 /
+// 2000; two interactions over 12 columns, 2^15 rows 111 / 73, 2^21 rows 673 / 858.
+static bool quotient_is_resident(const pg_air_program* prog, uint32_t rows) {
+    const QResident* const r = prog->resident.get();
+    if (!r) return false;
+    const uint64_t S = prog->nstages, N = prog->code.size() - S;
+    const uint64_t W = r->slices.size(), L = r->longest, held = W / 2;  // pieces prefetched: 32 rows of a wave's 64 / W
+    const uint64_t late = r->pieces.size() > held ? r->pieces.size() - held : 0;
+    const uint64_t work = std::max<uint64_t>(1500 * r->folds.size(), 1000 * W * L);
+    const uint64_t windowed = 32000 + std::max<uint64_t>(360 * N + 900 * S, ((3000 * N + 15000 * S) * rows) >> 21);
+    const uint64_t resident = 40000 + std::max<uint64_t>(170 * L, ((110000 + work + 50000 * late) * rows) >> 21);
+    return resident <= windowed;
 }
 
 template <class F>
@@ -4193,8 +4515,29 @@ static int quotient_t(pg_ctx* ctx, hipStream_t s, const pg_air_program* prog, co
             for (int c = 0; c < 4; c++) apow[(size_t)i * 4 + c] = v.c[c];
         }
     }
-    // the kernel reads one instruction past the end (zero padding)
-    const size_t b_code = round_up((prog->code.size() + 1) * sizeof(QInstr), 256), b_zh = round_up(zh.size() * 4, 256),
+    const QResident* const res = quotient_is_resident(prog, q) ? prog->resident.get() : nullptr;
+    // resident: pieces, slices, the code, and a power of alpha per
+    // instruction; windowed: one instruction past the end is read
+    const size_t b_pieces = res ? round_up(res->pieces.size() * sizeof(QrPiece), 256) : 0;
+    const size_t b_slices = res ? b_pieces + round_up(res->slices.size() * sizeof(QrSlice), 256) : 0;
+    if (res) {
+        std::vector<uint32_t> per(4 * (res->folds.size() + QR_PAD), 0);
+        for (size_t i = 0; i < res->folds.size(); i++)
+            if (res->folds[i] != ~0u) memcpy(&per[4 * i], &apow[4 * (size_t)res->folds[i]], 16);
+        apow = std::move(per);
+        consts.clear();
+        for (const auto& c : res->consts) {
+            switch (c.first) {
+                case PG_AIR_PUBLIC: consts.push_back(publics[c.second]); break;
+                case LK_CHAL: consts.push_back(chal[c.second]); break;
+                case LK_RSUM: consts.push_back(rsum[c.second]); break;
+                case LK_GSUM: consts.push_back(gsum[c.second]); break;
+                default: consts.push_back(to_monty<F>(c.second % F::P)); break;
+            }
+        }
+    }
+    const size_t b_code = res ? b_slices + round_up(res->code.size() * 4, 256)
+                              : round_up((prog->code.size() + 1) * sizeof(QInstr), 256), b_zh = round_up(zh.size() * 4, 256),
                  b_const = round_up(consts.size() * 4, 256), b_pow = apow.size() * 4;
     int rc;
     std::shared_ptr<DevMem> tw;
@@ -4209,9 +4552,16 @@ static int quotient_t(pg_ctx* ctx, hipStream_t s, const pg_air_program* prog, co
     auto put = [&](size_t off, const void* src, size_t bytes) {
         if (e == hipSuccess && bytes) e = hipMemcpyAsync(dd + off, src, bytes, hipMemcpyHostToDevice, s);
     };
-    std::vector<QInstr> code = prog->code;
-    code.push_back(QInstr{QOP_STAGE, 0, 0, 0});
-    put(0, code.data(), code.size() * sizeof(QInstr));
+    std::vector<QInstr> code;
+    if (res) {
+        put(0, res->pieces.data(), res->pieces.size() * sizeof(QrPiece));
+        put(b_pieces, res->slices.data(), res->slices.size() * sizeof(QrSlice));
+        put(b_slices, res->code.data(), res->code.size() * 4);
+    } else {
+        code = prog->code;
+        code.push_back(QInstr{QOP_STAGE, 0, 0, 0});
+        put(0, code.data(), code.size() * sizeof(QInstr));
+    }
     put(b_code, zh.data(), zh.size() * 4);
     put(b_code + b_zh, consts.data(), consts.size() * 4);
     put(b_code + b_zh + b_const, apow.data(), b_pow);
@@ -4243,10 +4593,38 @@ static int quotient_t(pg_ctx* ctx, hipStream_t s, const pg_air_program* prog, co
     a.omega_n_inv = finv<F>(to_monty<F>(two_adic_gen_canon<F>(log_n)));
     a.need_selectors = prog->need_selectors;
     a.out = o->ptr;
+    QrArgs ra{};
+    if (res) {
+        const pg_buf* const src[3] = {mm, pm, qm};
+        for (int k = 0; k < 3; k++) {
+            ra.src[k] = src[k] ? src[k]->ptr : nullptr;
+            ra.ld[k] = src[k] ? (uint32_t)src[k]->ld : 0;
+        }
+        ra.pieces = (const QrPiece*)dd;
+        ra.npieces = (uint32_t)res->pieces.size();
+        ra.waves = (uint32_t)res->slices.size();
+        ra.slices = (const QrSlice*)(dd + b_pieces);
+        ra.prog = (const uint32_t*)(dd + b_slices);
+        ra.consts = a.consts;
+        ra.nconsts = a.nconsts;
+        ra.const0 = res->const0;
+        for (int k = 0; k < 3; k++) ra.sel_word[k] = res->sel_word[k];
+        ra.apow = a.apow;
+        ra.tw = a.tw;
+        ra.zh = a.zh;
+        ra.zh_mask = a.zh_mask;
+        ra.q = a.q;
+        ra.log_q = a.log_q;
+        ra.next_step = a.next_step;
+        ra.shift = a.shift;
+        ra.omega_n_inv = a.omega_n_inv;
+        ra.lds_words = res->lds_words;
+        ra.out = a.out;
+    }
     auto kt = make_timer(ctx);
     if (e == hipSuccess) {
         if (kt) kt->begin("quotient", s);
-        e = launch_quotient(prog->field, a, s);
+        e = res ? launch_quotient_resident(prog->field, ra, s) : launch_quotient(prog->field, a, s);
         if (kt) kt->end(s);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);

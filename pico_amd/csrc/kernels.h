@@ -279,6 +279,52 @@ struct QuotientArgs {
     int need_selectors;
     uint32_t* out;         // |Q| x 4
 };
+// The resident form: a workgroup keeps every column its program reads, for 64
+// rows and their next rows, in LDS, and its waves evaluate disjoint slices of
+// the constraints over the same rows (lane = row).  LDS holds, in words: the
+// column slots (QRS_COL words each), then constants, selectors and every
+// slice's registers (64 words each).  An instruction is two words, `a | b <<
+// 16` and `dst | flags << 16`, operands and destination being LDS word indexes
+// to which the lane is added.
+constexpr int QRL = 64;       // rows per workgroup
+constexpr int QRS_COL = 65;   // words per column slot (conflict-free staging writes)
+constexpr uint32_t QF_ADD = 0, QF_SUB = 1, QF_MUL = 2, QF_OP = 3;
+constexpr uint32_t QF_PREV_A = 4, QF_PREV_B = 8, QF_ASSERT = 16, QF_WRITE = 32;
+constexpr int QR_MAX_WAVES = 16, QR_MAX_PIECES = 16;
+constexpr int QR_MIN_SLICE = 24;  // instructions worth a wave
+constexpr int QR_PAD = 128;
+constexpr uint32_t QR_MAX_WORDS = 40832;  // 160 KB of LDS less 512 bytes
+// At most 64 adjacent columns of one source, staged a row per wave-wide load.
+struct QrPiece {
+    uint32_t col, slot;  // first column in its matrix, its slot
+    uint32_t how;        // columns | source << 8 (0 main, 1 preprocessed, 2 permutation) | next rows << 10
+    uint32_t pad_;
+};
+struct QrSlice {
+    uint32_t start, end;  // instructions, whole groups of 4
+    uint32_t regs;        // first register word
+    uint32_t pad_;
+};
+struct QrArgs {
+    const uint32_t* src[3];  // main, preprocessed, permutation (null when unread)
+    uint32_t ld[3];
+    const QrPiece* pieces;
+    uint32_t npieces;
+    uint32_t waves;  // 4, 8 or 16
+    const QrSlice* slices;
+    const uint32_t* prog;     // 2 words each
+    const uint32_t* consts;
+    uint32_t nconsts, const0;
+    // per instruction, its power of alpha where it asserts (ext4), then QR_PAD entries
+    const uint32_t* apow;
+    uint32_t sel_word[3];     // is_first_row, is_last_row, is_transition: LDS word, or 0 when unread
+    const uint32_t* tw;
+    const uint32_t* zh;
+    uint32_t zh_mask, q, log_q, next_step, shift, omega_n_inv;
+    uint32_t lds_words;
+    uint32_t* out;
+};
+hipError_t launch_quotient_resident(int field, const QrArgs& a, hipStream_t stream);
 size_t quotient_lds_bytes(uint32_t nregs, uint32_t nslots, bool selectors, uint32_t nconsts);
 hipError_t launch_quotient(int field, const QuotientArgs& a, hipStream_t stream);
 }  // namespace pg

@@ -34,6 +34,7 @@
 // is_last_row = Z_H(x) / (x - w_n^-1), is_transition = x - w_n^-1.  x^n =
 // GEN^n w_{2^qdb}^(i mod 2^qdb) takes 2^qdb values, tabulated with their
 // inverses on the host.
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.h"
@@ -92,8 +93,9 @@ __global__ void __launch_bounds__(QT) quotient_kernel(QuotientArgs a) {
             const uint32_t x = fmul<F>(a.shift, ((gcptr)a.tw)[i]);
             const uint32_t trans = fsub<F>(x, a.omega_n_inv);
             uint32_t* const sel = lds + sbase + t + (uint32_t)(QT * k);
-            sel[0] = fmul<F>(zh, finv<F>(fsub<F>(x, F::R1)));  // is_first_row
-            sel[QB] = fmul<F>(zh, finv<F>(trans));               // is_last_row
+            const uint32_t first = fsub<F>(x, F::R1), inv = fmul<F>(zh, finv<F>(fmul<F>(first, trans)));
+            sel[0] = fmul<F>(trans, inv);   // is_first_row = Z_H / (x - 1)
+            sel[QB] = fmul<F>(first, inv);  // is_last_row = Z_H / (x - w_n^-1)
             sel[2 * QB] = trans;                                  // is_transition
         }
     }
@@ -253,6 +255,209 @@ __global__ void __launch_bounds__(QT) quotient_kernel(QuotientArgs a) {
             const Ext4 q = escale<F>(acc[k], inv_zh[k]);
             reinterpret_cast<GLOBAL u32x4*>((gptr)a.out)[nat[k]] = u32x4{q.c[0], q.c[1], q.c[2], q.c[3]};
         }
+    }
+}
+
+// ---- resident form ------------------------------------------------------------
+// What bounded the windowed form above: a window takes 32 bytes of each row's
+// 128-byte line and the line is gone from L2 before its next window (34 GB
+// fetched for 4.3 GB over 2^21 rows x 256 columns), and one wave runs the whole
+// program alone at about 0.4 us an instruction, so a short domain is latency.
+// Here the 64 rows of a workgroup are read once, whole runs of columns at a
+// time, and stay in LDS (160 KB: 512 column slots and the registers); the
+// constraints are split over up to 16 waves, each with its own registers, whose
+// sums meet at the end of a block.  The next block's rows are fetched into VGPRs
+// while the program runs.  Rows map to lanes; the next row of lane u sits in
+// lane u of its slot, so every operand is LDS word index + lane.
+//
+// Now bound by the vector operations of the interpreter: about 14 an
+// instruction, of which the arithmetic is 5 (product) or 4 (sum) and an assert
+// adds 4 products; staging alone takes 0.93 of the 2.0 ms below.  Measured
+// against the windowed form: 2^21 rows x 256 columns 4.45 -> 2.00 ms, 2^18 rows
+// x 90 columns with 24 interactions 1.39 -> 0.44 ms, 2^9 rows x 256 columns 560
+// -> 79 us.  Handling an instruction without branches (both results, always
+// written) took 2.33 ms and 0.43, reading the powers with the program 2.33 and
+// 0.48.
+template <class F, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4, 4)))
+quotient_resident_kernel(const QrArgs a) {
+    extern __shared__ uint32_t lds[];
+    constexpr int RW = QRL / WAVES;  // rows of a block that a wave stages
+    constexpr int PF = 32 / RW;      // pieces whose words are in flight during the program
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    constexpr uint32_t nt = 64 * WAVES;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    // With |Q| < 64 one block of B = |Q| rows; the lanes above compute on
+    // whatever their words hold and are never stored.
+    const uint32_t log_b = a.log_q < 6u ? a.log_q : 6u, B = 1u << log_b;
+    const uint32_t log_nb = a.log_q - log_b, nb = 1u << log_nb;
+    // contiguous ranges of logical blocks (see quotient_block) per workgroup,
+    // consecutive workgroups of an XCD side by side
+    const uint32_t g = gridDim.x, x8 = blockIdx.x & 7u, y8 = blockIdx.x >> 3, q8 = g >> 3, r8 = g & 7u;
+    const uint32_t wg = x8 * q8 + (x8 < r8 ? x8 : r8) + y8;
+    const uint32_t b0 = (uint32_t)((uint64_t)wg * nb / g), b1 = (uint32_t)((uint64_t)(wg + 1) * nb / g);
+    for (uint32_t w = tid; w < a.nconsts * 64u; w += nt) lds[a.const0 + w] = a.consts[w >> 6];
+    const QrSlice sl = a.slices[wave];
+    // The program by scalar loads, four instructions at a time (the compiler's
+    // constant address space); taking it from lanes with readlane, as the windowed
+    // form does, cost 2 of ~14 vector operations an instruction.
+    typedef const __attribute__((address_space(4))) u32x4* cptr;
+    const cptr cg = (cptr)(uintptr_t)a.prog;
+    const GLOBAL u32x4* const pw = reinterpret_cast<const GLOBAL u32x4*>((gcptr)a.apow) + sl.start;
+    const uint32_t ninstr = sl.end - sl.start;
+    // Every block stages the same pieces and runs the same program: lane k
+    // holds piece k; the powers of alpha of the first 128 instructions stay in
+    // VGPRs.  (Vector loads return in order: one in the program would wait for
+    // the prefetch before it.)
+    uint32_t t_col = 0, t_slot = 0, t_how = 0;
+    if (lane < a.npieces) {
+        const QrPiece t = a.pieces[lane];
+        t_col = t.col;
+        t_slot = t.slot;
+        t_how = t.how;
+    }
+    const u32x4 w0 = pw[lane], w1 = pw[64 + lane];  // padded past the end
+
+    // Logical block b has natural indexes (rev(v) << log_nb) + b for its rows
+    // v < B (log_b-bit reversal), so the next rows are those of block (b +
+    // step) mod nb, with v's reversal advanced by the carry: row v of that
+    // block is the next row of lane u = rev(rev(v) - carry).  The wave stages
+    // rows v0 .. v0 + RW - 1, a row per load, columns across the lanes.
+    const uint32_t v0 = wave * (uint32_t)RW;
+    auto piece = [&](uint32_t k, uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)k); };
+    auto fetch = [&](uint32_t k, uint32_t b, uint32_t* out) {
+        const uint32_t how = piece(k, t_how), s = (how >> 8) & 3u, last = (how & 255u) - 1u;
+        const uint32_t r = rev_bits((how >> 10) ? (b + a.next_step) & (nb - 1u) : b, log_nb) << log_b;
+        const uint32_t ld = s == 0 ? a.ld[0] : s == 1 ? a.ld[1] : a.ld[2];
+        const gcptr base = (gcptr)(s == 0 ? a.src[0] : s == 1 ? a.src[1] : a.src[2]) + piece(k, t_col);
+        const uint32_t c = lane < last ? lane : last;  // surplus lanes repeat the last column
+#pragma unroll
+        for (int i = 0; i < RW; i++) {
+            const uint32_t v = v0 + i < B ? v0 + i : B - 1u;  // and rows past a short block its last row
+            out[i] = (base + (uint64_t)(r + v) * ld)[c];
+        }
+    };
+    auto put = [&](uint32_t k, const uint32_t* in, uint32_t carry) {
+        const uint32_t how = piece(k, t_how), n = how & 255u;
+        const uint32_t w = (piece(k, t_slot) + lane) * (uint32_t)QRS_COL;
+        if (lane >= n) return;
+        if (B < 64u || ((how >> 10) && carry)) {
+#pragma unroll
+            for (int i = 0; i < RW; i++) {
+                uint32_t u = v0 + i;
+                if (u >= B) continue;
+                if (how >> 10) u = rev_bits((rev_bits(u, log_b) - carry) & (B - 1u), log_b);
+                lds[w + u] = in[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < RW; i++) lds[w + v0 + i] = in[i];
+        }
+    };
+    uint32_t pf[PF * RW], x_tw = 0, x_zh = 0, x_zi = 0;
+    auto prefetch = [&](uint32_t b) {
+#pragma unroll
+        for (uint32_t k = 0; k < (uint32_t)PF; k++)
+            if (k < a.npieces) fetch(k, b, &pf[k * RW]);
+        // w_Q^i and Z_H of the lane's row (selectors), 1 / Z_H of the row whose sum the thread finishes
+        const uint32_t i = (rev_bits(lane & (B - 1u), log_b) << log_nb) + b;
+        x_tw = ((gcptr)a.tw)[i];
+        x_zh = ((gcptr)a.zh)[i & a.zh_mask];
+        const uint32_t j = (rev_bits((tid >> 2) & (B - 1u), log_b) << log_nb) + b;
+        x_zi = ((gcptr)a.zh)[a.zh_mask + 1 + (j & a.zh_mask)];
+    };
+    if (b0 < b1) prefetch(b0);
+    for (uint32_t b = b0; b < b1; b++) {
+        const uint32_t carry = (b + a.next_step) >> log_nb;
+#pragma unroll
+        for (uint32_t k = 0; k < (uint32_t)PF; k++)
+            if (k < a.npieces) put(k, &pf[k * RW], carry);
+        for (uint32_t k = PF; k < a.npieces; k++) {
+            uint32_t late[RW];
+            fetch(k, b, late);
+            put(k, late, carry);
+        }
+        for (uint32_t k = wave; k < 3; k += WAVES) {
+            if (!a.sel_word[k]) continue;
+            const uint32_t x = fmul<F>(a.shift, x_tw), trans = fsub<F>(x, a.omega_n_inv);
+            lds[a.sel_word[k] + lane] = k == 2 ? trans : fmul<F>(x_zh, finv<F>(k == 0 ? fsub<F>(x, F::R1) : trans));
+        }
+        const uint32_t zi = x_zi;
+        __syncthreads();
+        if (b + 1 < b1) prefetch(b + 1);
+        // the wave's slice
+        LazyDot<F> acc[4];
+        uint32_t prev = 0, since_fold = 0;
+        auto one = [&](uint32_t ops, uint32_t dst, u32x4 wl, uint32_t at) {
+            const uint32_t fl = dst >> 16;
+            const uint32_t la = lds[(ops & 0xffffu) + lane], lb = lds[(ops >> 16) + lane];
+            const uint32_t va = (fl & QF_PREV_A) ? prev : la, vb = (fl & QF_PREV_B) ? prev : lb;
+            if (fl & QF_MUL)
+                prev = fmul<F>(va, vb);
+            else
+                prev = fadd<F>(va, (fl & QF_SUB) ? F::P - vb : vb);  // vb = 0: va + p reduces to va
+            if (fl & QF_WRITE) lds[(dst & 0xffffu) + lane] = prev;
+            if (fl & QF_ASSERT) {  // the power is in lane `at` of wl
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e].add(prev, (uint32_t)__builtin_amdgcn_readlane((int)wl[e], (int)at));
+                if (++since_fold == 3) {
+                    since_fold = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[e].fold();
+                }
+            }
+        };
+        auto run = [&](uint32_t pc0, u32x4 wl, uint32_t cnt) {
+            for (uint32_t i = 0; i < cnt; i += 4) {
+                const u32x4 c0 = cg[(pc0 + i) / 2], c1 = cg[(pc0 + i) / 2 + 1];
+                one(c0[0], c0[1], wl, i);
+                one(c0[2], c0[3], wl, i + 1);
+                one(c1[0], c1[1], wl, i + 2);
+                one(c1[2], c1[3], wl, i + 3);
+            }
+        };
+        run(sl.start, w0, ninstr < 64u ? ninstr : 64u);
+        if (ninstr > 64u) run(sl.start + 64u, w1, ninstr < 128u ? ninstr - 64u : 64u);
+        for (uint32_t pc = 128; pc < ninstr; pc += 64) run(sl.start + pc, pw[pc + lane], ninstr - pc < 64u ? ninstr - pc : 64u);
+#pragma unroll
+        for (int e = 0; e < 4; e++) lds[sl.regs + 64u * e + lane] = acc[e].value();
+        __syncthreads();
+        // sum over the slices, times 1 / Z_H: thread -> (row, coordinate)
+        if (tid < 4u * B) {
+            const uint32_t e = tid & 3u, u = tid >> 2;
+            uint32_t s = 0;
+            for (uint32_t w = 0; w < (uint32_t)WAVES; w++) s = fadd<F>(s, lds[a.slices[w].regs + 64u * e + u]);
+            const uint32_t n = (rev_bits(u, log_b) << log_nb) + b;
+            ((gptr)a.out)[4 * (uint64_t)n + e] = fmul<F>(s, zi);
+        }
+    }
+}
+
+template <class F, int WAVES>
+static hipError_t run_resident(const QrArgs& a, hipStream_t stream) {
+    const uint32_t nb = (a.q + QRL - 1) / QRL;
+    const size_t lds = (size_t)a.lds_words * 4;
+    // 16 waves per CU (128 registers): as many workgroups as waves and LDS allow
+    const uint32_t per_cu = std::max<uint32_t>(1u, std::min<uint32_t>(16u / WAVES, (uint32_t)(163840 / lds)));
+    const unsigned grid = std::min(nb, 256u * per_cu);
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)quotient_resident_kernel<F, WAVES>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    quotient_resident_kernel<F, WAVES><<<grid, 64 * WAVES, lds, stream>>>(a);
+    return hipGetLastError();
+}
+
+hipError_t launch_quotient_resident(int field, const QrArgs& a, hipStream_t stream) {
+    if (a.q == 0) return hipSuccess;
+    if (a.npieces > (uint32_t)QR_MAX_PIECES || a.lds_words == 0 || a.lds_words > QR_MAX_WORDS) return hipErrorInvalidValue;
+    const bool kb = field == FIELD_KOALABEAR;
+    switch (a.waves) {
+        case 16: return kb ? run_resident<KoalaBear, 16>(a, stream) : run_resident<BabyBear, 16>(a, stream);
+        case 8: return kb ? run_resident<KoalaBear, 8>(a, stream) : run_resident<BabyBear, 8>(a, stream);
+        case 4: return kb ? run_resident<KoalaBear, 4>(a, stream) : run_resident<BabyBear, 4>(a, stream);
+        default: return hipErrorInvalidValue;
     }
 }
 
