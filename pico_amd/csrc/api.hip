@@ -3079,7 +3079,9 @@ extern "C" int pg_fri_grind(pg_ctx* ctx, int field, pg_challenger* ch, int bits,
     hipError_t e = hipMemcpyAsync(dstate, ch->state, 64, hipMemcpyHostToDevice, l.s);
     if (e == hipSuccess) e = hipMemcpyAsync(din, ch->input, 32, hipMemcpyHostToDevice, l.s);
     if (e == hipSuccess) e = hipMemcpyAsync(dres, &hres, 4, hipMemcpyHostToDevice, l.s);
-    const uint32_t chunk = 1u << 22;
+    // eight times the expected number of candidates per launch (a wave leaves it
+    // once a smaller witness is known), 2^16 to 2^22
+    const uint32_t chunk = 1u << std::min(std::max(bits + 3, 16), 22);
     for (uint32_t start = 0; e == hipSuccess && start < P; start += chunk) {
         const uint32_t count = std::min<uint32_t>(chunk, P - start);
         e = launch_pow_search(field, dstate, din, ch->n_input, bits, start, count, dres, l.s);

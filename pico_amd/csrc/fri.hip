@@ -1,5 +1,4 @@
-// fri.hip -- FRI arity-2 fold, proof-of-work search, and the
-// element-wise helpers (representation conversion, seeded synthetic inputs).
+// fri.hip -- FRI arity-2 fold, and the element-wise helpers (representation conversion, seeded synthetic inputs).
 //
 // Fold semantics (p3 fold_even_odd; pinned in-tree by the query check at
 // vm/src/compiler/recursion/circuit/fri.rs:288-387): the committed vector is
@@ -7,10 +6,8 @@
 // values at x_i and -x_i with x_i = w_n^{rev_{log(n/2)}(i)}; the folded value
 // is the line through both points evaluated at beta:
 //   out[i] = (v[2i] + v[2i+1]) / 2 + beta/2 * (v[2i] - v[2i+1]) * x_i^{-1}.
-// PoW semantics: DuplexChallenger::check_witness (circuit/challenger.rs:210-222):
-// observe(w) then sample_bits(bits) == 0.
 #include "kernels.h"
-#include "poseidon2.h"
+#include "field.h"
 
 namespace pg {
 
@@ -43,30 +40,6 @@ __global__ void __launch_bounds__(256) fri_fold_kernel(const uint32_t* __restric
         o = eadd<F>(o, Ext4{{w.x, w.y, w.z, w.w}});
     }
     reinterpret_cast<uint4*>(out)[i] = make_uint4(o.c[0], o.c[1], o.c[2], o.c[3]);
-}
-
-template <class F>
-__global__ void __launch_bounds__(256) pow_kernel(const uint32_t* __restrict__ state,
-                                                  const uint32_t* __restrict__ in, int n_in, int bits,
-                                                  uint32_t start, uint32_t count, uint32_t* result) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const uint32_t w = start + i;
-    if (w >= F::P) return;
-    // observe(w) then sample(): either way the pending inputs and w overwrite
-    // state[0..n_in], one permutation runs, and the sample is state[7].
-    uint32_t st[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) st[j] = state[j];
-    const uint32_t wm = to_monty<F>(w);
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        if (j < n_in) st[j] = in[j];
-        if (j == n_in) st[j] = wm;
-    }
-    permute<F>(st);
-    const uint32_t v = from_monty<F>(st[7]);
-    if ((v & ((1u << bits) - 1u)) == 0u) atomicMin(result, w);
 }
 
 template <class F>
@@ -133,16 +106,6 @@ hipError_t launch_rows_bitrev(const uint32_t* src, uint64_t ld, uint32_t w, int 
                               uint32_t* dst, hipStream_t stream) {
     if (nrows == 0 || w == 0) return hipSuccess;
     rows_bitrev_kernel<<<blocks(nrows * w), 256, 0, stream>>>(src, ld, w, q, r0, nrows, dst);
-    return hipGetLastError();
-}
-
-hipError_t launch_pow_search(int field, const uint32_t* state, const uint32_t* in, int n_in, int bits,
-                             uint32_t start, uint32_t count, uint32_t* result, hipStream_t stream) {
-    if (count == 0) return hipSuccess;
-    if (field == FIELD_KOALABEAR)
-        pow_kernel<KoalaBear><<<blocks(count), 256, 0, stream>>>(state, in, n_in, bits, start, count, result);
-    else
-        pow_kernel<BabyBear><<<blocks(count), 256, 0, stream>>>(state, in, n_in, bits, start, count, result);
     return hipGetLastError();
 }
 

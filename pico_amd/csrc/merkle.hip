@@ -737,6 +737,67 @@ static unsigned small_grid(uint64_t n) { return (unsigned)((n + 16 * S_WAVES - 1
 // so the table load of a workgroup is shared by its waves' nodes.
 static unsigned mx_grid_loop(uint64_t n) { return std::min(mx_grid(n), 1024u); }
 
+// ---- proof of work ------------------------------------------------------------
+// check_witness (circuit/challenger.rs:210-222): observe(w), then sample_bits(bits)
+// == 0.  Either way the n_in pending inputs and w overwrite words 0..n_in of the
+// state, one permutation runs, and the sample is word 7.  64 candidates per wave,
+// ascending over the grid; a wave stops once a smaller witness is known, so a
+// launch costs what the smallest witness needs and not its whole range (2^22
+// candidates, one thread each, took 500 us whatever the witness; 16 bits now 26).
+template <class F>
+MX_KERNEL pow_kernel(const uint32_t* state, const uint32_t* in, int n_in, uint32_t mask, uint32_t start,
+                     uint32_t count, uint32_t* result) {
+    __shared__ MxTable<F> tab;
+    mx_load<F>(tab);
+    MxView<F> v(tab);
+    const MxLane l;
+    uint32_t word[2][4];  // of the lane: words 4 h + i and 8 + 4 h + i
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int j = 4 * (int)l.h + i;
+        word[0][i] = j < n_in ? in[j] : state[j];
+        word[1][i] = state[8 + j];
+    }
+    const uint64_t stride = (uint64_t)gridDim.x * MX_WAVES;
+    for (uint64_t group = mx_wave(); 64 * group < count; group += stride) {
+        const uint32_t w0 = start + (uint32_t)(64 * group);
+        const uint32_t known = __hip_atomic_load(result, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)known) < w0) return;
+        mx4 st[2][2], b[2][2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint32_t wm = to_monty<F>(w0 + 32 * t + l.n);  // past count: computed, not reported
+            u32x4 rate;
+#pragma unroll
+            for (int i = 0; i < 4; i++) rate[i] = 4 * (int)l.h + i == n_in ? wm : word[0][i];
+            st[t][0] = mx_op(rate);
+            st[t][1] = mx_op(u32x4{word[1][0], word[1][1], word[1][2], word[1][3]});
+        }
+        int x[2][8];
+        uint32_t out[2][8];
+        v.fresh();
+        mx_init<F>(x, st, v);
+        mx_rounds<F>(b, x, v);
+        mx_last<F>(out, b, v);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint64_t c = 64 * group + 32 * t + l.n;
+            if (l.h && c < count && (from_monty<F>(out[t][3]) & mask) == 0) atomicMin(result, start + (uint32_t)c);
+        }
+    }
+}
+
+hipError_t launch_pow_search(int field, const uint32_t* state, const uint32_t* in, int n_in, int bits,
+                             uint32_t start, uint32_t count, uint32_t* result, hipStream_t stream) {
+    if (count == 0) return hipSuccess;
+    const uint32_t mask = (1u << bits) - 1u;
+    if (field == FIELD_KOALABEAR)
+        pow_kernel<KoalaBear><<<mx_grid_loop(count), MX_THREADS, 0, stream>>>(state, in, n_in, mask, start, count, result);
+    else
+        pow_kernel<BabyBear><<<mx_grid_loop(count), MX_THREADS, 0, stream>>>(state, in, n_in, mask, start, count, result);
+    return hipGetLastError();
+}
+
 hipError_t launch_gather_roots(const uint32_t* const* src, uint32_t* dst, int n, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     gather_roots_kernel<<<grid_for((uint64_t)n * 8, 256), 256, 0, stream>>>(src, dst, n);
