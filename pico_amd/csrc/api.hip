@@ -1929,13 +1929,20 @@ static Ext4 bary_factor(const Ext4& z, uint32_t s_mont, int log_h) {
 // matrices of one Pcs::open that share both (every matrix of a round's
 // height, opened at zeta and its own next point) share one computation.
 // Key: log height, point count, the points' words.
-struct WeightCache {
-    std::map<std::vector<uint32_t>, std::shared_ptr<DevMem>> bufs;
+// The matrices of one Pcs::open also share one stream: their launches are queued
+// without a wait between them, the partial sums in one scratch buffer (the stream
+// orders its uses), the values side by side in `out`.
+struct OpenQueue {
+    std::map<std::vector<uint32_t>, std::shared_ptr<DevMem>> weights;
+    std::vector<std::shared_ptr<DevMem>> scratch;  // the last is the largest; the others may be in use
+    size_t scratch_bytes = 0;
+    std::vector<std::shared_ptr<DevMem>> twiddles;
+    uint8_t* out = nullptr;  // of the next matrix
 };
 
 template <class F>
 static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k, uint32_t log_blowup,
-                         const uint32_t* points, size_t npts, uint32_t* out, WeightCache* wc = nullptr,
+                         const uint32_t* points, size_t npts, uint32_t* out, OpenQueue* oq = nullptr,
                          const FixedScratch* fixed = nullptr) {
     const pg_buf* m = t->mats[k];
     if (!is_pow2(m->rows) || (m->rows >> log_blowup) == 0 || log2_of(m->rows) < (int)log_blowup)
@@ -1967,10 +1974,10 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
         // column sums in slices of about 64 chunks (at most 64 slices)
         y.nslices = std::max<uint32_t>(1, std::min<uint32_t>(64, y.nchunks / 64));
         y.b_t = fixed ? round_up(4 * h, 256) : 0;
-        y.b_w = wc ? 0 : round_up(q_max * h * 16, 256);
+        y.b_w = oq ? 0 : round_up(q_max * h * 16, 256);
         y.b_p = round_up(q_max * y.nchunks * w * 16, 256);
         y.b_s = round_up(q_max * y.nslices * w * 16, 256);
-        y.b_o = npts * w * 16;
+        y.b_o = oq ? 0 : npts * w * 16;
         return y;
     };
     Layout y = layout(chunk_rows);
@@ -1992,8 +1999,19 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
         PG_TRY(get_twiddles(ctx, s, t->field, log_h, &tw));
         twp = (const uint32_t*)tw->ptr;
         int rc;
-        scratch = make_devmem(ctx, y.total(), &rc);
-        if (!scratch) return rc;
+        if (oq && y.total() <= oq->scratch_bytes) {
+            scratch = oq->scratch.back();
+        } else {
+            scratch = make_devmem(ctx, y.total(), &rc);
+            if (!scratch) return rc;
+        }
+        if (oq) {
+            if (y.total() > oq->scratch_bytes) {
+                oq->scratch.push_back(scratch);
+                oq->scratch_bytes = y.total();
+            }
+            oq->twiddles.push_back(tw);
+        }
         base = (uint8_t*)scratch->ptr;
     }
     SyncGuard guard(s);  // an early return waits for queued kernels before the scratch is released
@@ -2001,7 +2019,7 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
     uint8_t* const wts = base + y.b_t;
     uint8_t* const partial = wts + y.b_w;
     uint8_t* const sums = partial + y.b_p;
-    uint8_t* const outs = sums + y.b_s;
+    uint8_t* const outs = oq ? oq->out : sums + y.b_s;
     const uint32_t s_mont = to_monty<F>(F::GEN);
     std::unique_ptr<EventTimer> kt = fixed ? nullptr : make_timer(ctx);
     for (size_t q0 = 0; q0 < npts; q0 += per) {
@@ -2013,11 +2031,11 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
         }
         Ext4* weights = (Ext4*)wts;
         int ready = 0;
-        if (wc) {
+        if (oq) {
             std::vector<uint32_t> key{(uint32_t)log_h, (uint32_t)nq};
             for (int q = 0; q < nq; q++) key.insert(key.end(), z[q].c, z[q].c + 4);
-            auto it = wc->bufs.find(key);
-            if (it != wc->bufs.end()) {
+            auto it = oq->weights.find(key);
+            if (it != oq->weights.end()) {
                 weights = (Ext4*)it->second->ptr;
                 ready = 1;
             } else {
@@ -2025,7 +2043,7 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
                 auto wb = make_devmem(ctx, (size_t)nq * h * 16, &rc);
                 if (!wb) return rc;
                 weights = (Ext4*)wb->ptr;
-                wc->bufs.emplace(std::move(key), std::move(wb));
+                oq->weights.emplace(std::move(key), std::move(wb));
             }
         }
         TIMED(kt, "open_values", s,
@@ -2033,26 +2051,25 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
                                  (Ext4*)partial, y.nchunks, chunk_rows, (Ext4*)sums, y.nslices,
                                  (Ext4*)(outs + q0 * w * 16), s));
     }
+    if (oq) {  // the caller waits
+        guard.armed = false;
+        oq->out += npts * w * 16;
+        return PG_OK;
+    }
     HIP_TRY(hipMemcpyAsync(out, outs, y.b_o, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     guard.armed = false;
     return PG_OK;
 }
 
-static int open_values_cached(pg_ctx* ctx, const pg_tree* t, size_t k, uint32_t log_blowup,
-                              const uint32_t* points_mont, size_t npts, uint32_t* out_mont, WeightCache* wc) {
+extern "C" int pg_pcs_open_values(pg_ctx* ctx, const pg_tree* t, size_t k, uint32_t log_blowup,
+                                  const uint32_t* points_mont, size_t npts, uint32_t* out_mont) {
     if (!ctx || !t || (npts && (!points_mont || !out_mont)) || k >= t->mats.size())
         return fail(PG_E_INVALID, "bad argument");
     PG_TRY(bind_device(ctx));
     Lease l(ctx);
-    return t->field == PG_KOALABEAR
-               ? open_values_t<KoalaBear>(ctx, l.s, t, k, log_blowup, points_mont, npts, out_mont, wc)
-               : open_values_t<BabyBear>(ctx, l.s, t, k, log_blowup, points_mont, npts, out_mont, wc);
-}
-
-extern "C" int pg_pcs_open_values(pg_ctx* ctx, const pg_tree* t, size_t k, uint32_t log_blowup,
-                                  const uint32_t* points_mont, size_t npts, uint32_t* out_mont) {
-    return open_values_cached(ctx, t, k, log_blowup, points_mont, npts, out_mont, nullptr);
+    return t->field == PG_KOALABEAR ? open_values_t<KoalaBear>(ctx, l.s, t, k, log_blowup, points_mont, npts, out_mont)
+                                    : open_values_t<BabyBear>(ctx, l.s, t, k, log_blowup, points_mont, npts, out_mont);
 }
 
 // The same values with the device's static scratch array instead of
@@ -3185,23 +3202,58 @@ extern "C" int pg_pcs_open(pg_ctx* ctx, const pg_tree* const* rounds, size_t nro
     if (!points_mont) return fail(PG_E_INVALID, "null points");
     std::unique_ptr<pg_open_proof> pf(new pg_open_proof);
     pf->field = field;
-    // 1. values, observed in order
+    // 1. values, observed in order.  Every matrix is queued first; the values come
+    // down and are observed a few matrices at a time while the rest is computed.
     pf->values.resize(nvals);
-    size_t voff = 0, poff = 0;
-    mi = 0;
     {
-        WeightCache wc;  // freed once every value is on the host (each call synchronises)
+        struct Part {  // values [begin, end) are ready at `done`
+            size_t begin, end;
+            hipEvent_t done;
+        };
+        struct Parts : std::vector<Part> {
+            ~Parts() {
+                for (Part& p : *this)
+                    if (p.done) (void)hipEventDestroy(p.done);
+            }
+        } parts;
+        constexpr size_t PART_WORDS = 2048;  // about 0.13 ms of observing
+        OpenQueue oq;
+        PG_TRY(bind_device(ctx));
+        int rc = PG_OK;
+        auto values = make_devmem(ctx, std::max<size_t>(nvals * 4, 16), &rc);
+        if (!values) return rc;
+        oq.out = (uint8_t*)values->ptr;
+        Lease l(ctx), down(ctx);
+        SyncGuard guard(l.s);
+        size_t voff = 0, poff = 0, begin = 0;
+        mi = 0;
         for (size_t r = 0; r < nrounds; r++)
             for (size_t k = 0; k < rounds[r]->mats.size(); k++, mi++) {
                 const uint32_t np = npoints[mi];
                 if (np)
-                    PG_TRY(open_values_cached(ctx, rounds[r], k, log_blowup, points_mont + 4 * poff, np,
-                                              pf->values.data() + voff, &wc));
+                    PG_TRY(field == PG_KOALABEAR ? open_values_t<KoalaBear>(ctx, l.s, rounds[r], k, log_blowup,
+                                                                            points_mont + 4 * poff, np, nullptr, &oq)
+                                                 : open_values_t<BabyBear>(ctx, l.s, rounds[r], k, log_blowup,
+                                                                           points_mont + 4 * poff, np, nullptr, &oq));
                 voff += (size_t)np * rounds[r]->mats[k]->cols * 4;
                 poff += np;
+                if (voff - begin >= PART_WORDS || (voff == nvals && voff > begin)) {
+                    parts.push_back(Part{begin, voff, nullptr});
+                    HIP_TRY(hipEventCreateWithFlags(&parts.back().done, hipEventDisableTiming));
+                    HIP_TRY(hipEventRecord(parts.back().done, l.s));
+                    begin = voff;
+                }
             }
+        pg_challenger observed = *ch;  // kept only if every value came down
+        for (const Part& p : parts) {
+            HIP_TRY(hipStreamWaitEvent(down.s, p.done, 0));
+            HIP_TRY(hipMemcpyAsync(pf->values.data() + p.begin, (const uint32_t*)values->ptr + p.begin,
+                                   (p.end - p.begin) * 4, hipMemcpyDeviceToHost, down.s));
+            HIP_TRY(hipStreamSynchronize(down.s));
+            for (size_t i = p.begin; i < p.end; i++) pg_challenger_observe(&observed, pf->values[i]);
+        }
+        *ch = observed;
     }
-    for (uint32_t v : pf->values) pg_challenger_observe(ch, v);
     // 2. alpha, reduced openings per height
     pg_challenger_sample_ext(ch, pf->alpha);
     pg_buf* by_log[33];

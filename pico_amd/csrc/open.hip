@@ -31,17 +31,22 @@ __device__ __forceinline__ u32x4 v4_of(const Ext4& e) { return u32x4{e.c[0], e.c
 typedef GLOBAL u32x4* gext;
 typedef const GLOBAL u32x4* gcext;
 
+// one value per point of a launch (grid z or y)
+struct OvPoints {
+    Ext4 v[4];
+};
+
 // c_r = w^j / (z - s w^j), j = rev_h(r): the weight of committed row r
 template <class F>
-__global__ void bary_weights_kernel(Ext4 z, uint32_t shift, int log_h, gcptr __restrict__ tw,
+__global__ void bary_weights_kernel(OvPoints z, uint32_t shift, int log_h, gcptr __restrict__ tw,
                                     gext __restrict__ out) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= (1u << log_h)) return;
     const uint32_t j = log_h ? __brev(r) >> (32 - log_h) : 0u;
     const uint32_t wj = tw[j];
-    Ext4 d = z;
+    Ext4 d = z.v[blockIdx.y];
     d.c[0] = fsub<F>(d.c[0], fmul<F>(shift, wj));
-    out[r] = v4_of(escale<F>(einv<F>(d), wj));
+    out[((uint64_t)blockIdx.y << log_h) + r] = v4_of(escale<F>(einv<F>(d), wj));
 }
 
 // partial[q][chunk][col] = sum over rows r of the chunk of M[r][col] c_q[r]
@@ -181,6 +186,7 @@ __global__ void __launch_bounds__(256) column_dot4_kernel(gcptr __restrict__ m, 
 // are 64 columns by 4 interleaved chunk lanes, so each wave reads 64
 // adjacent columns' partials (1 KB contiguous) per step; the 4 lanes meet in
 // LDS.  Stage 2: per column, the slices' sums times the barycentric factor.
+// Grid z (stage 1) and y (stage 2) are the points.
 constexpr int SUM_UNROLL = 8;  // partial sums loaded per round trip
 
 template <class F>
@@ -190,6 +196,8 @@ __global__ void __launch_bounds__(256) column_slice_sum_kernel(gcext __restrict_
     __shared__ uint32_t red[4][4][64];
     const uint32_t cl = threadIdx.x % 64, kl = threadIdx.x / 64;
     const uint32_t col = blockIdx.x * 64 + cl, y = blockIdx.y;
+    partial += (uint64_t)blockIdx.z * nchunks * w;
+    sums += (uint64_t)blockIdx.z * nslices * w;
     const uint32_t per = (nchunks + nslices - 1) / nslices;
     const uint32_t k0 = y * per, k1 = k0 + per < nchunks ? k0 + per : nchunks;
     Ext4 s{{0, 0, 0, 0}};
@@ -221,9 +229,10 @@ __global__ void __launch_bounds__(256) column_slice_sum_kernel(gcext __restrict_
 
 template <class F>
 __global__ void __launch_bounds__(256) column_finish_kernel(gcext __restrict__ sums, uint32_t nslices, uint32_t w,
-                                                            Ext4 factor, gext __restrict__ out) {
+                                                            OvPoints factor, gext __restrict__ out) {
     const uint32_t col = blockIdx.x * blockDim.x + threadIdx.x;
     if (col >= w) return;
+    sums += (uint64_t)blockIdx.y * nslices * w;
     Ext4 s{{0, 0, 0, 0}};
     for (uint32_t y = 0; y < nslices; y += SUM_UNROLL) {
         Ext4 v[SUM_UNROLL];
@@ -233,7 +242,7 @@ __global__ void __launch_bounds__(256) column_finish_kernel(gcext __restrict__ s
 #pragma unroll
         for (int u = 0; u < SUM_UNROLL; u++) s = eadd<F>(s, v[u]);
     }
-    out[col] = v4_of(emul<F>(s, factor));
+    out[(uint64_t)blockIdx.y * w + col] = v4_of(emul<F>(s, factor.v[blockIdx.y]));
 }
 
 // Reduced opening of one log-height: a 64-thread block owns 64 rows, thread
@@ -243,15 +252,27 @@ __global__ void __launch_bounds__(256) column_finish_kernel(gcext __restrict__ s
 // words keeps the banks distinct).  Measured on MI355X over a 2^21 x 256
 // LDE: 0.448 ms, against 0.452 (128 x 16), 0.455 (128 x 32), 0.474 (256 x
 // 16), 0.615 (128 x 8) and 1.0 ms and more with 64-column tiles.
-constexpr int RO_ROWS = 64, RO_COLS = 32;
-template <class F>
-__global__ void __launch_bounds__(RO_ROWS) reduce_rows_kernel(const RoMat* __restrict__ mats, int nmats,
+// A height of few rows leaves the chip idle while each wave walks all its
+// matrices: up to RO_SPLIT_ROWS rows, RO_SPLIT waves of a block share 64 rows and
+// take every RO_SPLIT-th matrix each, and their sums meet in LDS (2^11 rows of six
+// matrices, 1264 columns: 103 -> 53 us; 2^13 rows of two, 499 columns: 59 -> 37).
+constexpr int RO_ROWS = 64, RO_COLS = 32, RO_SPLIT = 4;
+constexpr uint32_t RO_SPLIT_ROWS = 1u << 15;
+// orders a wave's own LDS accesses (other waves use other words)
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <class F, int WAVES>
+__global__ void __launch_bounds__(RO_ROWS * WAVES) reduce_rows_kernel(const RoMat* __restrict__ mats, int nmats,
                                                               const Ext4* __restrict__ pts, int npts,
                                                               gcext __restrict__ alpha_pows, uint32_t shift,
                                                               int log_n, gcptr __restrict__ tw,
                                                               gext __restrict__ out) {
-    __shared__ uint32_t tile[RO_ROWS * (RO_COLS + 1)];
-    const uint32_t n = 1u << log_n, t = threadIdx.x;
+    __shared__ uint32_t tiles[WAVES][RO_ROWS * (RO_COLS + 1)];
+    const uint32_t n = 1u << log_n, t = threadIdx.x % RO_ROWS;
+    const uint32_t wave = WAVES == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / RO_ROWS));
+    uint32_t* const tile = tiles[wave];
     const uint32_t base = blockIdx.x * RO_ROWS, i = base + t;
     const bool live = i < n;
     const uint32_t ir = live ? i : n - 1;
@@ -270,7 +291,7 @@ __global__ void __launch_bounds__(RO_ROWS) reduce_rows_kernel(const RoMat* __res
     // loader coordinates: thread t loads column t % 16 of rows t / 16 + 16 k
     const uint32_t lc = t % RO_COLS, lr = t / RO_COLS;
     Ext4 ro{{0, 0, 0, 0}};
-    for (int k = 0; k < nmats; k++) {
+    for (int k = (int)wave; k < nmats; k += WAVES) {
         const RoMat* mk = mats + k;  // read in place: uniform, scalar loads
         const uint32_t width = mk->width;
         const uint64_t ld = mk->ld;
@@ -296,7 +317,7 @@ __global__ void __launch_bounds__(RO_ROWS) reduce_rows_kernel(const RoMat* __res
 #pragma unroll
             for (int kk = 0; kk < LPT; kk++)
                 tile[(lr + (RO_ROWS / RO_COLS) * kk) * (RO_COLS + 1) + lc] = col_live ? nxt[kk] : 0u;
-            __syncthreads();
+            wave_fence();
             if (c0 + RO_COLS < width) load_tile(c0 + RO_COLS);
             const uint32_t cn = width - c0 < (uint32_t)RO_COLS ? width - c0 : (uint32_t)RO_COLS;
             for (uint32_t c = 0; c < cn; c++) {
@@ -310,7 +331,7 @@ __global__ void __launch_bounds__(RO_ROWS) reduce_rows_kernel(const RoMat* __res
                     for (int q = 0; q < 4; q++) acc[q].fold();
                 }
             }
-            __syncthreads();
+            wave_fence();
         }
         const Ext4 r = Ext4{{acc[0].value(), acc[1].value(), acc[2].value(), acc[3].value()}};
         const int np = mk->npts;
@@ -328,6 +349,17 @@ __global__ void __launch_bounds__(RO_ROWS) reduce_rows_kernel(const RoMat* __res
             ro = eadd<F>(ro, emul<F>(term, iv));
         }
     }
+    if constexpr (WAVES > 1) {
+        wave_fence();
+        if (wave)
+#pragma unroll
+            for (int e = 0; e < 4; e++) tile[64 * e + t] = ro.c[e];
+        __syncthreads();
+        if (wave) return;
+        for (int u = 1; u < WAVES; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) ro.c[e] = fadd<F>(ro.c[e], tiles[u][64 * e + t]);
+    }
     if (live) out[i] = v4_of(ro);
 }
 
@@ -339,10 +371,14 @@ static hipError_t open_values_t(const uint32_t* m, uint64_t ld, uint32_t w, int 
                                 Ext4* partial, uint32_t nchunks, uint32_t chunk_rows, Ext4* sums, uint32_t nslices,
                                 Ext4* out, hipStream_t s) {
     const uint32_t h = 1u << log_h;
+    OvPoints zs{}, factors{};
+    for (int q = 0; q < npts; q++) {
+        zs.v[q] = z[q];
+        factors.v[q] = factor[q];
+    }
     if (!weights_ready)  // else computed for these points and this height by an earlier call
-        for (int q = 0; q < npts; q++)
-            bary_weights_kernel<F><<<blocks_for(h, 256), 256, 0, s>>>(z[q], to_monty<F>(F::GEN), log_h, (gcptr)tw,
-                                                                        (gext)(weights + (uint64_t)q * h));
+        bary_weights_kernel<F><<<dim3(blocks_for(h, 256), npts), 256, 0, s>>>(zs, to_monty<F>(F::GEN), log_h,
+                                                                              (gcptr)tw, (gext)weights);
     const uint64_t nt = (uint64_t)nchunks * w;
     if (open_values_vec4(m, ld, w, npts)) {
         const uint64_t nt4 = nt / 4;
@@ -362,13 +398,9 @@ static hipError_t open_values_t(const uint32_t* m, uint64_t ld, uint32_t w, int 
         default: column_dot_kernel<F, 4><<<blocks_for(nt, 256), 256, 0, s>>>((gcptr)m, ld, w, (gcext)weights, h,
                                                                            chunk_rows, nt, (gext)partial); break;
     }
-    for (int q = 0; q < npts; q++) {
-        Ext4* sq = sums + (uint64_t)q * nslices * w;
-        column_slice_sum_kernel<F><<<dim3(blocks_for(w, 64), nslices), 256, 0, s>>>(
-            (gcext)(partial + (uint64_t)q * nt), nchunks, w, nslices, (gext)sq);
-        column_finish_kernel<F><<<blocks_for(w, 256), 256, 0, s>>>((gcext)sq, nslices, w, factor[q],
-                                                                    (gext)(out + (uint64_t)q * w));
-    }
+    column_slice_sum_kernel<F><<<dim3(blocks_for(w, 64), nslices, npts), 256, 0, s>>>((gcext)partial, nchunks, w,
+                                                                                     nslices, (gext)sums);
+    column_finish_kernel<F><<<dim3(blocks_for(w, 256), npts), 256, 0, s>>>((gcext)sums, nslices, w, factors, (gext)out);
     return hipGetLastError();
 }
 
@@ -394,14 +426,25 @@ hipError_t launch_reduce_rows(int field, const RoMat* mats, int nmats, const Ext
                               const Ext4* alpha_pows, int log_n, const uint32_t* tw, Ext4* out,
                               hipStream_t stream) {
     const uint64_t n = 1ull << log_n;
-    if (field == FIELD_KOALABEAR)
-        reduce_rows_kernel<KoalaBear><<<blocks_for(n, RO_ROWS), RO_ROWS, 0, stream>>>(
-            mats, nmats, pts, npts, (gcext)alpha_pows, to_monty<KoalaBear>(KoalaBear::GEN), log_n,
-            (gcptr)tw, (gext)out);
-    else
-        reduce_rows_kernel<BabyBear><<<blocks_for(n, RO_ROWS), RO_ROWS, 0, stream>>>(
-            mats, nmats, pts, npts, (gcext)alpha_pows, to_monty<BabyBear>(BabyBear::GEN), log_n,
-            (gcptr)tw, (gext)out);
+    const bool split = n <= RO_SPLIT_ROWS && nmats > 1;
+    const unsigned g = blocks_for(n, RO_ROWS);
+    const uint32_t kb = to_monty<KoalaBear>(KoalaBear::GEN), bb = to_monty<BabyBear>(BabyBear::GEN);
+    const gcext ap = (gcext)alpha_pows;
+    if (field == FIELD_KOALABEAR) {
+        if (split)
+            reduce_rows_kernel<KoalaBear, RO_SPLIT><<<g, RO_ROWS * RO_SPLIT, 0, stream>>>(mats, nmats, pts, npts, ap, kb,
+                                                                                         log_n, (gcptr)tw, (gext)out);
+        else
+            reduce_rows_kernel<KoalaBear, 1><<<g, RO_ROWS, 0, stream>>>(mats, nmats, pts, npts, ap, kb, log_n,
+                                                                        (gcptr)tw, (gext)out);
+    } else {
+        if (split)
+            reduce_rows_kernel<BabyBear, RO_SPLIT><<<g, RO_ROWS * RO_SPLIT, 0, stream>>>(mats, nmats, pts, npts, ap, bb,
+                                                                                        log_n, (gcptr)tw, (gext)out);
+        else
+            reduce_rows_kernel<BabyBear, 1><<<g, RO_ROWS, 0, stream>>>(mats, nmats, pts, npts, ap, bb, log_n,
+                                                                       (gcptr)tw, (gext)out);
+    }
     return hipGetLastError();
 }
 
