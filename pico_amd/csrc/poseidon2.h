@@ -1,5 +1,6 @@
-// poseidon2.h -- Poseidon2 width-16 permutation over KoalaBear / BabyBear,
-// one permutation state per thread (16 x u32 in VGPRs), Montgomery form.
+// poseidon2.h -- Poseidon2 width-16 permutation over KoalaBear / BabyBear in
+// Montgomery form: its constants, and one state word by word (the host's form;
+// the device hashes on the matrix cores, poseidon2_mx.h).
 //
 // Structure (vm/src/primitives/mod.rs:305-346 with the p3 Poseidon2 layout;
 // restated in-tree at gnark/poseidon2/poseidon2_koalabear.go:71-196):
@@ -200,103 +201,6 @@ PG_HD void external_layer_wide(uint32_t (&s)[16]) {
     for (int i = 0; i < 4; i++) col[i] = (y[i] + y[4 + i]) + (y[8 + i] + y[12 + i]);
 #pragma unroll
     for (int i = 0; i < 16; i++) s[i] = reduce_wide<F>(y[i] + col[i & 3]);
-}
-
-// Sum of 16 reduced elements.  Pairs are added in 32 bits (< 2p), the rest in
-// 64 bits (< 16p < 2^35); then q = T >> 31 <= 15 and T - q p lies in
-// [0, 2^31 + 15 (2^31 - p)), below 2p for KoalaBear (one conditional
-// subtraction) and below 3p for BabyBear (two).
-template <class F>
-PG_HD uint32_t sum16(const uint32_t (&s)[16]) {
-    uint32_t l1[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) l1[i] = s[2 * i] + s[2 * i + 1];
-    uint64_t l2[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) l2[i] = (uint64_t)l1[2 * i] + l1[2 * i + 1];
-    const uint64_t t = (l2[0] + l2[1]) + (l2[2] + l2[3]);
-    const uint32_t q = (uint32_t)(t >> 31);
-    uint32_t r = (uint32_t)t - q * F::P;
-    r = freduce<F>(r);
-    if constexpr ((1ull << 31) + 15ull * ((1ull << 31) - F::P) >= 2ull * F::P) r = freduce<F>(r);
-    return r;
-}
-
-// S + c x mod p for a small constant c, x and S below p.  v = c x + S < (c+1) p
-// is one 64-bit multiply-add; with q = v >> 31 <= c, v - q p lies in
-// [0, 2^31 + c (2^31 - p)), which fits 32 bits for c < 2^31 / (2^31 - p)
-// (128 for KoalaBear, 16 for BabyBear) and needs one conditional subtraction
-// when it is below 2p, two otherwise.  The low word of v + q (2^32 - p) is
-// v - q p.
-template <class F, uint32_t C>
-PG_HD uint32_t fmadd_small(uint32_t x, uint32_t S) {
-    static_assert((uint64_t)C * ((1ull << 31) - F::P) < (1ull << 31), "bound needs c < 2^31 / (2^31 - p)");
-    const uint64_t v = (uint64_t)x * C + S;
-    const uint32_t q = (uint32_t)(v >> 31);
-    uint32_t r = (uint32_t)v + q * (0u - F::P);
-    r = freduce<F>(r);
-    if constexpr ((1ull << 31) + (uint64_t)C * ((1ull << 31) - F::P) > 2ull * F::P) r = freduce<F>(r);
-    return r;
-}
-
-// S - c x = S + c (p - x)
-template <class F, uint32_t C>
-PG_HD uint32_t fmsub_small(uint32_t x, uint32_t S) {
-    return fmadd_small<F, C>(F::P - x, S);
-}
-
-// x 2^-K mod p for x < p, where p = 1 (mod 2^K) (KoalaBear: K <= 24,
-// BabyBear: K <= 27).  With m = -x mod 2^K, x + m p = x + m = 0 (mod 2^K),
-// and x + m p < 2^K p, so (x + m p) / 2^K is the product, already below p:
-// a masked negation, one 64-bit multiply-add and a funnel shift.  The map is
-// linear, so it applies to Montgomery representatives as they are.
-template <class F, int K>
-PG_HD uint32_t fdiv_pow2(uint32_t x) {
-    static_assert(K >= 1 && K < 32 && ((F::P - 1u) & ((1u << K) - 1u)) == 0, "needs p = 1 mod 2^K");
-    const uint32_t m = (0u - x) & ((1u << K) - 1u);
-    const uint64_t v = (uint64_t)m * F::P + x;
-    return (uint32_t)(v >> K);
-}
-
-// s_i <- s_i * diag_i + S.  Both fields' diagonals (consts.rs:110-154) are
-//   -2, 1, 2, 1/2, 3, 4, -1/2, -3, -4, then +-2^-k entries and +-c
-// with c = 127 (KoalaBear: entries 11 = -127, 15 = 127) or c = 15 (BabyBear:
-// 12 = -15, 15 = 15).  The entries -2 .. 1/2 and -1/2 use additions and a
-// halving, the small integers a 64-bit multiply-add (fmadd_small), the
-// powers of two fdiv_pow2.  As integers the table holds p - (p-1)/2^k
-// (= +2^-k) and (p-1)/2^k (= -2^-k):
-//   KoalaBear  9: +2^-8  10: +2^-3  12: -2^-8  13: -2^-3  14: -2^-4
-//   BabyBear   9: +2^-8  10: +2^-2  11: +2^-3  13: -2^-8  14: -2^-4
-template <class F>
-PG_HD void internal_layer(uint32_t (&s)[16]) {
-    constexpr bool KB = F::P == KoalaBear::P;
-    constexpr uint32_t CBIG = KB ? 127u : 15u;
-    const uint32_t sum = sum16<F>(s);
-    s[0] = fsub<F>(sum, fadd<F>(s[0], s[0]));
-    s[1] = fadd<F>(sum, s[1]);
-    s[2] = fadd<F>(sum, fadd<F>(s[2], s[2]));
-    s[3] = fadd<F>(sum, fhalve<F>(s[3]));
-    s[4] = fmadd_small<F, 3>(s[4], sum);
-    s[5] = fmadd_small<F, 4>(s[5], sum);
-    s[6] = fsub<F>(sum, fhalve<F>(s[6]));
-    s[7] = fmsub_small<F, 3>(s[7], sum);
-    s[8] = fmsub_small<F, 4>(s[8], sum);
-    if constexpr (KB) {
-        s[11] = fmsub_small<F, CBIG>(s[11], sum);
-        s[9] = fadd<F>(fdiv_pow2<F, 8>(s[9]), sum);
-        s[10] = fadd<F>(fdiv_pow2<F, 3>(s[10]), sum);
-        s[12] = fsub<F>(sum, fdiv_pow2<F, 8>(s[12]));
-        s[13] = fsub<F>(sum, fdiv_pow2<F, 3>(s[13]));
-        s[14] = fsub<F>(sum, fdiv_pow2<F, 4>(s[14]));
-    } else {
-        s[12] = fmsub_small<F, CBIG>(s[12], sum);
-        s[9] = fadd<F>(fdiv_pow2<F, 8>(s[9]), sum);
-        s[10] = fadd<F>(fdiv_pow2<F, 2>(s[10]), sum);
-        s[11] = fadd<F>(fdiv_pow2<F, 3>(s[11]), sum);
-        s[13] = fsub<F>(sum, fdiv_pow2<F, 8>(s[13]));
-        s[14] = fsub<F>(sum, fdiv_pow2<F, 4>(s[14]));
-    }
-    s[15] = fmadd_small<F, CBIG>(s[15], sum);
 }
 
 // Internal layer with one Montgomery reduction per element, on lazy inputs
