@@ -1073,8 +1073,25 @@ using TreePtr = std::unique_ptr<pg_tree, void (*)(pg_tree*)>;
 // Allocates a tree's digest layers and device metadata (matrix descriptors
 // in original and height-sorted order, height shifts, column offsets, layer
 // offsets) without hashing anything.  The tree owns none of `mats` yet.
-static int tree_prepare(pg_ctx* ctx, hipStream_t s, int field, const std::vector<pg_buf*>& mats, TreePtr* out,
-                        std::vector<size_t>* order_out, MatRef** d_sorted_out) {
+struct PreparedTree {
+    TreePtr tree{nullptr, tree_discard};
+    std::vector<size_t> order;    // of the matrices, tallest first
+    MatRef* sorted = nullptr;     // device descriptors in that order
+    std::vector<uint8_t> meta;    // the device metadata, until it is uploaded
+};
+static int tree_upload(hipStream_t s, PreparedTree* p) {
+    HIP_TRY(hipMemcpyAsync(p->tree->meta, p->meta.data(), p->meta.size(), hipMemcpyHostToDevice, s));
+    return PG_OK;
+}
+// One matrix whose leaves are hashed from kernel arguments: nothing that builds
+// the tree reads its metadata, so the copy can follow the hashing.
+static bool tree_reads_no_meta(const std::vector<pg_buf*>& mats) {
+    const pg_buf* m = mats[0];
+    return mats.size() == 1 && m->cols > 0 &&
+           (m->rows <= SMALL_MAX_NODES || (m->cols % 8 == 0 && ((uintptr_t)m->ptr % 16) == 0));
+}
+static int tree_prepare(pg_ctx* ctx, hipStream_t s, int field, const std::vector<pg_buf*>& mats, PreparedTree* out,
+                        bool upload = true) {
     const size_t n = mats.size();
     if (n == 0) return fail(PG_E_INVALID, "no matrices to commit");
     size_t H = 0;
@@ -1134,7 +1151,6 @@ static int tree_prepare(pg_ctx* ctx, hipStream_t s, int field, const std::vector
     t->d_shift = (uint32_t*)(dm + off_shift);
     t->d_coloff = (uint32_t*)(dm + off_col);
     t->d_layer_off = (uint64_t*)(dm + off_layer);
-    HIP_TRY(hipMemcpyAsync(t->meta, hm.data(), meta_bytes, hipMemcpyHostToDevice, s));
 
     t->digest_bytes = (2 * H - 1) * 32;
     {
@@ -1142,10 +1158,11 @@ static int tree_prepare(pg_ctx* ctx, hipStream_t s, int field, const std::vector
         PG_TRY(ctx_alloc(ctx, t->digest_bytes, &p));
         t->digests = (uint32_t*)p;
     }
-    *order_out = std::move(order);
-    *d_sorted_out = d_sorted;
-    *out = std::move(t);
-    return PG_OK;
+    out->order = std::move(order);
+    out->sorted = d_sorted;
+    out->tree = std::move(t);
+    out->meta = std::move(hm);
+    return upload ? tree_upload(s, out) : PG_OK;
 }
 
 // `stage`, when given, is called with each run [g0, g1) of equal-height
@@ -1162,15 +1179,21 @@ static constexpr int STAGE_HASHED = 1;
 using StageFn = std::function<int(const std::vector<size_t>& order, size_t g0, size_t g1, uint32_t* leaves,
                                   const MatRef* sorted, const uint32_t** inj)>;
 
+// prepared: what tree_prepare gave for `mats` before the work that fills them
+// was queued, or null.  The metadata is uploaded by then (the copy stands ahead
+// of that work, not between it and the hashing) unless tree_reads_no_meta.
 static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const std::vector<pg_buf*>& mats,
                                  const std::vector<bool>& owned, uint32_t root[8], pg_tree** out,
-                                 const StageFn& stage = nullptr) {
+                                 const StageFn& stage = nullptr, PreparedTree* prepared = nullptr) {
     *out = nullptr;
     const size_t n = mats.size();
-    TreePtr t(nullptr, tree_discard);
-    std::vector<size_t> order;
-    MatRef* d_sorted = nullptr;
-    PG_TRY(tree_prepare(ctx, s, field, mats, &t, &order, &d_sorted));
+    PreparedTree own;
+    PreparedTree& pt = prepared ? *prepared : own;
+    const bool late_meta = !stage && n && mats[0] && tree_reads_no_meta(mats);
+    if (!prepared) PG_TRY(tree_prepare(ctx, s, field, mats, &pt, !late_meta));
+    pg_tree* const t = pt.tree.get();
+    const std::vector<size_t>& order = pt.order;
+    MatRef* const d_sorted = pt.sorted;
     SyncGuard guard(s);  // on an error below: wait for queued kernels before `t` frees
     const size_t H = t->H;
     // layer 0: every matrix of height H
@@ -1194,9 +1217,10 @@ static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const st
     };
     size_t len = H, off = 0, gi = g1;
     if (hashed) {
-    } else if (g1 - g0 == 1 && first->cols == 8 && H <= SMALL_MAX_NODES) {
+    } else if (g1 - g0 == 1 && first->cols > 0 && H <= SMALL_MAX_NODES) {
         const int c = layers_below(H, g1);
-        TIMED(kt, "leaf_hash_w8", s, launch_tree_layers(field, first->ptr, 8, 1, H, 1 + c, t->digests, s));
+        TIMED(kt, first->cols % 8 ? "leaf_hash" : "leaf_hash_w8", s,
+              launch_tree_layers(field, first->ptr, first->cols, (uint32_t)first->cols, H, 1 + c, t->digests, s));
         for (int k = 0; k < c; k++, len /= 2) off += len;
     } else if (g1 - g0 == 1 && first->cols % 8 == 0 && first->cols > 0 && ((uintptr_t)first->ptr % 16) == 0 &&
              H > SMALL_MAX_NODES)
@@ -1230,12 +1254,13 @@ static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const st
         len = nl;
         gi = gj;
     }
+    if (late_meta) PG_TRY(tree_upload(s, &pt));
     HIP_TRY(hipMemcpyAsync(t->root, t->digests + 8 * off, 32, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     guard.armed = false;
     memcpy(root, t->root, 32);
     t->owned = owned;
-    *out = t.release();
+    *out = pt.tree.release();
     return PG_OK;
 }
 
@@ -1623,6 +1648,13 @@ extern "C" int pg_pcs_commit(pg_ctx* ctx, int field, const pg_buf* const* evals,
             return rc;
         }
     }
+    PreparedTree prepared;
+    rc = tree_prepare(ctx, l.s, field, ldes, &prepared, !tree_reads_no_meta(ldes));
+    if (rc != PG_OK) {
+        (void)hipStreamSynchronize(l.s);
+        cleanup();
+        return rc;
+    }
     auto kt = make_timer(ctx);
     hipError_t e = hipSuccess;
     if (desc) e = hipMemcpyAsync(desc->ptr, st.bytes.data(), st.bytes.size(), hipMemcpyHostToDevice, l.s);
@@ -1650,7 +1682,7 @@ extern "C" int pg_pcs_commit(pg_ctx* ctx, int field, const pg_buf* const* evals,
         return fail(PG_E_DEVICE, "coset LDE launch failed: %s", hipGetErrorString(e));
     }
     // the tree consumes the LDEs (it owns them from here) and synchronises
-    rc = mmcs_commit_on_stream(ctx, l.s, field, ldes, std::vector<bool>(n, true), root, out);
+    rc = mmcs_commit_on_stream(ctx, l.s, field, ldes, std::vector<bool>(n, true), root, out, nullptr, &prepared);
     if (rc != PG_OK) {
         (void)hipStreamSynchronize(l.s);
         cleanup();
@@ -2324,17 +2356,15 @@ extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* eval
     for (size_t j = 0; j < njobs; j++) {
         pg_buf* o;
         PG_TRY(buf_new(ctx, N[j], W[j], &o));
-        TreePtr t(nullptr, tree_discard);
-        std::vector<size_t> order;
-        MatRef* ds;
-        const int rc = tree_prepare(ctx, l.s, field, {o}, &t, &order, &ds);
+        PreparedTree t;
+        const int rc = tree_prepare(ctx, l.s, field, {o}, &t);
         if (rc != PG_OK) {
             pg_buf_free(o);
             return rc;
         }
-        t->owned = {true};
-        digests[j] = t->digests;
-        b->trees[j] = t.release();
+        t.tree->owned = {true};
+        digests[j] = t.tree->digests;
+        b->trees[j] = t.tree.release();
     }
     std::shared_ptr<DevMem> scratch;
     if (tmp_words) {
@@ -3050,7 +3080,7 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
                                      l.s, &tc));
         } else {
             TIMED(kt, "leaf_hash_w8", l.s,
-                  launch_tree_layers(field, v, 8, 1, len, t->log_h + 1, t->digests, l.s, &tc));
+                  launch_tree_layers(field, v, 8, 8, len, t->log_h + 1, t->digests, l.s, &tc));
         }
         const pg_buf* const add = inputs[t->log_h];  // the vectors have 2^(log_h + 1) and 2^log_h elements
         uint32_t* const next = r + 1 < R ? f->trees[r + 1]->mats[0]->ptr : (uint32_t*)(dres + o_fin);

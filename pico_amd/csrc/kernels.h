@@ -56,8 +56,8 @@ hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size
 hipError_t launch_compress_digest(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
                                   const uint32_t* inj, hipStream_t stream);
 // Up to log2(n0) + 1 layers of a tree at once, n0 <= SMALL_MAX_NODES a power of
-// two: the first layer's nodes are C(in[2i], in[2i+1]), or with leaf8 the
-// hashes of n0 rows of 8 words (row pitch `stride`); the layers n0, n0/2, ...
+// two: the first layer's nodes are C(in[2i], in[2i+1]), or with leaf_width the
+// hashes of n0 rows of that many words (row pitch `stride`); the layers n0, n0/2, ...
 // are written one after the other at out.
 constexpr uint64_t SMALL_MAX_NODES = 1u << 15;
 // With `ch` the layers end at the root, which the duplex challenger at ch.state
@@ -68,8 +68,8 @@ struct TreeChallenge {
     uint32_t* beta;   // 4 words out
 };
 constexpr int CHALLENGER_WORDS = 35;
-hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
-                              uint32_t* out, hipStream_t stream, const TreeChallenge* ch = nullptr);
+hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0,
+                              int layers, uint32_t* out, hipStream_t stream, const TreeChallenge* ch = nullptr);
 // FRI query answers: for query q and round r, the sibling v_r[(idx[q] >> r) ^ 1]
 // (4 words at siblings[(q rounds + r) 4]) and the Merkle path of leaf
 // (idx[q] >> r) >> 1 (at paths[q path_words + path_off]).

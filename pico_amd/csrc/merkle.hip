@@ -495,9 +495,10 @@ MX16_KERNEL compress_small_kernel(const uint32_t* prev, uint32_t* next, uint64_t
 }
 
 // Several layers of a tree in one launch.  The first layer's n0 nodes are
-// C(in[2i], in[2i+1]) or, with LEAF8, the hashes of n0 rows of exactly 8 words
-// (one sponge chunk, st = (row, 0^8)); layers n0, n0/2, ... follow each other
-// at `out`, as a tree stores them.  A workgroup computes the `layers` layers
+// C(in[2i], in[2i+1]) or, with LEAF, the hashes of n0 rows of one matrix (a
+// launch and the wait for a table of matrix descriptors less: commit of 2^8 x
+// 13, 512 leaves, 78.7 -> 74.4 us); layers n0, n0/2, ... follow each other at `out`,
+// as a tree stores them.  A workgroup computes the `layers` layers
 // over its 2^log_per nodes of the first one: their children pass through LDS,
 // so a layer costs one permutation's latency instead of a launch (4.3 us and
 // the gap before it).
@@ -545,9 +546,38 @@ __device__ __forceinline__ void challenge_root(const Mx16<F>& P, const Mx16Lane&
     }
 }
 
-template <class F, bool LEAF8>
-MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0, int log_per, int layers, uint32_t* out,
-                               TreeChallenge ch) {
+// Digest (lane groups 0 and 1) of one row of one matrix; the whole wave calls it.
+template <class F>
+__device__ __forceinline__ u32x4 mx16_hash_row(const Mx16<F>& P, gcptr row, uint32_t width, uint32_t q) {
+    auto chunk = [&](uint32_t off) {  // words off + 4 (q & 1) ..; past the row: its last word
+        const uint32_t j = off + 4 * (q & 1u);
+        u32x4 v;
+        if (off + 8 <= width) {
+            v = *reinterpret_cast<const GLOBAL u32x4u*>(row + j);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) v[i] = row[j + i < width ? j + i : width - 1];
+        }
+        return v;
+    };
+    u32x4 next = chunk(0);
+    mx4 st = mx4{0};
+#pragma clang loop unroll(disable)
+    for (uint32_t off = 0; off < width; off += 8) {
+        const u32x4 cur = next;
+        const uint32_t left = width - off;
+        if (left > 8) next = chunk(off + 8);  // in flight
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (4 * q + i < (left < 8u ? left : 8u)) st[i] = (int)cur[i];
+        st = P.permute(Mx16<F>::op(st));
+    }
+    return mx16_words<F>(st);
+}
+
+template <class F, bool LEAF>
+MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint32_t width, uint64_t n0, int log_per, int layers,
+                               uint32_t* out, TreeChallenge ch) {
     __shared__ u32x4 buf[2][2 * TREE_MAX_PER];
     const Mx16<F> P;
     const Mx16Lane l;
@@ -559,13 +589,15 @@ MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint64_t n0,
         for (uint32_t g = wave; 16 * g < cnt; g += waves) {  // the wave's group of 16 nodes
             const uint32_t nd = 16 * g + l.n, nr = nd < cnt ? nd : cnt - 1;
             u32x4 w;
-            if (i > 0)
-                w = buf[(i - 1) & 1][4 * nr + l.q];
-            else if constexpr (LEAF8)
-                w = l.q < 2 ? u32x4(*reinterpret_cast<const GLOBAL u32x4u*>((gcptr)in + (base + nr) * stride + 4 * l.q)) : u32x4{0};
-            else
-                w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)in + 16 * (base + nr) + 4 * l.q);
-            w = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
+            if (LEAF && i == 0) {
+                w = mx16_hash_row<F>(P, (gcptr)in + (base + nr) * stride, width, l.q);
+            } else {
+                if (i > 0)
+                    w = buf[(i - 1) & 1][4 * nr + l.q];
+                else
+                    w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)in + 16 * (base + nr) + 4 * l.q);
+                w = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
+            }
             if (l.q < 2 && nd < cnt) {
                 buf[i & 1][2 * nd + l.q] = w;
                 *reinterpret_cast<GLOBAL u32x4*>(layer + 8 * (base + nd) + 4 * l.q) = w;
@@ -877,41 +909,43 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
     return hipGetLastError();
 }
 
-// Nodes (or 8-word rows) of the first layer, at most SMALL_MAX_NODES: 64 per
-// workgroup and seven layers a launch, one workgroup for all the rest once a
-// layer has at most 128 nodes.
+// Nodes (or rows) of the first layer, at most SMALL_MAX_NODES: 64 per workgroup
+// and seven layers a launch, one workgroup for all the rest once a layer has at
+// most 128 nodes (rows of several chunks stay at 64: a wave would hash its two
+// groups of rows one after the other).
 template <class F>
-static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, bool leaf8, uint64_t n0, int layers, uint32_t* out,
-                                hipStream_t s, const TreeChallenge* ch) {
+static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0, int layers,
+                                uint32_t* out, hipStream_t s, const TreeChallenge* ch) {
     while (layers > 0) {
         int log_per = 6;
-        if (n0 <= (uint64_t)TREE_MAX_PER)
+        if (n0 <= (uint64_t)(leaf_width > 8 ? 64 : TREE_MAX_PER))
             log_per = __builtin_ctzll(n0);
         const int now = std::min(layers, log_per + 1);
         const TreeChallenge c = ch && now == layers ? *ch : TreeChallenge{};
         const unsigned threads = std::min((unsigned)S_THREADS, std::max(64u, 4u << log_per));
-        if (leaf8)
-            tree_layers_kernel<F, true><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, stride, n0, log_per, now, out, c);
+        const unsigned g = (unsigned)(n0 >> log_per);
+        if (leaf_width)
+            tree_layers_kernel<F, true><<<g, threads, 0, s>>>(in, stride, leaf_width, n0, log_per, now, out, c);
         else
-            tree_layers_kernel<F, false><<<(unsigned)(n0 >> log_per), threads, 0, s>>>(in, 0, n0, log_per, now, out, c);
+            tree_layers_kernel<F, false><<<g, threads, 0, s>>>(in, 0, 0, n0, log_per, now, out, c);
         for (int i = 0; i < now; i++) {  // the last layer written feeds the next launch
             in = out;
             out += 8 * n0;
             n0 >>= 1;
         }
-        leaf8 = false;
+        leaf_width = 0;
         layers -= now;
     }
     return hipGetLastError();
 }
 
-hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, int leaf8, uint64_t n0, int layers,
-                              uint32_t* out, hipStream_t stream, const TreeChallenge* ch) {
+hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0,
+                              int layers, uint32_t* out, hipStream_t stream, const TreeChallenge* ch) {
     if (layers <= 0) return hipSuccess;
     if (ch && (n0 >> (layers - 1)) != 1) return hipErrorInvalidValue;  // sampled from the root
     if (n0 == 0 || n0 > SMALL_MAX_NODES || (n0 & (n0 - 1)) || (n0 >> (layers - 1)) == 0) return hipErrorInvalidValue;
-    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf8 != 0, n0, layers, out, stream, ch)
-                                    : tree_layers_t<BabyBear>(in, stride, leaf8 != 0, n0, layers, out, stream, ch);
+    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf_width, n0, layers, out, stream, ch)
+                                    : tree_layers_t<BabyBear>(in, stride, leaf_width, n0, layers, out, stream, ch);
 }
 
 hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size_t n_out,

@@ -85,3 +85,13 @@ def test_batched_leaf_groups(ctx, oracle, f):
         ot = oracle.MerkleTree(f, [oracle.coset_lde(f, a, b, g)])
         assert np.array_equal(roots[k], ot.root), k
     batch.free()
+
+
+@pytest.mark.parametrize("f", FIELDS)
+@pytest.mark.parametrize("width", [3, 13, 24, 61])
+def test_leaves_and_layers_in_one_launch(ctx, oracle, f, width):
+    # one tallest matrix of one or several chunks, then injected rows: leaves and
+    # the layers down to them share a launch (64 rows per workgroup, then more)
+    for log_h, log_inj in ((4, 2), (6, 0), (7, 3), (9, 1), (13, 5)):
+        check_tree(ctx, oracle, f, [oracle.random_matrix(f, log_h, 1 << log_h, width),
+                                    oracle.random_matrix(f, 99, 1 << log_inj, 10)])
