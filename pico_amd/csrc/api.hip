@@ -3063,6 +3063,7 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
     HIP_TRY(hipMemcpyAsync(R ? (void*)f->trees[0]->mats[0]->ptr : (void*)(dres + o_fin), inputs[L0]->ptr,
                            (size_t)16 << L0, hipMemcpyDeviceToDevice, l.s));
     auto kt = make_timer(ctx);
+    TreeFold fold{};  // of the vector round r commits to, where its tree's launch folds it
     for (int r = 0; r < R; r++) {
         const pg_tree* const t = f->trees[r];
         const uint32_t* const v = t->mats[0]->ptr;
@@ -3080,13 +3081,18 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
                                      l.s, &tc));
         } else {
             TIMED(kt, "leaf_hash_w8", l.s,
-                  launch_tree_layers(field, v, 8, 8, len, t->log_h + 1, t->digests, l.s, &tc));
+                  launch_tree_layers(field, v, 8, 8, len, t->log_h + 1, t->digests, l.s, &tc,
+                                     fold.out ? &fold : nullptr));
         }
+        fold.out = nullptr;
         const pg_buf* const add = inputs[t->log_h];  // the vectors have 2^(log_h + 1) and 2^log_h elements
         uint32_t* const next = r + 1 < R ? f->trees[r + 1]->mats[0]->ptr : (uint32_t*)(dres + o_fin);
-        TIMED(kt, "fri_fold", l.s,
-              launch_fri_fold(field, v, t->H, beta, nullptr, (const uint32_t*)tws[r]->ptr, add ? add->ptr : nullptr,
-                              next, l.s));
+        if (r + 1 < R && f->trees[r + 1]->H <= SMALL_MAX_NODES)
+            fold = TreeFold{v, beta, (const uint32_t*)tws[r]->ptr, add ? add->ptr : nullptr, next};
+        else
+            TIMED(kt, "fri_fold", l.s,
+                  launch_fri_fold(field, v, t->H, beta, nullptr, (const uint32_t*)tws[r]->ptr, add ? add->ptr : nullptr,
+                                  next, l.s));
     }
     std::vector<uint8_t> host(res_bytes);
     HIP_TRY(hipMemcpyAsync(host.data(), dres, res_bytes, hipMemcpyDeviceToHost, l.s));

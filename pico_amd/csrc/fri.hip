@@ -8,6 +8,7 @@
 //   out[i] = (v[2i] + v[2i+1]) / 2 + beta/2 * (v[2i] - v[2i+1]) * x_i^{-1}.
 #include "kernels.h"
 #include "field.h"
+#include "fri_fold.h"
 
 namespace pg {
 
@@ -21,25 +22,10 @@ __global__ void __launch_bounds__(256) fri_fold_kernel(const uint32_t* __restric
                                                        uint32_t* __restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_out) return;
-    const uint4 a4 = reinterpret_cast<const uint4*>(v)[2 * i];
-    const uint4 b4 = reinterpret_cast<const uint4*>(v)[2 * i + 1];
-    const Ext4 a = {{a4.x, a4.y, a4.z, a4.w}}, b = {{b4.x, b4.y, b4.z, b4.w}};
-    const uint32_t mask = (uint32_t)(2 * n_out - 1);
-    const uint32_t r = log_n_out == 0 ? 0u : (__brev((uint32_t)i) >> (32 - log_n_out));
-    const uint32_t x_inv = tw[(0u - r) & mask];  // w_n^{-rev(i)}
-    Ext4 s = eadd<F>(a, b);
+    uint32_t bt[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) s.c[k] = fhalve<F>(s.c[k]);
-    const Ext4 d = escale<F>(esub<F>(a, b), x_inv);
-    Ext4 half_beta;
-#pragma unroll
-    for (int k = 0; k < 4; k++) half_beta.c[k] = fhalve<F>(beta ? beta[k] : host_beta.c[k]);
-    Ext4 o = eadd<F>(s, emul<F>(d, half_beta));
-    if (add) {
-        const uint4 w = reinterpret_cast<const uint4*>(add)[i];
-        o = eadd<F>(o, Ext4{{w.x, w.y, w.z, w.w}});
-    }
-    reinterpret_cast<uint4*>(out)[i] = make_uint4(o.c[0], o.c[1], o.c[2], o.c[3]);
+    for (int k = 0; k < 4; k++) bt[k] = beta ? beta[k] : host_beta.c[k];
+    reinterpret_cast<GLOBAL u32x4*>((gptr)out)[i] = fri_fold_at<F>((gcptr)v, i, log_n_out, bt, (gcptr)tw, (gcptr)add);
 }
 
 template <class F>

@@ -67,9 +67,20 @@ struct TreeChallenge {
     uint32_t* root;   // 8 words out
     uint32_t* beta;   // 4 words out
 };
+// With `fold` the first layer's nodes are the hashes of the pairs (v[2i], v[2i+1])
+// of a folded FRI vector (2 n0 ext4 elements), computed here from the vector
+// before it and written to `out`.
+struct TreeFold {
+    const uint32_t* prev;  // 4 n0 ext4 elements
+    const uint32_t* beta;  // 4 words
+    const uint32_t* tw;    // w^e, e < 4 n0
+    const uint32_t* add;   // 2 n0 ext4 elements added, or null
+    uint32_t* out;
+};
 constexpr int CHALLENGER_WORDS = 35;
 hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0,
-                              int layers, uint32_t* out, hipStream_t stream, const TreeChallenge* ch = nullptr);
+                              int layers, uint32_t* out, hipStream_t stream, const TreeChallenge* ch = nullptr,
+                              const TreeFold* fold = nullptr);
 // FRI query answers: for query q and round r, the sibling v_r[(idx[q] >> r) ^ 1]
 // (4 words at siblings[(q rounds + r) 4]) and the Merkle path of leaf
 // (idx[q] >> r) >> 1 (at paths[q path_words + path_off]).

@@ -17,6 +17,7 @@
 #include "kernels.h"
 #include "poseidon2.h"
 #include "poseidon2_mx.h"
+#include "fri_fold.h"
 
 namespace pg {
 
@@ -495,9 +496,11 @@ MX16_KERNEL compress_small_kernel(const uint32_t* prev, uint32_t* next, uint64_t
 }
 
 // Several layers of a tree in one launch.  The first layer's n0 nodes are
-// C(in[2i], in[2i+1]) or, with LEAF, the hashes of n0 rows of one matrix (a
+// C(in[2i], in[2i+1]) or, with TREE_ROWS, the hashes of n0 rows of one matrix (a
 // launch and the wait for a table of matrix descriptors less: commit of 2^8 x
-// 13, 512 leaves, 78.7 -> 74.4 us); layers n0, n0/2, ... follow each other at `out`,
+// 13, 512 leaves, 78.7 -> 74.4 us) or, with TREE_FOLDED, of the pairs of a FRI
+// vector folded here (a launch of 4.5 us less a round; commit phase of 2^18 with
+// an injected 2^15: 694 -> 651 us); layers n0, n0/2, ... follow each other at `out`,
 // as a tree stores them.  A workgroup computes the `layers` layers
 // over its 2^log_per nodes of the first one: their children pass through LDS,
 // so a layer costs one permutation's latency instead of a launch (4.3 us and
@@ -575,10 +578,25 @@ __device__ __forceinline__ u32x4 mx16_hash_row(const Mx16<F>& P, gcptr row, uint
     return mx16_words<F>(st);
 }
 
-template <class F, bool LEAF>
+enum { TREE_NODES, TREE_ROWS, TREE_FOLDED };  // what the first layer hashes
+template <class F, int FIRST>
 MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint32_t width, uint64_t n0, int log_per, int layers,
-                               uint32_t* out, TreeChallenge ch) {
+                               uint32_t* out, TreeChallenge ch, TreeFold fold) {
     __shared__ u32x4 buf[2][2 * TREE_MAX_PER];
+    if constexpr (FIRST == TREE_FOLDED) {  // before the hash tables fill the registers
+        uint32_t beta[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) beta[k] = ((gcptr)fold.beta)[k];
+        const int log_n_out = 64 - __builtin_clzll(n0);  // of 2 n0 elements
+        const uint32_t cnt = 2u << log_per;
+        for (uint32_t t = threadIdx.x; t < cnt; t += blockDim.x) {
+            const uint64_t i = (uint64_t)blockIdx.x * cnt + t;
+            const u32x4 o = fri_fold_at<F>((gcptr)fold.prev, i, log_n_out, beta, (gcptr)fold.tw, (gcptr)fold.add);
+            reinterpret_cast<GLOBAL u32x4*>((gptr)fold.out)[i] = o;
+            buf[1][t] = o;
+        }
+        __syncthreads();
+    }
     const Mx16<F> P;
     const Mx16Lane l;
     const uint32_t wave = mx16_wave(), waves = blockDim.x >> 6;
@@ -589,11 +607,13 @@ MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint32_t wid
         for (uint32_t g = wave; 16 * g < cnt; g += waves) {  // the wave's group of 16 nodes
             const uint32_t nd = 16 * g + l.n, nr = nd < cnt ? nd : cnt - 1;
             u32x4 w;
-            if (LEAF && i == 0) {
+            if (FIRST == TREE_ROWS && i == 0) {
                 w = mx16_hash_row<F>(P, (gcptr)in + (base + nr) * stride, width, l.q);
             } else {
                 if (i > 0)
                     w = buf[(i - 1) & 1][4 * nr + l.q];
+                else if constexpr (FIRST == TREE_FOLDED)
+                    w = l.q < 2 ? buf[1][2 * nr + l.q] : u32x4{0};
                 else
                     w = *reinterpret_cast<const GLOBAL u32x4*>((gcptr)in + 16 * (base + nr) + 4 * l.q);
                 w = mx16_words<F>(P.permute(Mx16<F>::op(__builtin_bit_cast(mx4, w))));
@@ -915,7 +935,7 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
 // groups of rows one after the other).
 template <class F>
 static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0, int layers,
-                                uint32_t* out, hipStream_t s, const TreeChallenge* ch) {
+                                uint32_t* out, hipStream_t s, const TreeChallenge* ch, const TreeFold* fold) {
     while (layers > 0) {
         int log_per = 6;
         if (n0 <= (uint64_t)(leaf_width > 8 ? 64 : TREE_MAX_PER))
@@ -924,28 +944,32 @@ static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, uint32_t le
         const TreeChallenge c = ch && now == layers ? *ch : TreeChallenge{};
         const unsigned threads = std::min((unsigned)S_THREADS, std::max(64u, 4u << log_per));
         const unsigned g = (unsigned)(n0 >> log_per);
-        if (leaf_width)
-            tree_layers_kernel<F, true><<<g, threads, 0, s>>>(in, stride, leaf_width, n0, log_per, now, out, c);
+        if (fold)
+            tree_layers_kernel<F, TREE_FOLDED><<<g, threads, 0, s>>>(nullptr, 0, 0, n0, log_per, now, out, c, *fold);
+        else if (leaf_width)
+            tree_layers_kernel<F, TREE_ROWS><<<g, threads, 0, s>>>(in, stride, leaf_width, n0, log_per, now, out, c, {});
         else
-            tree_layers_kernel<F, false><<<g, threads, 0, s>>>(in, 0, 0, n0, log_per, now, out, c);
+            tree_layers_kernel<F, TREE_NODES><<<g, threads, 0, s>>>(in, 0, 0, n0, log_per, now, out, c, {});
         for (int i = 0; i < now; i++) {  // the last layer written feeds the next launch
             in = out;
             out += 8 * n0;
             n0 >>= 1;
         }
         leaf_width = 0;
+        fold = nullptr;
         layers -= now;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_tree_layers(int field, const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0,
-                              int layers, uint32_t* out, hipStream_t stream, const TreeChallenge* ch) {
+                              int layers, uint32_t* out, hipStream_t stream, const TreeChallenge* ch,
+                              const TreeFold* fold) {
     if (layers <= 0) return hipSuccess;
     if (ch && (n0 >> (layers - 1)) != 1) return hipErrorInvalidValue;  // sampled from the root
     if (n0 == 0 || n0 > SMALL_MAX_NODES || (n0 & (n0 - 1)) || (n0 >> (layers - 1)) == 0) return hipErrorInvalidValue;
-    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf_width, n0, layers, out, stream, ch)
-                                    : tree_layers_t<BabyBear>(in, stride, leaf_width, n0, layers, out, stream, ch);
+    return field == FIELD_KOALABEAR ? tree_layers_t<KoalaBear>(in, stride, leaf_width, n0, layers, out, stream, ch, fold)
+                                    : tree_layers_t<BabyBear>(in, stride, leaf_width, n0, layers, out, stream, ch, fold);
 }
 
 hipError_t launch_compress(int field, const uint32_t* prev, uint32_t* next, size_t n_out,
