@@ -568,21 +568,17 @@ __device__ __forceinline__ void mx_swap(int& a, int& b) {
     b = (int)r[1];
 }
 
-// a k + t for a constant k: one v_mad_i64_i32 (the compiler makes products by
-// constants near powers of two shifts and 64-bit subtractions)
+// a k + t for a constant k: one v_mad_i64_i32.  The constant passes through an
+// empty asm, which hides its value: the compiler makes products by constants
+// near powers of two shifts and 64-bit subtractions.  The instruction itself is
+// left to the compiler, because between a matrix instruction and a vector
+// instruction that touches its registers the program has to wait (the hardware
+// does not), and the compiler places those waits only for instructions it knows.
 template <int32_t K>
 __device__ __forceinline__ int64_t mx_mad(int a, int64_t t) {
-    int64_t r, carry;
-    asm("v_mad_i64_i32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(carry) : "v"(a), "s"(K), "v"(t));
-    (void)carry;
-    return r;
-}
-template <int32_t K>
-__device__ __forceinline__ int64_t mx_mul(int a) {
-    int64_t r, carry;
-    asm("v_mad_i64_i32 %0, %1, %2, %3, 0" : "=v"(r), "=s"(carry) : "v"(a), "s"(K));
-    (void)carry;
-    return r;
+    int k = K;
+    asm("" : "+s"(k));
+    return (int64_t)a * k + t;
 }
 
 // The four S-boxes of a block of partial rounds: u the forms over everything
@@ -595,7 +591,7 @@ __device__ __forceinline__ void mx_block(int (&u)[4], int rounds) {
         if (o >= rounds) continue;
         int v = u[o];
         if (o > 0) {
-            int64_t w = mx_mad<R::C1>(u[o - 1], mx_mul<R::ONE>(v));
+            int64_t w = mx_mad<R::C1>(u[o - 1], mx_mad<R::ONE>(v, 0));
             if (o > 1) w = mx_mad<R::C2>(u[o - 2], w);
             if (o > 2) w = mx_mad<R::C3>(u[o - 3], w);
             v = mx_redc<F>(w);
