@@ -34,8 +34,7 @@ def to_monty(field, a):
 
 def from_monty(field, a):
     p = PRIMES[field]
-    a = np.asarray(a)
-    if a.dtype == np.uint32:
+    if isinstance(a, (np.ndarray, np.generic)) and a.dtype == np.uint32:
         # (a + m p) / 2^32 with m = -a / p mod 2^32, which is at most p: no 64-bit
         # division, in blocks whose temporaries stay in cache.  230 thousand words
         # (an open's) take a quarter of the division's time.
@@ -54,9 +53,9 @@ def from_monty(field, a):
             r[:] = tt
             np.subtract(r, np.uint32(p), out=mm)
             np.minimum(r, mm, out=r)
-        return out.reshape(a.shape)
+        return out.reshape(a.shape)[()]  # a scalar for a scalar
     rinv = np.uint64(pow(2 ** 32, p - 2, p))
-    return ((a.astype(np.uint64) * rinv) % np.uint64(p)).astype(np.uint32)
+    return ((np.asarray(a, dtype=np.uint64) * rinv) % np.uint64(p)).astype(np.uint32)
 
 
 def device_synchronize(device=0):
