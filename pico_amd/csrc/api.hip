@@ -3963,16 +3963,43 @@ static bool air_is_leaf(const pg_air_node& n) {
 static std::unique_ptr<QResident> air_resident(const std::vector<pg_air_node>& nodes,
                                                const std::vector<LAssert>& las) {
     if (las.empty()) return nullptr;
-    // emission order of asserts [j0, j1): inner nodes operands first, then the assert
+    const size_t nn = nodes.size();
+    // inner operands of each inner node (NO_NODE: a leaf or none)
+    constexpr uint32_t NO_NODE = ~0u;
+    std::vector<std::array<uint32_t, 2>> kids(nn, {NO_NODE, NO_NODE});
+    for (size_t k = 0; k < nn; k++) {
+        const pg_air_node& nd = nodes[k];
+        if (air_is_leaf(nd)) continue;
+        if (!air_is_leaf(nodes[nd.a])) kids[k][0] = nd.a;
+        if (nd.kind != PG_AIR_NEG && !air_is_leaf(nodes[nd.b])) kids[k][1] = nd.b;
+    }
+    std::vector<uint32_t> stamp(nn, 0);
+    uint32_t now = 0;
+    std::vector<uint32_t> stack;
+    // instructions that assert j adds to a slice (the nodes not yet stamped, and the assert)
+    auto cost = [&](size_t j) {
+        uint32_t added = 1;
+        auto visit = [&](uint32_t k) {
+            if (k == NO_NODE || stamp[k] == now) return;
+            stamp[k] = now;
+            added++;
+            stack.push_back(k);
+        };
+        if (!air_is_leaf(nodes[las[j].node])) visit(las[j].node);
+        while (!stack.empty()) {
+            const uint32_t k = stack.back();
+            stack.pop_back();
+            visit(kids[k][0]);
+            visit(kids[k][1]);
+        }
+        return added;
+    };
+    // the same in emission order: inner nodes operands first, then the assert
     struct Item {
         bool is_assert;
         uint32_t node;
     };
-    std::vector<uint32_t> stamp(nodes.size(), 0);
-    uint32_t now = 0;
-    std::vector<uint32_t> stack;
-    auto emit = [&](size_t j, std::vector<Item>* order) {  // the nodes assert j adds under the current stamp
-        uint32_t added = 0;
+    auto emit = [&](size_t j, std::vector<Item>& order) {
         if (!air_is_leaf(nodes[las[j].node])) stack.push_back(las[j].node);
         while (!stack.empty()) {
             const uint32_t k = stack.back();
@@ -3980,30 +4007,129 @@ static std::unique_ptr<QResident> air_resident(const std::vector<pg_air_node>& n
                 stack.pop_back();
                 continue;
             }
-            const pg_air_node& nd = nodes[k];
-            const bool binary = nd.kind != PG_AIR_NEG;
-            const bool wa = !air_is_leaf(nodes[nd.a]) && stamp[nd.a] != now;
-            const bool wb = binary && !air_is_leaf(nodes[nd.b]) && stamp[nd.b] != now;
+            const bool wa = kids[k][0] != NO_NODE && stamp[kids[k][0]] != now;
+            const bool wb = kids[k][1] != NO_NODE && stamp[kids[k][1]] != now;
             if (wa || wb) {
-                if (wb) stack.push_back(nd.b);
-                if (wa) stack.push_back(nd.a);
+                if (wb) stack.push_back(kids[k][1]);
+                if (wa) stack.push_back(kids[k][0]);
                 continue;
             }
             stamp[k] = now;
             stack.pop_back();
-            added++;
-            if (order) order->push_back(Item{false, k});
+            order.push_back(Item{false, k});
         }
-        if (order) order->push_back(Item{true, las[j].node});
-        return added + 1;
+        order.push_back(Item{true, las[j].node});
     };
+
+    // What every cut shares: the columns read, as runs and pieces, and the words
+    // of columns, constants and selectors.  Programs that do not fit end here.
+    QResident base_plan;
+    std::vector<uint32_t> word_of(nn, 0);  // of a leaf
+    uint32_t base_words = 0, zero = 0;
+    {
+        std::array<std::vector<std::pair<uint32_t, uint32_t>>, 6> cols;  // column, node
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> consts;
+        std::vector<std::pair<uint32_t, uint32_t>> sels;  // selector, node
+        std::vector<uint32_t> const_nodes;
+        auto leaf = [&](uint32_t k) {
+            if (stamp[k] == now) return;
+            stamp[k] = now;
+            const pg_air_node& nd = nodes[k];
+            switch (nd.kind) {
+                case PG_AIR_MAIN: cols[nd.a].push_back({nd.b, k}); break;
+                case PG_AIR_PREPROCESSED: cols[2 + nd.a].push_back({nd.b, k}); break;
+                case LK_PERM: cols[4 + nd.a].push_back({nd.b, k}); break;
+                case PG_AIR_IS_FIRST_ROW: sels.push_back({0, k}); break;
+                case PG_AIR_IS_LAST_ROW: sels.push_back({1, k}); break;
+                case PG_AIR_IS_TRANSITION: sels.push_back({2, k}); break;
+                default:
+                    consts.emplace(std::make_pair(nd.kind, nd.kind == PG_AIR_CONSTANT ? nd.a : nd.b), 0);
+                    const_nodes.push_back(k);
+                    break;
+            }
+        };
+        const auto zero_key = std::make_pair((uint32_t)PG_AIR_CONSTANT, 0u);  // negations, asserted leaves
+        consts.emplace(zero_key, 0);
+        now++;
+        for (const LAssert& la : las) {
+            if (air_is_leaf(nodes[la.node])) {
+                leaf(la.node);
+                continue;
+            }
+            if (stamp[la.node] == now) continue;
+            stamp[la.node] = now;
+            stack.push_back(la.node);
+            while (!stack.empty()) {
+                const pg_air_node& nd = nodes[stack.back()];
+                stack.pop_back();
+                for (int o = 0; o < (nd.kind == PG_AIR_NEG ? 1 : 2); o++) {
+                    const uint32_t k = o ? nd.b : nd.a;
+                    if (air_is_leaf(nodes[k])) {
+                        leaf(k);
+                    } else if (stamp[k] != now) {
+                        stamp[k] = now;
+                        stack.push_back(k);
+                    }
+                }
+            }
+        }
+        for (auto& c : cols) std::sort(c.begin(), c.end());
+        for (uint32_t gap = 8;; gap *= 4) {
+            base_plan.runs.clear();
+            uint32_t slot = 0;
+            for (uint32_t g = 0; g < 6; g++) {
+                uint32_t last = 0;
+                bool open = false;
+                for (const auto& [c, node] : cols[g]) {
+                    if (!open || c - last > gap) {
+                        base_plan.runs.push_back(QResident::Run{g / 2, g % 2, c, 0, slot});
+                        open = true;
+                    }
+                    QResident::Run& r = base_plan.runs.back();
+                    slot += c + 1 - r.col0 - r.count;
+                    r.count = c + 1 - r.col0;
+                    last = c;
+                    word_of[node] = (r.slot0 + c - r.col0) * QRS_COL;
+                }
+            }
+            if (slot > QR_MAX_WORDS / QRS_COL) return nullptr;
+            base_plan.const0 = slot * QRS_COL;
+            base_plan.pieces.clear();
+            for (const auto& r : base_plan.runs)
+                for (uint32_t c = 0; c < r.count; c += 64)
+                    base_plan.pieces.push_back(
+                        QrPiece{r.col0 + c, r.slot0 + c, std::min(64u, r.count - c) | r.src << 8 | r.next << 10, 0});
+            if (base_plan.pieces.size() <= (size_t)QR_MAX_PIECES) break;
+            if (gap > (1u << 24)) return nullptr;
+        }
+        if (base_plan.const0 + 64ull * consts.size() > QR_MAX_WORDS) return nullptr;
+        uint32_t next = base_plan.const0;
+        for (auto& c : consts) {
+            c.second = next;
+            next += 64;
+            base_plan.consts.push_back(c.first);
+        }
+        zero = consts[zero_key];
+        for (uint32_t k : const_nodes) {
+            const pg_air_node& nd = nodes[k];
+            word_of[k] = consts[std::make_pair(nd.kind, nd.kind == PG_AIR_CONSTANT ? nd.a : nd.b)];
+        }
+        std::sort(sels.begin(), sels.end());
+        for (const auto& [s, node] : sels) {
+            word_of[node] = base_plan.sel_word[s] = next;
+            next += 64;
+        }
+        base_words = next;
+        if (base_words + 4 * 256 > QR_MAX_WORDS) return nullptr;  // four slices or more, 256 words each or more
+    }
+
     // greedy cut at `target` instructions; returns the slices' first asserts
-    uint64_t total = 0;
-    auto cut = [&](uint64_t target, size_t most) {  // gives up past `most` slices
+    uint64_t total = 0, largest = 0;  // largest: instructions of one original assert at the start of a slice
+    auto cut = [&](uint64_t target, size_t most, uint64_t budget) {  // gives up past `most` slices or `budget` instructions
         std::vector<size_t> first;
         uint64_t cur = 0;
-        total = 0;
-        for (size_t j = 0; j < las.size() && first.size() <= most;) {
+        total = largest = 0;
+        for (size_t j = 0; j < las.size() && first.size() <= most && total <= budget;) {
             size_t j1 = j + 1;
             while (j1 < las.size() && las[j1].orig == las[j].orig) j1++;
             if (first.empty()) {
@@ -4011,126 +4137,59 @@ static std::unique_ptr<QResident> air_resident(const std::vector<pg_air_node>& n
                 now++;
             }
             uint64_t c = 0;
-            for (size_t i = j; i < j1; i++) c += emit(i, nullptr);
+            for (size_t i = j; i < j1; i++) c += cost(i);
             if (cur && cur + c > target) {  // starts a slice of its own
                 first.push_back(j);
                 now++;
                 cur = c = 0;
-                for (size_t i = j; i < j1; i++) c += emit(i, nullptr);
-                total += c;
-                cur = c;
-            } else {
-                cur += c;
-                total += c;
+                for (size_t i = j; i < j1; i++) c += cost(i);
             }
+            if (cur == 0) largest = std::max(largest, c);
+            total += c;
+            cur += c;
             j = j1;
         }
         return first;
     };
-    cut(UINT64_MAX, 1);
+    cut(UINT64_MAX, 1, UINT64_MAX);
     const uint64_t alone = total;
+    cut(0, SIZE_MAX, 2 * alone);  // every original assert by itself
+    const uint64_t biggest = largest;
     for (uint32_t W = QR_MAX_WAVES; W >= 4; W /= 2) {
         if (W > 4 && alone < (uint64_t)W * QR_MIN_SLICE) continue;
-        uint64_t lo = 1, hi = alone;  // the smallest target that gives at most W slices
+        auto fits_waves = [&](uint64_t target) { return cut(target, W, UINT64_MAX).size() <= W; };
+        // The smallest target that gives at most W slices: below alone / W only where
+        // single asserts exceed it; else a slice ends within `biggest` of the target,
+        // so without shared nodes alone / W + biggest is enough, and with the quarter
+        // more work that is allowed alone / 4 W above that.  A program that needs a
+        // higher one shares too much.
+        uint64_t lo = (alone + W - 1) / W, hi = lo + biggest;
+        if (lo > 1 && fits_waves(lo - 1)) {
+            hi = lo - 1;
+            lo = 1;
+        } else if (!fits_waves(hi)) {
+            lo = hi + 1;
+            hi = lo + alone / (4 * W);
+            if (!fits_waves(hi)) continue;
+        }
         while (lo < hi) {
             const uint64_t mid = (lo + hi) / 2;
-            if (cut(mid, W).size() <= W)
+            if (fits_waves(mid))
                 hi = mid;
             else
                 lo = mid + 1;
         }
-        std::vector<size_t> first = cut(lo, W);
+        std::vector<size_t> first = cut(lo, W, UINT64_MAX);
         if (first.size() > W || total * 4 > alone * 5) continue;
         first.push_back(las.size());
         const size_t S = first.size() - 1;
-        auto plan = std::make_unique<QResident>();
-        // columns read, as runs
-        std::array<std::set<uint32_t>, 6> cols;
-        std::map<std::pair<uint32_t, uint32_t>, uint32_t> consts;
-        uint32_t sel = 0;
-        auto leaf = [&](uint32_t k) {
-            const pg_air_node& nd = nodes[k];
-            switch (nd.kind) {
-                case PG_AIR_MAIN: cols[nd.a].insert(nd.b); break;
-                case PG_AIR_PREPROCESSED: cols[2 + nd.a].insert(nd.b); break;
-                case LK_PERM: cols[4 + nd.a].insert(nd.b); break;
-                case PG_AIR_IS_FIRST_ROW: sel |= 1; break;
-                case PG_AIR_IS_LAST_ROW: sel |= 2; break;
-                case PG_AIR_IS_TRANSITION: sel |= 4; break;
-                default: consts.emplace(std::make_pair(nd.kind, nd.kind == PG_AIR_CONSTANT ? nd.a : nd.b), 0); break;
-            }
-        };
-        consts.emplace(std::make_pair((uint32_t)PG_AIR_CONSTANT, 0u), 0);  // zero: negations, asserted leaves
+        auto plan = std::make_unique<QResident>(base_plan);
         std::vector<std::vector<Item>> order(S);
         for (size_t k = 0; k < S; k++) {
             now++;
-            for (size_t j = first[k]; j < first[k + 1]; j++) emit(j, &order[k]);
-            for (const Item& it : order[k]) {
-                const pg_air_node& nd = nodes[it.node];
-                if (air_is_leaf(nd)) {
-                    leaf(it.node);
-                } else if (!it.is_assert) {
-                    if (air_is_leaf(nodes[nd.a])) leaf(nd.a);
-                    if (nd.kind != PG_AIR_NEG && air_is_leaf(nodes[nd.b])) leaf(nd.b);
-                }
-            }
+            for (size_t j = first[k]; j < first[k + 1]; j++) emit(j, order[k]);
         }
-        for (uint32_t gap = 8;; gap *= 4) {
-            plan->runs.clear();
-            uint32_t slot = 0;
-            for (uint32_t g = 0; g < 6; g++) {
-                uint32_t last = 0;
-                bool open = false;
-                for (uint32_t c : cols[g]) {
-                    if (!open || c - last > gap) {
-                        plan->runs.push_back(QResident::Run{g / 2, g % 2, c, 0, slot});
-                        open = true;
-                    }
-                    QResident::Run& r = plan->runs.back();
-                    slot += c + 1 - r.col0 - r.count;
-                    r.count = c + 1 - r.col0;
-                    last = c;
-                }
-            }
-            plan->const0 = slot * QRS_COL;
-            plan->pieces.clear();
-            for (const auto& r : plan->runs)
-                for (uint32_t c = 0; c < r.count; c += 64)
-                    plan->pieces.push_back(
-                        QrPiece{r.col0 + c, r.slot0 + c, std::min(64u, r.count - c) | r.src << 8 | r.next << 10, 0});
-            if (plan->pieces.size() <= (size_t)QR_MAX_PIECES) break;
-            if (gap > (1u << 24)) return nullptr;
-        }
-        if (plan->const0 > QR_MAX_WORDS) return nullptr;
-        uint32_t next = plan->const0;
-        for (auto& c : consts) {
-            c.second = next;
-            next += 64;
-            plan->consts.push_back(c.first);
-        }
-        for (int k = 0; k < 3; k++)
-            if (sel >> k & 1) {
-                plan->sel_word[k] = next;
-                next += 64;
-            }
-        const uint32_t zero = consts[std::make_pair((uint32_t)PG_AIR_CONSTANT, 0u)];
-        auto leaf_word = [&](uint32_t k) -> uint32_t {
-            const pg_air_node& nd = nodes[k];
-            uint32_t src;
-            switch (nd.kind) {
-                case PG_AIR_MAIN: src = 0; break;
-                case PG_AIR_PREPROCESSED: src = 1; break;
-                case LK_PERM: src = 2; break;
-                case PG_AIR_IS_FIRST_ROW: return plan->sel_word[0];
-                case PG_AIR_IS_LAST_ROW: return plan->sel_word[1];
-                case PG_AIR_IS_TRANSITION: return plan->sel_word[2];
-                default: return consts[std::make_pair(nd.kind, nd.kind == PG_AIR_CONSTANT ? nd.a : nd.b)];
-            }
-            for (const auto& r : plan->runs)
-                if (r.src == src && r.next == nd.a && nd.b >= r.col0 && nd.b < r.col0 + r.count)
-                    return (r.slot0 + nd.b - r.col0) * QRS_COL;
-            return 0;
-        };
+        uint32_t next = base_words;
         std::vector<size_t> last_use(nodes.size()), item_of(nodes.size());
         std::vector<uint32_t> reg(nodes.size(), 0);
         bool fits = true;
@@ -4154,7 +4213,7 @@ static std::unique_ptr<QResident> air_resident(const std::vector<pg_air_node>& n
             sl.start = (uint32_t)(plan->code.size() / 2);
             sl.regs = base;
             auto word = [&](uint32_t n, size_t t, uint32_t prev_flag, uint32_t& fl) -> uint32_t {
-                if (air_is_leaf(nodes[n])) return leaf_word(n);
+                if (air_is_leaf(nodes[n])) return word_of[n];
                 if (item_of[n] + 1 == t) {
                     fl |= prev_flag;
                     return zero;
@@ -4178,7 +4237,7 @@ static std::unique_ptr<QResident> air_resident(const std::vector<pg_air_node>& n
                         continue;
                     }
                     fl = QF_ADD | QF_ASSERT;
-                    a = air_is_leaf(nd) ? leaf_word(n) : base + 64 * reg[n];
+                    a = air_is_leaf(nd) ? word_of[n] : base + 64 * reg[n];
                     b = zero;
                     release(n, t);
                 } else {
