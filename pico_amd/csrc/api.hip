@@ -2439,12 +2439,42 @@ extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* eval
     std::vector<size_t> tall(njobs);
     for (size_t j = 0; j < njobs; j++) tall[j] = j;
     std::stable_sort(tall.begin(), tall.end(), [&](size_t a, size_t c) { return N[a] > N[c]; });
+    // Leaves: a wave hashes 64 rows of one matrix; matrices of fewer than 64 rows
+    // share waves, those of equal chunk counts together.
     std::vector<LeafJob> leaves;
     std::vector<uint64_t> leaf_prefix(1, 0);
+    auto add_leaves = [&](const LeafJob& lj) {
+        leaves.push_back(lj);
+        leaf_prefix.push_back(leaf_prefix.back() + lj.rows / 64);
+    };
+    std::vector<size_t> low;
     for (size_t j : tall) {
-        leaves.push_back(LeafJob{b->trees[j]->mats[0]->ptr, W[j], (uint32_t)W[j], (uint32_t)N[j], digests[j]});
-        leaf_prefix.push_back(leaf_prefix.back() + (N[j] + 63) / 64);  // a wave hashes 64 rows of one job
+        if (N[j] < 64)
+            low.push_back(j);
+        else
+            add_leaves(LeafJob{b->trees[j]->mats[0]->ptr, W[j], (uint32_t)W[j], (uint32_t)N[j], digests[j],
+                               LeafJob::NO_PACK, 0});
     }
+    auto chunks = [&](size_t j) { return (W[j] + 7) / 8; };
+    std::stable_sort(low.begin(), low.end(), [&](size_t a, size_t c) { return chunks(a) > chunks(c); });
+    std::vector<LeafRow> pack_rows;
+    for (size_t i = 0; i < low.size();) {
+        const uint64_t c = chunks(low[i]);
+        const size_t first = pack_rows.size();
+        LeafJob lj{nullptr, 0, 0, 64, nullptr, (uint32_t)first, 1};
+        for (; i < low.size() && chunks(low[i]) == c && pack_rows.size() - first + N[low[i]] <= 64; i++) {
+            const size_t j = low[i];
+            for (uint64_t r = 0; r < N[j]; r++)
+                pack_rows.push_back(LeafRow{b->trees[j]->mats[0]->ptr + r * W[j], digests[j] + 8 * r, (uint32_t)W[j], 0});
+            lj.width = std::max(lj.width, (uint32_t)W[j]);
+            if (W[j] % 8) lj.whole = 0;
+        }
+        LeafRow pad = pack_rows.back();
+        pad.digest = nullptr;
+        pack_rows.resize(first + 64, pad);
+        add_leaves(lj);
+    }
+    const size_t off_pack_rows = st.put(pack_rows.data(), pack_rows.size() * sizeof(LeafRow));
     const size_t off_leaf = st.put(leaves.data(), leaves.size() * sizeof(LeafJob));
     const size_t off_leaf_prefix = st.put(leaf_prefix.data(), leaf_prefix.size() * 8);
     struct LevelRec {
@@ -2493,9 +2523,10 @@ extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* eval
     {
         const LeafJob* lj = (const LeafJob*)(dd + off_leaf);
         const uint64_t* lp = (const uint64_t*)(dd + off_leaf_prefix);
+        const LeafRow* pr = pack_rows.empty() ? nullptr : (const LeafRow*)(dd + off_pack_rows);
         const uint64_t total = leaf_prefix.back();
-        const int nj = (int)njobs;
-        b->launches.push_back([=](hipStream_t s) { return launch_leaf_hash_batch(field, lj, lp, nj, total, s); });
+        const int nj = (int)leaves.size();
+        b->launches.push_back([=](hipStream_t s) { return launch_leaf_hash_batch(field, lj, lp, nj, total, pr, s); });
     }
     for (const auto& lv : levels) {
         const CompressJob* cj = (const CompressJob*)(dd + lv.off_jobs);

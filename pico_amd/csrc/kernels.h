@@ -102,22 +102,34 @@ hipError_t launch_open_gather(const MatRef* mats, const uint32_t* shift, const u
                               hipStream_t stream);
 
 // ---- batched Merkle (merkle.hip): many single-matrix commits per launch ---
-// Jobs are found by binary search of the wave's group of 64 rows (leaves; a
-// job's last group may be partial) or the lane's node index in a prefix array
-// (njobs + 1 entries, prefix[0] = 0).
+// Jobs are found by binary search of the wave's group of 64 rows (leaves) or the
+// lane's node index in a prefix array (njobs + 1 entries, prefix[0] = 0).
+// A leaf job is the rows of one matrix (its last group may be partial) or a
+// pack: rows of several matrices of as many 8-word chunks each, 64 entries of a
+// table of rows from `pack` on, those past its own repeating one with a null digest.
+struct LeafRow {
+    const uint32_t* src;  // `width` words
+    uint32_t* digest;     // 8 words, or null
+    uint32_t width;
+    uint32_t pad_;
+};
 struct LeafJob {
+    static constexpr uint32_t NO_PACK = ~0u;
     const uint32_t* data;  // rows x width, row stride `stride`
     uint64_t stride;
-    uint32_t width;
-    uint32_t rows;
+    uint32_t width;  // pack: of the widest row
+    uint32_t rows;   // pack: 64
     uint32_t* digests;  // rows x 8
+    uint32_t pack;   // NO_PACK, or its first entry
+    uint32_t whole;  // pack: every row is whole chunks
 };
 struct CompressJob {
     const uint32_t* prev;  // 2 n x 8
     uint32_t* next;        // n x 8
 };
+// pack_rows: the table of rows, or null where no job is a pack
 hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t* group_prefix, int njobs,
-                                  uint64_t total_groups, hipStream_t stream);
+                                  uint64_t total_groups, const LeafRow* pack_rows, hipStream_t stream);
 hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint64_t* node_prefix,
                                  int njobs, uint64_t total_nodes, hipStream_t stream);
 // dst[8 j + k] = src[j][k] for j < n (root digests of n trees)

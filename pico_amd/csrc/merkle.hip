@@ -118,9 +118,16 @@ struct MxSponge {
     }
     // Absorbs one chunk: cnt of its 8 words overwrite the rate words.
     __device__ __forceinline__ void absorb(const u32x4 (&in)[2], uint32_t cnt, uint32_t h, MxView<F>& v) {
+        const uint32_t each[2] = {cnt, cnt};
+        absorb(in, cnt == 8, each, h, v);
+    }
+    // The same with a count per state: cnt[t] for the lane's state of tile t, 8
+    // in all of them where `whole`.
+    __device__ __forceinline__ void absorb(const u32x4 (&in)[2], bool whole, const uint32_t (&cnt)[2], uint32_t h,
+                                           MxView<F>& v) {
         int x[2][8];
         v.fresh();
-        if (cnt == 8) {
+        if (whole) {
             const mx4 rate[2] = {mx_op(in[0]), mx_op(in[1])};
             mx_next<F>(x, rate, b, v);
         } else {
@@ -131,7 +138,7 @@ struct MxSponge {
             for (int t = 0; t < 2; t++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    if (4 * h + i < cnt) st[t][i] = in[t][i];
+                    if (4 * h + i < cnt[t]) st[t][i] = in[t][i];
                 full[t][0] = mx_op_words(&st[t][0]);
                 full[t][1] = mx_op_words(&st[t][4]);
             }
@@ -682,10 +689,14 @@ __device__ __forceinline__ int find_job(const uint64_t* __restrict__ prefix, int
 }
 
 // Leaf layer of many jobs: wave -> (job, group of 64 rows); rows of any width.
-template <class F>
-MX_KERNEL leaf_hash_batch_kernel(const LeafJob* __restrict__ jobs,
-                                                                     const uint64_t* __restrict__ prefix,
-                                                                     int njobs, uint64_t total) {
+// A permutation takes a wave the same time with one row as with 64, so matrices
+// of fewer than 64 rows share waves (PACKS): 4096 of 16 rows x 50 hash in 65 us,
+// with a wave each in 143 us (one row per lane without matrix instructions: 74).
+// A batch without such matrices takes the form without packs, whose widths are
+// the same in every lane (64 jobs of 2^11 rows and more: 92.0 ms, 92.7 with packs).
+template <class F, bool PACKS>
+MX_KERNEL leaf_hash_batch_kernel(const LeafJob* __restrict__ jobs, const uint64_t* __restrict__ prefix, int njobs,
+                                 uint64_t total, const LeafRow* __restrict__ pack_rows) {
     __shared__ MxTable<F> tab;
     mx_load<F>(tab);
     const uint64_t wave = mx_wave();
@@ -695,34 +706,56 @@ MX_KERNEL leaf_hash_batch_kernel(const LeafJob* __restrict__ jobs,
     const uint64_t group = wave - prefix[j];
     MxView<F> v(tab);
     const MxLane l;
-    uint64_t row[2];
-    mx_group_rows(row, group, jb->rows, l);
-    const uint32_t width = jb->width;
+    const uint32_t widest = jb->width;
     gcptr rp[2];
+    uint32_t width[2] = {widest, widest};
+    bool pack = false;
+    if constexpr (PACKS) pack = jb->pack != LeafJob::NO_PACK;
+    if (pack) {
 #pragma unroll
-    for (int t = 0; t < 2; t++) rp[t] = (gcptr)jb->data + row[t] * jb->stride + 4 * l.h;
+        for (int t = 0; t < 2; t++) {
+            const LeafRow* const r = pack_rows + jb->pack + 32 * t + l.n;
+            rp[t] = (gcptr)r->src + 4 * l.h;
+            width[t] = r->width;
+        }
+    } else {
+        uint64_t row[2];
+        mx_group_rows(row, group, jb->rows, l);
+#pragma unroll
+        for (int t = 0; t < 2; t++) rp[t] = (gcptr)jb->data + row[t] * jb->stride + 4 * l.h;
+    }
+    const bool whole = pack ? jb->whole != 0 : widest % 8 == 0;
     MxSponge<F> sp;
-    auto load = [&](uint32_t off, u32x4 (&out)[2]) {  // words past the row's end read as word 0
-        if (off + 8 <= width) {
+    auto load = [&](uint32_t off, u32x4 (&out)[2]) {  // words past a row's end read as word 0
+        if (whole || off + 8 < widest) {
 #pragma unroll
             for (int t = 0; t < 2; t++) out[t] = *reinterpret_cast<const GLOBAL u32x4u*>(rp[t] + off);
         } else {
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) out[t][i] = rp[t][off + 4 * l.h + i < width ? (int64_t)(off + i) : -(int64_t)(4 * l.h)];
+                for (int i = 0; i < 4; i++)
+                    out[t][i] = rp[t][off + 4 * l.h + i < width[t] ? (int64_t)(off + i) : -(int64_t)(4 * l.h)];
         }
     };
     u32x4 next[2];
     load(0, next);
-    for (uint32_t off = 0; off < width; off += 8) {
+    for (uint32_t off = 0; off < widest; off += 8) {
         const u32x4 cur[2] = {next[0], next[1]};
-        if (off + 8 < width) load(off + 8, next);
-        sp.absorb(cur, width - off < 8u ? width - off : 8u, l.h, v);
+        if (off + 8 < widest) load(off + 8, next);
+        const uint32_t cnt[2] = {width[0] - off, width[1] - off};
+        sp.absorb(cur, whole || off + 8 < widest, cnt, l.h, v);
     }
     uint32_t st[2][8];
     mx_last<F>(st, sp.b, v);
-    mx_store_digests(jb->digests, group, jb->rows, l, st);
+    if (!pack) {
+        mx_store_digests(jb->digests, group, jb->rows, l, st);
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+        if (uint32_t* const d = pack_rows[jb->pack + 32 * t + l.n].digest)
+            *reinterpret_cast<GLOBAL u32x4*>((gptr)d + 4 * l.h) = u32x4{st[t][0], st[t][1], st[t][2], st[t][3]};
 }
 
 template <class F>
@@ -856,14 +889,21 @@ hipError_t launch_gather_roots(const uint32_t* const* src, uint32_t* dst, int n,
     return hipGetLastError();
 }
 
-hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t* prefix, int njobs,
-                                  uint64_t total, hipStream_t stream) {
-    if (total == 0) return hipSuccess;
-    if (field == FIELD_KOALABEAR)
-        leaf_hash_batch_kernel<KoalaBear><<<grid_for(total, MX_WAVES), MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
+template <class F>
+static hipError_t leaf_hash_batch_t(const LeafJob* jobs, const uint64_t* prefix, int njobs, uint64_t total,
+                                    const LeafRow* pack_rows, hipStream_t stream) {
+    const unsigned g = grid_for(total, MX_WAVES);
+    if (pack_rows)
+        leaf_hash_batch_kernel<F, true><<<g, MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total, pack_rows);
     else
-        leaf_hash_batch_kernel<BabyBear><<<grid_for(total, MX_WAVES), MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total);
+        leaf_hash_batch_kernel<F, false><<<g, MX_THREADS, 0, stream>>>(jobs, prefix, njobs, total, nullptr);
     return hipGetLastError();
+}
+hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t* prefix, int njobs, uint64_t total,
+                                  const LeafRow* pack_rows, hipStream_t stream) {
+    if (total == 0) return hipSuccess;
+    return field == FIELD_KOALABEAR ? leaf_hash_batch_t<KoalaBear>(jobs, prefix, njobs, total, pack_rows, stream)
+                                    : leaf_hash_batch_t<BabyBear>(jobs, prefix, njobs, total, pack_rows, stream);
 }
 
 hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint64_t* prefix, int njobs,
