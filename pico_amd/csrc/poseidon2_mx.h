@@ -442,6 +442,21 @@ struct MxRec {
 };
 
 // ---- device ------------------------------------------------------------------
+// The recurrence's constants in scalar registers, one v_mad_i64_i32 a product.
+// They pass through an empty asm, which hides their values: the compiler makes
+// products by constants near powers of two shifts and 64-bit subtractions.  A set
+// is made for each block of rounds: one for the whole kernel lets the sign
+// extensions leave loops, and each product becomes a full 64-bit one.  The
+// instruction itself is left to the compiler, because between a matrix
+// instruction and a vector instruction that touches its registers the program has
+// to wait (the hardware does not), and the compiler places those waits only for
+// instructions it knows.
+template <class F>
+struct MxConst {
+    int one = MxRec<F>::ONE, c1 = MxRec<F>::C1, c2 = MxRec<F>::C2, c3 = MxRec<F>::C3;
+    __device__ __forceinline__ MxConst() { asm("" : "+s"(one), "+s"(c1), "+s"(c2), "+s"(c3)); }
+};
+
 static __device__ const MxTable<KoalaBear> kMxKb = make_mx_table<KoalaBear>();
 static __device__ const MxTable<BabyBear> kMxBb = make_mx_table<BabyBear>();
 
@@ -568,32 +583,19 @@ __device__ __forceinline__ void mx_swap(int& a, int& b) {
     b = (int)r[1];
 }
 
-// a k + t for a constant k: one v_mad_i64_i32.  The constant passes through an
-// empty asm, which hides its value: the compiler makes products by constants
-// near powers of two shifts and 64-bit subtractions.  The instruction itself is
-// left to the compiler, because between a matrix instruction and a vector
-// instruction that touches its registers the program has to wait (the hardware
-// does not), and the compiler places those waits only for instructions it knows.
-template <int32_t K>
-__device__ __forceinline__ int64_t mx_mad(int a, int64_t t) {
-    int k = K;
-    asm("" : "+s"(k));
-    return (int64_t)a * k + t;
-}
-
 // The four S-boxes of a block of partial rounds: u the forms over everything
 // before the block, x' out
 template <class F>
 __device__ __forceinline__ void mx_block(int (&u)[4], int rounds) {
-    using R = MxRec<F>;
+    const MxConst<F> k;
 #pragma unroll
     for (int o = 0; o < 4; o++) {
         if (o >= rounds) continue;
         int v = u[o];
         if (o > 0) {
-            int64_t w = mx_mad<R::C1>(u[o - 1], mx_mad<R::ONE>(v, 0));
-            if (o > 1) w = mx_mad<R::C2>(u[o - 2], w);
-            if (o > 2) w = mx_mad<R::C3>(u[o - 3], w);
+            int64_t w = (int64_t)v * k.one + (int64_t)u[o - 1] * k.c1;
+            if (o > 1) w += (int64_t)u[o - 2] * k.c2;
+            if (o > 2) w += (int64_t)u[o - 3] * k.c3;
             v = mx_redc<F>(w);
         }
         u[o] = mx_sbox<F>(v);
@@ -797,6 +799,9 @@ struct Mx16 {
             const auto hi = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
             int w[4] = {(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};
             mx_block<F>(w, S::RP - 4 * b);
+            // all four are made in every lane: the compiler would move some under the
+            // selects' conditions, as branches
+            asm("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
             in[1 + b / 4][b % 4] = (int)((uint32_t)(q1 ? (q2 ? w[3] : w[1]) : (q2 ? w[2] : w[0])) ^ MX_BIAS);
         }
         in[0] = sbox(layer<S::STEPS>(in, S::FINAL, 4));
