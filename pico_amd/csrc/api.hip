@@ -2319,7 +2319,10 @@ extern "C" void pg_batch_free(pg_batch* b) {
     delete b;
 }
 
-// host staging for one device descriptor block
+// Waves of trees that run side by side, two per SIMD (their hash tables fill the
+// registers).
+static constexpr uint64_t TREE_BATCH_WAVES = 2048;
+
 extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* evals, const uint32_t* dshift,
                                const uint32_t* log_blowups, size_t njobs, int use_graph, pg_batch** out) {
     if (!ctx || !evals || !log_blowups || !out || !field_ok(field) || njobs == 0)
@@ -2477,27 +2480,61 @@ extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* eval
     const size_t off_pack_rows = st.put(pack_rows.data(), pack_rows.size() * sizeof(LeafRow));
     const size_t off_leaf = st.put(leaves.data(), leaves.size() * sizeof(LeafJob));
     const size_t off_leaf_prefix = st.put(leaf_prefix.data(), leaf_prefix.size() * 8);
+    // Levels above: one launch per level over the nodes of every job, 16 to a wave,
+    // until few enough trees are left that a workgroup can take several levels of
+    // one: where their waves all run at once (TREE_BATCH_WAVES).
     struct LevelRec {
         size_t off_jobs, off_prefix;
         int njobs;
-        uint64_t total;
+        uint64_t total;    // nodes, or workgroups
+        unsigned threads;  // 0: a single level
     };
     std::vector<LevelRec> levels;
-    const int max_log = log2_of(N[tall[0]]);
-    for (int lv = 1; lv <= max_log; lv++) {
-        std::vector<CompressJob> cj;
-        std::vector<uint64_t> pf(1, 0);
-        for (size_t j : tall) {
-            const int lj = log2_of(N[j]);
-            if (lj < lv) break;
-            uint64_t off_prev = 0;
-            for (int t = 0; t < lv - 1; t++) off_prev += N[j] >> t;
-            const uint64_t off_next = off_prev + (N[j] >> (lv - 1));
-            cj.push_back(CompressJob{digests[j] + 8 * off_prev, digests[j] + 8 * off_next});
-            pf.push_back(pf.back() + (N[j] >> lv));
+    struct Rest {  // what is left of a tree
+        const uint32_t* in;
+        uint32_t* out;
+        uint64_t n0;
+        int layers;
+    };
+    std::vector<Rest> rest;
+    for (size_t j : tall)
+        if (N[j] > 1) rest.push_back(Rest{digests[j], digests[j] + 8 * N[j], N[j] / 2, log2_of(N[j])});
+    while (!rest.empty()) {
+        uint64_t nodes = 0, blocks = 0;
+        unsigned threads = 64;
+        int most = 0;
+        for (const Rest& t : rest) {
+            const TreeStep ts = tree_step(t.n0, t.layers, 0);
+            nodes += t.n0;
+            blocks += ts.blocks;
+            threads = std::max(threads, ts.threads);
+            most = std::max(most, ts.layers);
         }
-        levels.push_back(LevelRec{st.put(cj.data(), cj.size() * sizeof(CompressJob)), st.put(pf.data(), pf.size() * 8),
-                                  (int)cj.size(), pf.back()});
+        const bool several = nodes <= SMALL_MAX_NODES && most > 1 && blocks * (threads / 64) <= TREE_BATCH_WAVES;
+        std::vector<CompressJob> cj;
+        std::vector<TreeJob> tj;
+        std::vector<uint64_t> pf(1, 0);
+        for (Rest& t : rest) {
+            int now = 1;
+            if (several) {
+                const TreeStep ts = tree_step(t.n0, t.layers, 0);
+                tj.push_back(TreeJob{t.in, t.out, (uint32_t)t.n0, (uint32_t)ts.log_per, (uint32_t)ts.layers, 0});
+                pf.push_back(pf.back() + ts.blocks);
+                now = ts.layers;
+            } else {
+                cj.push_back(CompressJob{t.in, t.out});
+                pf.push_back(pf.back() + t.n0);
+            }
+            for (int i = 0; i < now; i++, t.n0 /= 2) {
+                t.in = t.out;
+                t.out += 8 * t.n0;
+            }
+            t.layers -= now;
+        }
+        levels.push_back(LevelRec{several ? st.put(tj.data(), tj.size() * sizeof(TreeJob))
+                                          : st.put(cj.data(), cj.size() * sizeof(CompressJob)),
+                                  st.put(pf.data(), pf.size() * 8), (int)rest.size(), pf.back(), several ? threads : 0});
+        rest.erase(std::remove_if(rest.begin(), rest.end(), [](const Rest& t) { return t.layers == 0; }), rest.end());
     }
     std::vector<const uint32_t*> root_src(njobs);
     for (size_t j = 0; j < njobs; j++) root_src[j] = digests[j] + 8 * (2 * N[j] - 2);
@@ -2529,8 +2566,15 @@ extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* eval
         b->launches.push_back([=](hipStream_t s) { return launch_leaf_hash_batch(field, lj, lp, nj, total, pr, s); });
     }
     for (const auto& lv : levels) {
-        const CompressJob* cj = (const CompressJob*)(dd + lv.off_jobs);
         const uint64_t* pf = (const uint64_t*)(dd + lv.off_prefix);
+        if (lv.threads) {
+            const TreeJob* tj = (const TreeJob*)(dd + lv.off_jobs);
+            b->launches.push_back([=](hipStream_t s) {
+                return launch_tree_layers_batch(field, tj, pf, lv.njobs, (unsigned)lv.total, lv.threads, s);
+            });
+            continue;
+        }
+        const CompressJob* cj = (const CompressJob*)(dd + lv.off_jobs);
         b->launches.push_back([=](hipStream_t s) { return launch_compress_batch(field, cj, pf, lv.njobs, lv.total, s); });
     }
     {

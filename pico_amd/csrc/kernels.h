@@ -130,6 +130,22 @@ struct CompressJob {
 // pack_rows: the table of rows, or null where no job is a pack
 hipError_t launch_leaf_hash_batch(int field, const LeafJob* jobs, const uint64_t* group_prefix, int njobs,
                                   uint64_t total_groups, const LeafRow* pack_rows, hipStream_t stream);
+// One launch of launch_tree_layers: 2^log_per first-layer nodes per workgroup and
+// `layers` layers of them.
+struct TreeStep {
+    int log_per, layers;
+    unsigned blocks, threads;
+};
+TreeStep tree_step(uint64_t n0, int layers, uint32_t leaf_width);
+// The same for several trees at once: workgroups are found by binary search in
+// the prefix array; `threads` is the most any job's step has.
+struct TreeJob {
+    const uint32_t* in;  // 2 n0 digests
+    uint32_t* out;       // the layers n0, n0/2, ... one after the other
+    uint32_t n0, log_per, layers, pad_;
+};
+hipError_t launch_tree_layers_batch(int field, const TreeJob* jobs, const uint64_t* block_prefix, int njobs,
+                                    unsigned blocks, unsigned threads, hipStream_t stream);
 hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint64_t* node_prefix,
                                  int njobs, uint64_t total_nodes, hipStream_t stream);
 // dst[8 j + k] = src[j][k] for j < n (root digests of n trees)

@@ -585,11 +585,36 @@ __device__ __forceinline__ u32x4 mx16_hash_row(const Mx16<F>& P, gcptr row, uint
     return mx16_words<F>(st);
 }
 
-enum { TREE_NODES, TREE_ROWS, TREE_FOLDED };  // what the first layer hashes
+// The job whose range of the prefix array (njobs + 1 entries) holds i
+__device__ __forceinline__ int find_job(const uint64_t* __restrict__ prefix, int njobs, uint64_t i) {
+    int lo = 0, hi = njobs;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (prefix[mid] <= i) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// What the first layer hashes.  TREE_JOBS: the nodes of one of several trees: `in`
+// is the table of n0 jobs and `stride` the address of the prefix array over their
+// workgroups (arguments of their own cost the other forms 1%: a cache line more).
+enum { TREE_NODES, TREE_ROWS, TREE_FOLDED, TREE_JOBS };
 template <class F, int FIRST>
 MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint32_t width, uint64_t n0, int log_per, int layers,
                                uint32_t* out, TreeChallenge ch, TreeFold fold) {
     __shared__ u32x4 buf[2][2 * TREE_MAX_PER];
+    uint32_t block = blockIdx.x;  // of the tree's first layer
+    if constexpr (FIRST == TREE_JOBS) {
+        const uint64_t* const prefix = reinterpret_cast<const uint64_t*>(stride);
+        const int j = __builtin_amdgcn_readfirstlane(find_job(prefix, (int)n0, block));
+        const TreeJob* const jb = reinterpret_cast<const TreeJob*>(in) + j;
+        block -= (uint32_t)prefix[j];
+        in = jb->in;
+        out = jb->out;
+        n0 = jb->n0;
+        log_per = (int)jb->log_per;
+        layers = (int)jb->layers;
+    }
     if constexpr (FIRST == TREE_FOLDED) {  // before the hash tables fill the registers
         uint32_t beta[4];
 #pragma unroll
@@ -597,7 +622,7 @@ MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint32_t wid
         const int log_n_out = 64 - __builtin_clzll(n0);  // of 2 n0 elements
         const uint32_t cnt = 2u << log_per;
         for (uint32_t t = threadIdx.x; t < cnt; t += blockDim.x) {
-            const uint64_t i = (uint64_t)blockIdx.x * cnt + t;
+            const uint64_t i = (uint64_t)block * cnt + t;
             const u32x4 o = fri_fold_at<F>((gcptr)fold.prev, i, log_n_out, beta, (gcptr)fold.tw, (gcptr)fold.add);
             reinterpret_cast<GLOBAL u32x4*>((gptr)fold.out)[i] = o;
             buf[1][t] = o;
@@ -610,7 +635,7 @@ MX16_KERNEL tree_layers_kernel(const uint32_t* in, uint64_t stride, uint32_t wid
     gptr layer = (gptr)out;
     for (int i = 0; i < layers; i++) {
         const uint32_t cnt = (1u << log_per) >> i;
-        const uint64_t base = (uint64_t)blockIdx.x * cnt;
+        const uint64_t base = (uint64_t)block * cnt;
         for (uint32_t g = wave; 16 * g < cnt; g += waves) {  // the wave's group of 16 nodes
             const uint32_t nd = 16 * g + l.n, nr = nd < cnt ? nd : cnt - 1;
             u32x4 w;
@@ -679,15 +704,6 @@ hipError_t launch_fri_open(const FriOpenRound* rounds, int nrounds, const uint64
 }
 
 // ---- batched single-matrix commits --------------------------------------
-__device__ __forceinline__ int find_job(const uint64_t* __restrict__ prefix, int njobs, uint64_t i) {
-    int lo = 0, hi = njobs;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (prefix[mid] <= i) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
 // Leaf layer of many jobs: wave -> (job, group of 64 rows); rows of any width.
 // A permutation takes a wave the same time with one row as with 64, so matrices
 // of fewer than 64 rows share waves (PACKS): 4096 of 16 rows x 50 hash in 65 us,
@@ -924,6 +940,32 @@ hipError_t launch_compress_batch(int field, const CompressJob* jobs, const uint6
     return hipGetLastError();
 }
 
+// Nodes (or rows) of the first layer, at most SMALL_MAX_NODES: 64 per workgroup
+// and seven layers a launch, one workgroup for all the rest once a layer has at
+// most 128 nodes (rows of several chunks stay at 64: a wave would hash its two
+// groups of rows one after the other).
+TreeStep tree_step(uint64_t n0, int layers, uint32_t leaf_width) {
+    TreeStep t;
+    t.log_per = 6;
+    if (n0 <= (uint64_t)(leaf_width > 8 ? 64 : TREE_MAX_PER)) t.log_per = __builtin_ctzll(n0);
+    t.layers = std::min(layers, t.log_per + 1);
+    t.threads = std::min((unsigned)S_THREADS, std::max(64u, 4u << t.log_per));
+    t.blocks = (unsigned)(n0 >> t.log_per);
+    return t;
+}
+
+hipError_t launch_tree_layers_batch(int field, const TreeJob* jobs, const uint64_t* prefix, int njobs, unsigned blocks,
+                                    unsigned threads, hipStream_t stream) {
+    if (blocks == 0) return hipSuccess;
+    const uint32_t* const in = reinterpret_cast<const uint32_t*>(jobs);
+    const uint64_t at = reinterpret_cast<uint64_t>(prefix);
+    if (field == FIELD_KOALABEAR)
+        tree_layers_kernel<KoalaBear, TREE_JOBS><<<blocks, threads, 0, stream>>>(in, at, 0, njobs, 0, 0, nullptr, {}, {});
+    else
+        tree_layers_kernel<BabyBear, TREE_JOBS><<<blocks, threads, 0, stream>>>(in, at, 0, njobs, 0, 0, nullptr, {}, {});
+    return hipGetLastError();
+}
+
 hipError_t launch_leaf_hash(int field, const MatRef* mats, int n, uint32_t total_width,
                             size_t rows, uint32_t* digests, hipStream_t stream) {
     if (rows == 0) return hipSuccess;
@@ -969,21 +1011,14 @@ hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride,
     return hipGetLastError();
 }
 
-// Nodes (or rows) of the first layer, at most SMALL_MAX_NODES: 64 per workgroup
-// and seven layers a launch, one workgroup for all the rest once a layer has at
-// most 128 nodes (rows of several chunks stay at 64: a wave would hash its two
-// groups of rows one after the other).
 template <class F>
 static hipError_t tree_layers_t(const uint32_t* in, uint64_t stride, uint32_t leaf_width, uint64_t n0, int layers,
                                 uint32_t* out, hipStream_t s, const TreeChallenge* ch, const TreeFold* fold) {
     while (layers > 0) {
-        int log_per = 6;
-        if (n0 <= (uint64_t)(leaf_width > 8 ? 64 : TREE_MAX_PER))
-            log_per = __builtin_ctzll(n0);
-        const int now = std::min(layers, log_per + 1);
+        const TreeStep t = tree_step(n0, layers, leaf_width);
+        const int log_per = t.log_per, now = t.layers;
+        const unsigned threads = t.threads, g = t.blocks;
         const TreeChallenge c = ch && now == layers ? *ch : TreeChallenge{};
-        const unsigned threads = std::min((unsigned)S_THREADS, std::max(64u, 4u << log_per));
-        const unsigned g = (unsigned)(n0 >> log_per);
         if (fold)
             tree_layers_kernel<F, TREE_FOLDED><<<g, threads, 0, s>>>(nullptr, 0, 0, n0, log_per, now, out, c, *fold);
         else if (leaf_width)

@@ -56,3 +56,30 @@ def test_many_jobs(ctx, oracle):
     batch.free()
     for m in mats:
         m.free()
+
+
+@pytest.mark.parametrize("f", [KOALABEAR, BABYBEAR])
+@pytest.mark.parametrize("jobs", [
+    [(L, 5, 1) for L in (14, 9, 7, 6, 5, 1, 0)],    # first layers of 2^14 .. 1 nodes, trees that end early
+    [(6, 3, 0), (7, 3, 0), (8, 3, 0), (0, 3, 0)],   # 64, 128 and 256 leaves, and one
+    [(5, 9, 1)] * 40,                               # one workgroup per tree
+    [(4, 9, 1)] * 1100 + [(8, 2, 1)],               # more trees than run side by side, then one
+], ids=["tall to short", "around a workgroup", "equal", "many"])
+def test_levels_match_oracle(ctx, oracle, f, jobs):
+    g = pico_amd.GENERATORS[f]
+    hosts = [oracle.random_matrix(f, 900 + k, 1 << L, w) for k, (L, w, _) in enumerate(jobs)]
+    mats = [ctx.upload(a, field=f) for a in hosts]
+    batch = pico_amd.CommitBatch(ctx, f, [(m, b) for m, (_, _, b) in zip(mats, jobs)])
+    for _ in range(2):
+        roots = batch.run()
+    for k, (a, (_, _, b)) in enumerate(zip(hosts, jobs)):
+        ot = oracle.MerkleTree(f, [oracle.coset_lde(f, a, b, g)])
+        assert np.array_equal(roots[k], ot.root), k
+        if k % 100 < 8:
+            tree = batch.take(k)
+            for j in range(tree.log_height + 1):
+                assert np.array_equal(tree.digest_layer(j), ot.layer(j)), (k, j)
+            tree.free()
+    batch.free()
+    for m in mats:
+        m.free()
