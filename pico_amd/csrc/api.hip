@@ -2320,7 +2320,9 @@ extern "C" void pg_batch_free(pg_batch* b) {
 }
 
 // Waves of trees that run side by side, two per SIMD (their hash tables fill the
-// registers).
+// registers).  Up to here several levels per launch are the faster form (2048 trees
+// of 32 leaves 120 -> 102 us, one of 2^11 111 -> 91), above it packed levels (4096
+// trees of 4 leaves 171 us, 182 with several levels; 16384 of 8 leaves 474, 532).
 static constexpr uint64_t TREE_BATCH_WAVES = 2048;
 
 extern "C" int pg_batch_create(pg_ctx* ctx, int field, const pg_buf* const* evals, const uint32_t* dshift,
@@ -3356,6 +3358,11 @@ extern "C" int pg_pcs_open(pg_ctx* ctx, const pg_tree* const* rounds, size_t nro
                 }
             }
         pg_challenger observed = *ch;  // kept only if every value came down
+        // The second stream is leased like the first, so a part can wait for what
+        // another call has queued there (an open beside a thread that commits 2^19 x
+        // 256 takes 8 ms).  A fifth stream for downloads alone gave 5.4 to 8.0 ms
+        // there, but it shares a hardware queue with one of the four: opening 2000
+        // columns at a point went from 72 to 83 us.
         for (const Part& p : parts) {
             HIP_TRY(hipStreamWaitEvent(down.s, p.done, 0));
             HIP_TRY(hipMemcpyAsync(pf->values.data() + p.begin, (const uint32_t*)values->ptr + p.begin,
