@@ -1966,11 +1966,48 @@ static Ext4 bary_factor(const Ext4& z, uint32_t s_mont, int log_h) {
 // orders its uses), the values side by side in `out`.
 struct OpenQueue {
     std::map<std::vector<uint32_t>, std::shared_ptr<DevMem>> weights;
-    std::vector<std::shared_ptr<DevMem>> scratch;  // the last is the largest; the others may be in use
-    size_t scratch_bytes = 0;
+    std::shared_ptr<DevMem> scratch;  // of the largest matrix
+    size_t scratch_limit = SIZE_MAX;
     std::vector<std::shared_ptr<DevMem>> twiddles;
     uint8_t* out = nullptr;  // of the next matrix
 };
+
+// Scratch of one matrix's opening at npts points, in bytes: twiddles, weights,
+// partials, slice sums, output.  In a fixed region the twiddle table is built in
+// the region itself and two points go per launch (weights of two points at a
+// time); a queue holds twiddles, weights and output elsewhere.  Chunks are made
+// taller until the partial sums fit `limit`, where they can.  Any chunking gives
+// the same values: every sum is exact mod p.
+enum class OvScratch { OWN, QUEUE, FIXED };
+struct OvLayout {
+    size_t per;  // points per launch
+    uint32_t chunk_rows, nchunks, nslices;
+    size_t b_t, b_w, b_p, b_s, b_o;
+    size_t total() const { return b_t + b_w + b_p + b_s + b_o; }
+};
+static OvLayout ov_layout(const pg_buf* m, size_t h, size_t npts, OvScratch where, size_t limit) {
+    const size_t w = m->cols;
+    OvLayout y;
+    y.per = where == OvScratch::FIXED ? 2 : 4;
+    const size_t q_max = std::min(npts, y.per);
+    // about 2^17 (chunk, column) threads, at least 16 rows per chunk: taller
+    // chunks write fewer partial sums (2^20 x 256 at two points: 0.29 ms
+    // against 0.30 with 2^18 threads, 0.34 with 2^20, 0.39 with 2^16)
+    const uint64_t col_threads = open_values_vec4(m->ptr, m->cols, (uint32_t)w, (int)q_max) ? w / 4 : w;
+    y.chunk_rows = 16;
+    while ((uint64_t)y.chunk_rows * (1u << 17) < (uint64_t)h * col_threads) y.chunk_rows <<= 1;
+    for (;; y.chunk_rows <<= 1) {
+        y.nchunks = (uint32_t)((h + y.chunk_rows - 1) / y.chunk_rows);
+        // column sums in slices of about 64 chunks (at most 64 slices)
+        y.nslices = std::max<uint32_t>(1, std::min<uint32_t>(64, y.nchunks / 64));
+        y.b_t = where == OvScratch::FIXED ? round_up(4 * h, 256) : 0;
+        y.b_w = where == OvScratch::QUEUE ? 0 : round_up(q_max * h * 16, 256);
+        y.b_p = round_up(q_max * y.nchunks * w * 16, 256);
+        y.b_s = round_up(q_max * y.nslices * w * 16, 256);
+        y.b_o = where == OvScratch::QUEUE ? 0 : npts * w * 16;
+        if (y.total() <= limit || y.chunk_rows >= h) return y;
+    }
+}
 
 template <class F>
 static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k, uint32_t log_blowup,
@@ -1983,44 +2020,15 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
     const int log_h = log2_of(m->rows) - (int)log_blowup;
     const size_t h = (size_t)1 << log_h, w = m->cols;
     if (npts == 0 || w == 0) return PG_OK;
-    // In a fixed region the twiddle table is built in the region itself, two
-    // points go per launch (weights of two points at a time), and chunks are
-    // made taller until the partial sums fit.  Any chunking gives the same
-    // values: every sum is exact mod p.
-    const size_t per = fixed ? 2 : 4;  // points per launch
-    const size_t q_max = std::min(npts, per);
-    // about 2^17 (chunk, column) threads, at least 16 rows per chunk: taller
-    // chunks write fewer partial sums (2^20 x 256 at two points: 0.29 ms
-    // against 0.30 with 2^18 threads, 0.34 with 2^20, 0.39 with 2^16)
-    const uint64_t col_threads = open_values_vec4(m->ptr, m->cols, (uint32_t)w, (int)q_max) ? w / 4 : w;
-    uint32_t chunk_rows = 16;
-    while ((uint64_t)chunk_rows * (1u << 17) < (uint64_t)h * col_threads) chunk_rows <<= 1;
-    struct Layout {
-        uint32_t nchunks, nslices;
-        size_t b_t, b_w, b_p, b_s, b_o;  // twiddles, weights, partials, slice sums, output
-        size_t total() const { return b_t + b_w + b_p + b_s + b_o; }
-    };
-    auto layout = [&](uint32_t cr) {
-        Layout y;
-        y.nchunks = (uint32_t)((h + cr - 1) / cr);
-        // column sums in slices of about 64 chunks (at most 64 slices)
-        y.nslices = std::max<uint32_t>(1, std::min<uint32_t>(64, y.nchunks / 64));
-        y.b_t = fixed ? round_up(4 * h, 256) : 0;
-        y.b_w = oq ? 0 : round_up(q_max * h * 16, 256);
-        y.b_p = round_up(q_max * y.nchunks * w * 16, 256);
-        y.b_s = round_up(q_max * y.nslices * w * 16, 256);
-        y.b_o = oq ? 0 : npts * w * 16;
-        return y;
-    };
-    Layout y = layout(chunk_rows);
-    if (fixed) {
-        while (y.total() > fixed->bytes && chunk_rows < h) y = layout(chunk_rows <<= 1);
-        if (y.total() > fixed->bytes)
-            return fail(PG_E_INVALID,
-                        "matrix %zu (trace height 2^%d, width %zu, %zu points) needs %zu bytes of scratch; the "
-                        "allocation-free form has %zu",
-                        k, log_h, w, npts, y.total(), fixed->bytes);
-    }
+    const OvLayout y = ov_layout(m, h, npts, fixed ? OvScratch::FIXED : oq ? OvScratch::QUEUE : OvScratch::OWN,
+                                 fixed ? fixed->bytes : oq ? oq->scratch_limit : SIZE_MAX);
+    const size_t per = y.per;
+    const uint32_t chunk_rows = y.chunk_rows;
+    if (fixed && y.total() > fixed->bytes)
+        return fail(PG_E_INVALID,
+                    "matrix %zu (trace height 2^%d, width %zu, %zu points) needs %zu bytes of scratch; the "
+                    "allocation-free form has %zu",
+                    k, log_h, w, npts, y.total(), fixed->bytes);
     std::shared_ptr<DevMem> tw, scratch;
     uint8_t* base;
     const uint32_t* twp;
@@ -2030,19 +2038,13 @@ static int open_values_t(pg_ctx* ctx, hipStream_t s, const pg_tree* t, size_t k,
     } else {
         PG_TRY(get_twiddles(ctx, s, t->field, log_h, &tw));
         twp = (const uint32_t*)tw->ptr;
-        int rc;
-        if (oq && y.total() <= oq->scratch_bytes) {
-            scratch = oq->scratch.back();
+        if (oq) {
+            scratch = oq->scratch;
+            oq->twiddles.push_back(tw);
         } else {
+            int rc;
             scratch = make_devmem(ctx, y.total(), &rc);
             if (!scratch) return rc;
-        }
-        if (oq) {
-            if (y.total() > oq->scratch_bytes) {
-                oq->scratch.push_back(scratch);
-                oq->scratch_bytes = y.total();
-            }
-            oq->twiddles.push_back(tw);
         }
         base = (uint8_t*)scratch->ptr;
     }
@@ -3333,7 +3335,38 @@ extern "C" int pg_pcs_open(pg_ctx* ctx, const pg_tree* const* rounds, size_t nro
         OpenQueue oq;
         PG_TRY(bind_device(ctx));
         int rc = PG_OK;
-        auto values = make_devmem(ctx, std::max<size_t>(nvals * 4, 16), &rc);
+        // One scratch buffer, the largest matrix's.  The values of all matrices stay on
+        // the device until they are observed, so where the budget is short the partial
+        // sums are made smaller by as much: no more memory than one matrix after the
+        // other takes.
+        auto each = [&](auto&& f) {  // the trace height and points of every opened matrix
+            size_t i = 0;
+            for (size_t r = 0; r < nrounds; r++)
+                for (const pg_buf* m : rounds[r]->mats) {
+                    const size_t np = npoints[i++], h = log_blowup < 32 ? m->rows >> log_blowup : 0;
+                    if (np && m->cols && h) f(m, h, np);
+                }
+        };
+        auto largest = [&] {
+            size_t most = 16;
+            each([&](const pg_buf* m, size_t h, size_t np) {
+                most = std::max(most, ov_layout(m, h, np, OvScratch::QUEUE, oq.scratch_limit).total());
+            });
+            return most;
+        };
+        size_t weight_bytes = 0;  // at most
+        each([&](const pg_buf*, size_t h, size_t np) { weight_bytes += np * h * 16; });
+        const size_t value_bytes = std::max<size_t>(nvals * 4, 16);
+        if (ctx->budget && ctx->in_use.load() + weight_bytes + value_bytes + largest() > ctx->budget) {
+            size_t serial = 16;  // one matrix after the other: its scratch and its values
+            each([&](const pg_buf* m, size_t h, size_t np) {
+                serial = std::max(serial, ov_layout(m, h, np, OvScratch::QUEUE, SIZE_MAX).total() + np * m->cols * 16);
+            });
+            oq.scratch_limit = serial > value_bytes + 1024 ? serial - value_bytes - 1024 : 0;  // 1024: rounding of two blocks
+        }
+        oq.scratch = make_devmem(ctx, largest(), &rc);
+        if (!oq.scratch) return rc;
+        auto values = make_devmem(ctx, value_bytes, &rc);
         if (!values) return rc;
         oq.out = (uint8_t*)values->ptr;
         Lease l(ctx), down(ctx);
