@@ -3246,23 +3246,45 @@ extern "C" int pg_fri_answer_queries(pg_ctx* ctx, const pg_fri* f, const uint64_
         rd[r] = FriOpenRound{t->mats[0]->ptr, t->digests, (uint32_t)t->log_h, (uint32_t)pw};
         pw += 8 * (size_t)t->log_h;
     }
-    // indices and rounds up, every round's answers down, one launch
-    const size_t o_idx = align_up(R * sizeof(FriOpenRound), 256), o_sib = align_up(o_idx + nq * 8, 256),
-                 sib_bytes = nq * R * 16, o_paths = o_sib + align_up(sib_bytes, 256), bytes = o_paths + nq * pw * 4;
+    // Indices and rounds up, every round's answers down, one launch; where the budget
+    // is short, as many queries at a time as fit what one round's answers to all of
+    // them take.
+    struct Layout {
+        size_t o_idx, o_sib, o_paths, bytes;
+    };
+    auto layout = [&](size_t n) {
+        Layout y;
+        y.o_idx = align_up(R * sizeof(FriOpenRound), 256);
+        y.o_sib = align_up(y.o_idx + n * 8, 256);
+        y.o_paths = y.o_sib + align_up(n * R * 16, 256);
+        y.bytes = y.o_paths + n * pw * 4;
+        return y;
+    };
+    size_t each = nq;
+    if (ctx->budget && ctx->in_use.load() + layout(nq).bytes > ctx->budget) {
+        const size_t one_round = align_up(nq * 8, 256) + align_up(nq * 32, 256) + nq * f->trees[0]->log_h * 32;
+        while (each > 1 && layout(each).bytes > one_round) each = (each + 1) / 2;
+    }
+    const Layout y = layout(each);
     int rc;
-    auto d = make_devmem(ctx, bytes, &rc);
+    auto d = make_devmem(ctx, y.bytes, &rc);
     if (!d) return rc;
     uint8_t* const dm = (uint8_t*)d->ptr;
-    std::vector<uint8_t> h(o_idx + nq * 8);
+    std::vector<uint8_t> h(y.o_idx + each * 8);
     memcpy(h.data(), rd.data(), R * sizeof(FriOpenRound));
-    memcpy(h.data() + o_idx, idx, nq * 8);
     SyncGuard guard(l.s);
-    HIP_TRY(hipMemcpyAsync(dm, h.data(), h.size(), hipMemcpyHostToDevice, l.s));
-    HIP_TRY(launch_fri_open((const FriOpenRound*)dm, R, (const uint64_t*)(dm + o_idx), (int)nq, (uint32_t)pw,
-                            (uint32_t*)(dm + o_sib), (uint32_t*)(dm + o_paths), l.s));
-    if (siblings_out) HIP_TRY(hipMemcpyAsync(siblings_out, dm + o_sib, sib_bytes, hipMemcpyDeviceToHost, l.s));
-    if (paths_out && pw) HIP_TRY(hipMemcpyAsync(paths_out, dm + o_paths, nq * pw * 4, hipMemcpyDeviceToHost, l.s));
-    HIP_TRY(hipStreamSynchronize(l.s));
+    for (size_t q = 0; q < nq; q += each) {
+        const size_t n = std::min(each, nq - q);
+        memcpy(h.data() + y.o_idx, idx + q, n * 8);
+        HIP_TRY(hipMemcpyAsync(dm, h.data(), y.o_idx + n * 8, hipMemcpyHostToDevice, l.s));
+        HIP_TRY(launch_fri_open((const FriOpenRound*)dm, R, (const uint64_t*)(dm + y.o_idx), (int)n, (uint32_t)pw,
+                                (uint32_t*)(dm + y.o_sib), (uint32_t*)(dm + y.o_paths), l.s));
+        if (siblings_out)
+            HIP_TRY(hipMemcpyAsync(siblings_out + q * R * 4, dm + y.o_sib, n * R * 16, hipMemcpyDeviceToHost, l.s));
+        if (paths_out && pw)
+            HIP_TRY(hipMemcpyAsync(paths_out + q * pw, dm + y.o_paths, n * pw * 4, hipMemcpyDeviceToHost, l.s));
+        HIP_TRY(hipStreamSynchronize(l.s));
+    }
     guard.armed = false;
     return PG_OK;
 }
