@@ -6,7 +6,7 @@
 namespace pg {
 // out[i] = (v[2i] + v[2i+1]) / 2 + beta / (2 x_i) (v[2i] - v[2i+1]) + add[i] for
 // ext4 vectors, i < 2^log_n_out; tw: w_n^e for n = 2^(log_n_out + 1); add may be
-// null.
+// null and, a caller's vector, at any word.
 template <class F>
 __device__ __forceinline__ u32x4 fri_fold_at(gcptr v, uint64_t i, int log_n_out, const uint32_t (&beta)[4], gcptr tw,
                                              gcptr add) {
@@ -24,7 +24,7 @@ __device__ __forceinline__ u32x4 fri_fold_at(gcptr v, uint64_t i, int log_n_out,
     for (int k = 0; k < 4; k++) half_beta.c[k] = fhalve<F>(beta[k]);
     Ext4 o = eadd<F>(s, emul<F>(d, half_beta));
     if (add) {
-        const u32x4 w = reinterpret_cast<const GLOBAL u32x4*>(add)[i];
+        const u32x4 w = reinterpret_cast<const GLOBAL u32x4u*>(add)[i];
         o = eadd<F>(o, Ext4{{w.x, w.y, w.z, w.w}});
     }
     return u32x4{o.c[0], o.c[1], o.c[2], o.c[3]};

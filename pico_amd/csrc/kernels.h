@@ -19,6 +19,7 @@ namespace pg {
 typedef GLOBAL const uint32_t* gcptr;
 typedef GLOBAL uint32_t* gptr;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // copyable across address spaces
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte access at word alignment
 
 // Optional per-launch timing hook: begin() before a kernel launch and end()
 // after it, on the launch stream (the implementation records HIP events).

@@ -31,7 +31,6 @@ constexpr int MX_THREADS = 64 * MX_WAVES;
 // the issue slots are not all filled (leaf hash of 2^21 x 256: 4.53 ms, 4.82
 // and 4.70).
 #define MX_KERNEL __global__ void __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
-typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16-byte access at word alignment
 
 // The lane's place in its wave: state 32 t + n of tile t, words 4 h + i of the
 // rate and of the capacity.
