@@ -3071,6 +3071,8 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
             return fail(PG_E_INVALID, "input %d must be 2^%d x 4", k, k);
     for (int k = 0; k <= max_log; k++) PG_TRY(need_dense(inputs[k], "pg_fri_commit_phase"));
     if (log_stop > L0) return fail(PG_E_INVALID, "log_stop > input length");
+    if (ch->n_input < 0 || ch->n_input > 7)  // the device places the root behind the pending inputs
+        return fail(PG_E_INVALID, "the challenger has %d pending inputs; a sponge chunk holds 8", ch->n_input);
     static_assert(sizeof(pg_challenger) == 4 * CHALLENGER_WORDS, "the device reads the challenger as words");
     PG_TRY(bind_device(ctx));
     Lease l(ctx);

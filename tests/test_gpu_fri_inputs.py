@@ -1,6 +1,6 @@
 """Inputs of the FRI commit phase as callers may hold them: vectors that join on
 the way in memory of the caller's own, at addresses that are multiples of 4 bytes
-only."""
+only, and challengers in a state that no sequence of calls makes (refused)."""
 import numpy as np
 import pytest
 
@@ -24,3 +24,15 @@ def test_joining_vector_at_any_word(ctx, oracle, f, log_n, log_in, offset):
     assert np.array_equal(fd.commits, roots) and np.array_equal(fd.betas, betas) and np.array_equal(fd.final_poly, final)
     for x in (fd, joined, held, top):
         x.free()
+
+
+@pytest.mark.parametrize("pending", [-1, 8, 9, 1 << 20])
+def test_impossible_challenger_is_refused(ctx, pending):
+    f = KOALABEAR
+    ch, v = pico_amd.DuplexChallenger(f), ctx.random_matrix(f, 3, 1 << 4, 4)
+    ch.c.n_input = pending
+    before = bytes(ch.c)
+    with pytest.raises(pico_amd.PgError):
+        pico_amd.fri_commit_phase(ctx, f, ch, {4: v}, 1, final_mode=1)
+    assert bytes(ch.c) == before
+    v.free()
