@@ -290,7 +290,7 @@ def main():
         step()
     ctx.profile(False)
     fams = ["lde_single", "lde_pass_a", "lde_pass_bc", "lde_pass_d", "leaf_hash", "leaf_hash_w8",
-            "compress", "compress_inject"]
+            "compress", "compress_inject", "tree_layers"]
     kern = {}
     for fam in fams:
         ms, n = ctx.profile_get(fam)

@@ -81,7 +81,11 @@ int pg_device_synchronize(int device);
 size_t pg_bytes_in_use(const pg_ctx *ctx);
 /* Per-kernel timing with HIP events on the launch stream (adds one host sync
  * per launch while enabled).  Families: lde_single, lde_pass_a, lde_pass_bc,
- * lde_pass_d, leaf_hash, leaf_hash_w8, compress, compress_inject, fri_fold.
+ * lde_pass_d, leaf_hash, leaf_hash_w8, compress (one layer of a tree or
+ * several), compress_inject, compress_digest, tree_layers (the leaves of a low
+ * tree and layers above them in one launch; in the FRI commit phase the fold
+ * before them too), absorb_segment, fri_fold, open_values, reduce_openings,
+ * quotient.
  * No counterpart in the reference (its spans time whole phases,
  * vm/src/machine/prover.rs:101,414,539,588); used by the benchmark. */
 int pg_profile_enable(pg_ctx *ctx, int enable);

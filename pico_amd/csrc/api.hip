@@ -1219,11 +1219,10 @@ static int mmcs_commit_on_stream(pg_ctx* ctx, hipStream_t s, int field, const st
     if (hashed) {
     } else if (g1 - g0 == 1 && first->cols > 0 && H <= SMALL_MAX_NODES) {
         const int c = layers_below(H, g1);
-        TIMED(kt, first->cols % 8 ? "leaf_hash" : "leaf_hash_w8", s,
+        TIMED(kt, "tree_layers", s,
               launch_tree_layers(field, first->ptr, first->cols, (uint32_t)first->cols, H, 1 + c, t->digests, s));
         for (int k = 0; k < c; k++, len /= 2) off += len;
-    } else if (g1 - g0 == 1 && first->cols % 8 == 0 && first->cols > 0 && ((uintptr_t)first->ptr % 16) == 0 &&
-             H > SMALL_MAX_NODES)
+    } else if (g1 - g0 == 1 && first->cols % 8 == 0 && first->cols > 0 && ((uintptr_t)first->ptr % 16) == 0)
         TIMED(kt, "leaf_hash_w8", s,
               launch_leaf_hash_w8(field, first->ptr, first->cols, (uint32_t)first->cols, H, t->digests, s));
     else
@@ -3161,7 +3160,7 @@ extern "C" int pg_fri_commit_phase(pg_ctx* ctx, int field, pg_challenger* ch, co
                   launch_tree_layers(field, t->digests + 8 * off, 0, 0, len / 2, log2_of(len), t->digests + 8 * (off + len),
                                      l.s, &tc));
         } else {
-            TIMED(kt, "leaf_hash_w8", l.s,
+            TIMED(kt, "tree_layers", l.s,
                   launch_tree_layers(field, v, 8, 8, len, t->log_h + 1, t->digests, l.s, &tc,
                                      fold.out ? &fold : nullptr));
         }
