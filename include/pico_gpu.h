@@ -379,6 +379,16 @@ typedef struct pg_air_program pg_air_program;
 int pg_air_compile(int field, const pg_air_node *nodes, size_t nnodes, const uint32_t *asserts, size_t nasserts,
                    pg_air_program **out, uint32_t *nregs, uint32_t *ninstr);
 void pg_air_program_free(pg_air_program *prog);
+/* The kernel that evaluates the program over quotient_rows = |Q| rows (a power
+ * of two): its columns resident in LDS with the constraints split over waves, or
+ * read through windows by one wave.  0 for bad arguments.  Both give the same
+ * quotient.  No counterpart in the reference. */
+#define PG_AIR_WINDOWED 1
+#define PG_AIR_RESIDENT 2
+int pg_air_program_form(const pg_air_program *prog, size_t quotient_rows);
+/* Fixes the form of one program for tests that compare the two (0: chosen per
+ * call again); PG_E_UNSUPPORTED where the program has no resident form. */
+int pg_debug_air_form(pg_air_program *prog, int form);
 /* main: matrix main_k of a committed tree at blowup 2^log_blowup (trace
  * height n = its height >> log_blowup); pre: the preprocessed matrix (may be
  * null when the program reads none), same n.  Requires log_quotient_degree <=

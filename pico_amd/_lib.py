@@ -101,6 +101,8 @@ SIGNATURES = {
     "pg_open_proof_free": (None, [_P]),
     "pg_air_compile": (_i, [_i, _P, _sz, _P, _sz, _pp, _P, _P]),
     "pg_air_program_free": (None, [_P]),
+    "pg_air_program_form": (_i, [_P, _sz]),
+    "pg_debug_air_form": (_i, [_P, _i]),
     "pg_quotient_values": (_i, [_P, _P, _P, _sz, _P, _sz, _u32, _u32, _P, _sz, _P, _pp]),
     "pg_quotient_values_perm": (_i, [_P, _P, _P, _sz, _P, _sz, _P, _sz, _u32, _u32, _P, _sz, _P, _sz, _P, _P, _sz,
                                      _P, _pp]),

@@ -24,6 +24,7 @@ from .core import PRIMES, DeviceMatrix, _ptr, from_monty, to_monty
 
 (MAIN, PREPROCESSED, PUBLIC, IS_FIRST_ROW, IS_LAST_ROW, IS_TRANSITION, CONSTANT, ADD, SUB, NEG, MUL, PERMUTATION,
  PERM_CHALLENGE, REGIONAL_SUM, GLOBAL_SUM) = range(15)
+WINDOWED, RESIDENT = 1, 2  # a program's kernel (AirProgram.form)
 
 
 class Expr:
@@ -173,6 +174,14 @@ class AirProgram:
                                    _ptr(asserts) if asserts.size else None, len(asserts), ctypes.byref(h),
                                    ctypes.byref(nregs), ctypes.byref(ninstr)))
         self.handle, self.nregs, self.ninstr = h, nregs.value, ninstr.value
+
+    def form(self, quotient_rows):
+        """The kernel for this many rows of the quotient domain: WINDOWED or RESIDENT."""
+        return lib().pg_air_program_form(self.handle, quotient_rows)
+
+    def debug_form(self, form):
+        """Fix the form (None: chosen per call), for tests that compare the two."""
+        check(lib().pg_debug_air_form(self.handle, form or 0))
 
     def free(self):
         if self.handle:

@@ -3923,6 +3923,7 @@ struct QResident {
 struct pg_air_program {
     int field = 0;
     std::unique_ptr<QResident> resident;  // null: the program does not fit LDS or shares too much
+    int form = 0;  // 0: chosen per call; PG_AIR_WINDOWED, PG_AIR_RESIDENT (tests)
     std::vector<QInstr> code;
     // Montgomery; at launch the public values, challenge words, regional sum
     // and global-sum coordinates follow them
@@ -4745,7 +4746,7 @@ static int air_compile_lowered(int field, const std::vector<pg_air_node>& lnodes
 // 2000; two interactions over 12 columns, 2^15 rows 111 / 73, 2^21 rows 673 / 858.
 static bool quotient_is_resident(const pg_air_program* prog, uint32_t rows) {
     const QResident* const r = prog->resident.get();
-    if (!r) return false;
+    if (!r || prog->form) return prog->form == PG_AIR_RESIDENT;
     const uint64_t S = prog->nstages, N = prog->code.size() - S;
     const uint64_t W = r->slices.size(), L = r->longest, held = W / 2;  // pieces prefetched: 32 rows of a wave's 64 / W
     const uint64_t late = r->pieces.size() > held ? r->pieces.size() - held : 0;
@@ -4753,6 +4754,19 @@ static bool quotient_is_resident(const pg_air_program* prog, uint32_t rows) {
     const uint64_t windowed = 32000 + std::max<uint64_t>(360 * N + 900 * S, ((3000 * N + 15000 * S) * rows) >> 21);
     const uint64_t resident = 40000 + std::max<uint64_t>(170 * L, ((110000 + work + 50000 * late) * rows) >> 21);
     return resident <= windowed;
+}
+
+extern "C" int pg_air_program_form(const pg_air_program* prog, size_t quotient_rows) {
+    if (!prog || !is_pow2(quotient_rows) || quotient_rows > UINT32_MAX) return 0;
+    return quotient_is_resident(prog, (uint32_t)quotient_rows) ? PG_AIR_RESIDENT : PG_AIR_WINDOWED;
+}
+
+extern "C" int pg_debug_air_form(pg_air_program* prog, int form) {
+    if (!prog || (form != 0 && form != PG_AIR_WINDOWED && form != PG_AIR_RESIDENT)) return fail(PG_E_INVALID, "bad argument");
+    if (form == PG_AIR_RESIDENT && !prog->resident)
+        return fail(PG_E_UNSUPPORTED, "the program has no resident form");
+    prog->form = form;
+    return PG_OK;
 }
 
 template <class F>
