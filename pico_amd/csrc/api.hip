@@ -1748,11 +1748,12 @@ extern "C" int pg_pcs_commit_host(pg_ctx* ctx, int field, const uint32_t* const*
         return rc;
     }
     auto kt = make_timer(ctx);
-    // The tallest matrices are cut into column blocks (Montgomery input only:
-    // the canonical conversion works on whole matrices): each block is
-    // uploaded, extended into its columns of the LDE and absorbed into every
-    // row's sponge, so the leaf hash runs behind the upload instead of after
-    // it.  On the device a block is stored dense (rows x cb words at word
+    // The tallest matrices are cut into column blocks where they are larger than
+    // one (Montgomery input only: the canonical conversion works on whole
+    // matrices): each block is uploaded, extended into its columns of the LDE and
+    // absorbed into every row's sponge, so the leaf hash runs behind the upload
+    // instead of after it.  A smaller matrix is one block, and all of its LDE and
+    // hashing follows its upload.  On the device a block is stored dense (rows x cb words at word
     // rows * c0 of the input buffer), so its upload is one contiguous DMA
     // from a stage into which host threads gather the block's row segments
     // (a DMA that reads the pitched rows itself is slower, from page-locked

@@ -328,7 +328,7 @@ struct QuotientArgs {
 // to which the lane is added.
 constexpr int QRL = 64;       // rows per workgroup
 constexpr int QRS_COL = 65;   // words per column slot (conflict-free staging writes)
-constexpr uint32_t QF_ADD = 0, QF_SUB = 1, QF_MUL = 2, QF_OP = 3;
+constexpr uint32_t QF_ADD = 0, QF_SUB = 1, QF_MUL = 2;
 constexpr uint32_t QF_PREV_A = 4, QF_PREV_B = 8, QF_ASSERT = 16, QF_WRITE = 32;
 constexpr int QR_MAX_WAVES = 16, QR_MAX_PIECES = 16;
 constexpr int QR_MIN_SLICE = 24;  // instructions worth a wave

@@ -27,9 +27,10 @@ namespace pg {
 // workgroup, read once per permutation and wave).
 constexpr int MX_WAVES = 4;  // waves per workgroup
 constexpr int MX_THREADS = 64 * MX_WAVES;
-// Three waves per SIMD (168 registers): at four (128) the kernels spill, at two
-// the issue slots are not all filled (leaf hash of 2^21 x 256: 4.53 ms, 4.82
-// and 4.70).
+// Three waves per SIMD (168 registers): at four (128) every kernel spills, at two
+// the issue slots are not all filled (leaf hash of 2^21 x 256: 4.53 ms, 4.82 and
+// 4.70).  At three a few spill 2 to 6 registers (the batched leaves for KoalaBear,
+// the segment absorb and the injecting compress for BabyBear).
 #define MX_KERNEL __global__ void __launch_bounds__(MX_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
 
 // The lane's place in its wave: state 32 t + n of tile t, words 4 h + i of the
@@ -983,9 +984,6 @@ hipError_t launch_leaf_hash(int field, const MatRef* mats, int n, uint32_t total
     return hipGetLastError();
 }
 
-// Fast path entry used by the host when a height group is one matrix with
-// width % 8 == 0 and 32-byte aligned rows (declared here, not in the shared
-// header, because only api.hip's commit planner chooses it).
 hipError_t launch_absorb_segment(int field, const uint32_t* data, uint64_t stride, uint32_t width, uint32_t pos0,
                                  int first, int last, uint64_t rows, uint32_t* state, uint32_t* digests,
                                  hipStream_t stream) {
@@ -999,6 +997,7 @@ hipError_t launch_absorb_segment(int field, const uint32_t* data, uint64_t strid
     return hipGetLastError();
 }
 
+// For a height group that is one matrix with width % 8 == 0 and 16-byte aligned rows.
 hipError_t launch_leaf_hash_w8(int field, const uint32_t* data, uint64_t stride, uint32_t width,
                                size_t rows, uint32_t* digests, hipStream_t stream) {
     if (rows == 0) return hipSuccess;

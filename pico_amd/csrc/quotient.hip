@@ -270,7 +270,8 @@ __global__ void __launch_bounds__(QT) quotient_kernel(QuotientArgs a) {
 // fetched for 4.3 GB over 2^21 rows x 256 columns), and one wave runs the whole
 // program alone at about 0.4 us an instruction, so a short domain is latency.
 // Here the 64 rows of a workgroup are read once, whole runs of columns at a
-// time, and stay in LDS (160 KB: 512 column slots and the registers); the
+// time, and stay in LDS (160 KB: 611 column slots at most, constants, selectors and
+// the slices' registers); the
 // constraints are split over up to 16 waves, each with its own registers, whose
 // sums meet at the end of a block.  The next block's rows are fetched into VGPRs
 // while the program runs.  Rows map to lanes; the next row of lane u sits in
